@@ -71,10 +71,8 @@ int ceil_log2(uint64_t x) {
   return b;
 }
 
-constexpr int kCapSmall = 512;
+constexpr int64_t kFirstVals = (int64_t)1 << 19;        // band cells a wavefront keeps for its traceback at the first level
 constexpr uint64_t kPassBytesPerHit = 140;   // device bytes a search pass holds per seed hit (hits, sort, lists, nodes, outcomes)
-constexpr int kCapLarge = 8192;
-
 }  // namespace
 
 struct oic_ctx {
@@ -110,7 +108,7 @@ struct oic_ctx {
   uint64_t h_alloc = 0;                 // seed hits the per-hit pass buffers are sized for
   int wallclock_khz = 0;                // rate of wall_clock64()
   DevBuf p_pairs, p_tmp, p_nodes, p_recs, p_pout, p_order, p_queue, p_stats, p_nout, p_noff, p_outrec, p_retry;
-  DevBuf sc_rowL, sc_rowR, sc_rowOff, sc_rowVal, sc_dbuf, sc_ld, sc_rd;
+  DevBuf sc_rowm, sc_rowVal, sc_dbuf, sc_ld, sc_rd;
   DevBuf b_outc, b_probe, b_spec, b_cnt, b_off, b_stats, b_order, b_ovf, b_novf;
   // learned cost model
   bool tracing = false;
@@ -118,7 +116,7 @@ struct oic_ctx {
   float mparam[MLP_NPARAM] = {0}, mmu[MLP_IN] = {0}, msd[MLP_IN] = {0};
   DevBuf m_param, m_mu, m_sd, m_feat, m_pred;
   int32_t sc_rows = 0;
-  int64_t sc_val = 0;
+  int64_t sc_val = 0, sc_stride = 0;    // cells a wavefront may keep, and cells from one wavefront's store to the next
   uint32_t sc_waves = 0;
   oic_counters ctr{};
   bool have_model = false;
@@ -655,27 +653,24 @@ extern "C" int oic_index_build(oic_ctx *c, uint32_t bgn, uint32_t end, uint32_t 
 
 // ------------------------------------------------------------------------------------ search
 
-static int ensure_wave_scratch(oic_ctx *c, uint32_t waves, int cap, int64_t val_cap) {
+static int ensure_wave_scratch(oic_ctx *c, uint32_t waves, int64_t val_cap) {
   const int32_t rows = c->T.error_bound[std::min<int32_t>(c->maxlen, (int32_t)oic::kMaxReadLen)] + 4;
-  ALLOC(c, c->sc_rowL, (size_t)waves * rows * 4);
-  ALLOC(c, c->sc_rowR, (size_t)waves * rows * 4);
-  ALLOC(c, c->sc_rowOff, (size_t)waves * rows * 8);
-  ALLOC(c, c->sc_rowVal, (size_t)waves * val_cap * 4);
+  ALLOC(c, c->sc_rowm, (size_t)waves * rows * 4);
+  const int64_t val_stride = val_cap + WR_VAL_SLACK(rows);
+  ALLOC(c, c->sc_rowVal, (size_t)waves * val_stride * 4);
   ALLOC(c, c->sc_dbuf, (size_t)waves * (rows + 4) * 4);
   ALLOC(c, c->sc_ld, (size_t)waves * (rows + 4) * 4);
   ALLOC(c, c->sc_rd, (size_t)waves * (rows + 4) * 4);
   c->sc_rows = rows;
   c->sc_val = val_cap;
+  c->sc_stride = val_stride;
   c->sc_waves = waves;
-  (void)cap;
   return OIC_OK;
 }
 
 static DPScratch scratch0(oic_ctx *c) {
   DPScratch s;
-  s.rowL = c->sc_rowL.as<int32_t>();
-  s.rowR = c->sc_rowR.as<int32_t>();
-  s.rowOff = c->sc_rowOff.as<int64_t>();
+  s.rowm = c->sc_rowm.as<int32_t>();
   s.rowVal = c->sc_rowVal.as<int32_t>();
   s.val_cap = c->sc_val;
   s.max_rows = c->sc_rows - 2;
@@ -702,21 +697,21 @@ static SearchConst search_const(oic_ctx *c, bool elide) {
   return C;
 }
 
-// runs k_process_pairs over order[0..n) with the given tile; returns the number of overflowed pairs
-template <int CAP>
+// runs k_process_pairs over order[0..n) at the given level
+template <int RING>
 static int run_pairs(oic_ctx *c, PairKernelArgs A, uint64_t n, uint32_t waves, int64_t val_cap, double *ms) {
   if (n == 0) return OIC_OK;
   waves = (uint32_t)std::min<uint64_t>(waves, n);
-  int rc = ensure_wave_scratch(c, waves, CAP, val_cap);
+  int rc = ensure_wave_scratch(c, waves, val_cap);
   if (rc) return rc;
   A.sc0 = scratch0(c);
   A.row_stride = c->sc_rows;
-  A.val_stride = c->sc_val;
+  A.val_stride = c->sc_stride;
   A.delta_stride = c->sc_rows + 4;
   A.norder = n;
   HIPCHK(c, hipMemsetAsync(A.queue, 0, 4, c->st));
   HIPCHK(c, hipEventRecord(c->ev0, c->st));
-  hipLaunchKernelGGL(k_process_pairs<CAP>, dim3(waves), dim3(OIC_WAVE), 0, c->st, A);
+  hipLaunchKernelGGL(k_process_pairs<RING>, dim3(waves), dim3(OIC_WAVE), 0, c->st, A);
   HIPCHK(c, hipGetLastError());
   c->ctr.pp_launches++;
   HIPCHK(c, hipEventRecord(c->ev1, c->st));
@@ -783,7 +778,9 @@ static void launch_fwd(oic_ctx *c, const FwdArgs &FA, uint32_t waves) {
       return;
     }
   }
-  if constexpr (!flat_only<G, CAP>())
+  if constexpr (G == 64)
+    hipLaunchKernelGGL((k_fwd_wave<CAP, STATS>), dim3(waves), dim3(OIC_WAVE), 0, c->st, FA);
+  else if constexpr (!flat_only<G, CAP>())
     hipLaunchKernelGGL((k_fwd_tasks<G, CAP, STATS>), dim3(waves), dim3(OIC_WAVE), 0, c->st, FA);
 }
 
@@ -808,7 +805,10 @@ static uint32_t fwd_waves(oic_ctx *c, uint64_t max_tasks) {
       if constexpr (G < 64) {
         if (sm) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_fwd_sm<G, CAP, STATS>, OIC_WAVE, 0);
       }
-      if (sm == 0) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_fwd_tasks<G, CAP, STATS>, OIC_WAVE, 0);
+      if constexpr (G == 64)
+        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_fwd_wave<CAP, STATS>, OIC_WAVE, 0);
+      else if (sm == 0)
+        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_fwd_tasks<G, CAP, STATS>, OIC_WAVE, 0);
     }
     if (e != hipSuccess || per_cu < 1) { (void)hipGetLastError(); per_cu = 16; }
     cached[sm] = per_cu;
@@ -873,17 +873,17 @@ static int run_fwd_binned(oic_ctx *c, FwdArgs FA, uint64_t n, double *ms) {
   HIPCHK(c, hipMemcpy(&nov, FA.novf, 4, hipMemcpyDeviceToHost));
   if (nov == 0) return OIC_OK;
   c->ctr.overflow_retries += nov;
-  // one per wavefront with a 512-cell tile, then what is wider still with an 8192-cell tile
+  // one per wavefront, then what is wider still at its wide level
   FA.tasks = FA.ovf;
   FA.ovf = FA.ovf + n;
   HIPCHK(c, hipMemsetAsync(FA.novf, 0, 4, c->st));
-  rc = c->tune.fwd_counters ? run_fwd<64, 512, true>(c, FA, nov, ms) : run_fwd<64, 512, false>(c, FA, nov, ms);
+  rc = c->tune.fwd_counters ? run_fwd<64, WR_FIRST, true>(c, FA, nov, ms) : run_fwd<64, WR_FIRST, false>(c, FA, nov, ms);
   if (rc) return rc;
   HIPCHK(c, hipMemcpy(&nov, FA.novf, 4, hipMemcpyDeviceToHost));
   if (nov == 0) return OIC_OK;
   FA.tasks = FA.ovf;
   FA.ovf = nullptr;
-  return c->tune.fwd_counters ? run_fwd<64, 8192, true>(c, FA, nov, ms) : run_fwd<64, 8192, false>(c, FA, nov, ms);
+  return c->tune.fwd_counters ? run_fwd<64, WR_WIDE, true>(c, FA, nov, ms) : run_fwd<64, WR_WIDE, false>(c, FA, nov, ms);
 }
 
 // probe pass over every pair's longest node, then every other node of the pairs whose probe
@@ -981,8 +981,7 @@ static int enqueue_fwd_narrow(oic_ctx *c, const FwdArgs &FA, uint64_t max_tasks,
 // task counts stay on the device (the spec count from the scan, overflow counts from each level),
 // buffers are sized by the batch's node count, and counters are cleared by a fill kernel rather
 // than memset nodes.  Each pass runs in three levels: the packed narrow kernel; the tasks whose
-// band outgrew its tile, one per wavefront with a 512-cell tile; those wider still with an
-// 8192-cell tile.  Results are the same as run_forward_passes'.
+// band outgrew its tile, one per wavefront (oic_wdp.h); those wider still at that kernel's wide level.  Results are the same as run_forward_passes'.
 static int run_forward_passes_graph(oic_ctx *c, uint64_t np, uint64_t H, uint64_t nnodes) {
   ALLOC(c, c->b_outc, std::max<uint64_t>(H, 1) * 8);
   ALLOC(c, c->b_probe, np * sizeof(FwdTask));
@@ -1029,12 +1028,12 @@ static int run_forward_passes_graph(oic_ctx *c, uint64_t np, uint64_t H, uint64_
       FA.tstamp = nullptr;
       FA.tasks = ov1; FA.ntasks = 0; FA.ntasks_dev = cnt + 8 + 2 * k;
       FA.queue = cnt + 3 * k + 1; FA.stats = stats + 8 * (3 * k + 1); FA.ovf = ov2; FA.novf = cnt + 9 + 2 * k;
-      if (c->tune.fwd_counters) enqueue_fwd<64, 512, true>(c, FA, cap, ev ? ev[6 * k + 2] : nullptr, ev ? ev[6 * k + 3] : nullptr);
-      else enqueue_fwd<64, 512, false>(c, FA, cap, ev ? ev[6 * k + 2] : nullptr, ev ? ev[6 * k + 3] : nullptr);
+      if (c->tune.fwd_counters) enqueue_fwd<64, WR_FIRST, true>(c, FA, cap, ev ? ev[6 * k + 2] : nullptr, ev ? ev[6 * k + 3] : nullptr);
+      else enqueue_fwd<64, WR_FIRST, false>(c, FA, cap, ev ? ev[6 * k + 2] : nullptr, ev ? ev[6 * k + 3] : nullptr);
       FA.tasks = ov2; FA.ntasks = 0; FA.ntasks_dev = cnt + 9 + 2 * k;
       FA.queue = cnt + 3 * k + 2; FA.stats = stats + 8 * (3 * k + 2); FA.ovf = nullptr; FA.novf = nullptr;
-      if (c->tune.fwd_counters) enqueue_fwd<64, 8192, true>(c, FA, cap, ev ? ev[6 * k + 4] : nullptr, ev ? ev[6 * k + 5] : nullptr);
-      else enqueue_fwd<64, 8192, false>(c, FA, cap, ev ? ev[6 * k + 4] : nullptr, ev ? ev[6 * k + 5] : nullptr);
+      if (c->tune.fwd_counters) enqueue_fwd<64, WR_WIDE, true>(c, FA, cap, ev ? ev[6 * k + 4] : nullptr, ev ? ev[6 * k + 5] : nullptr);
+      else enqueue_fwd<64, WR_WIDE, false>(c, FA, cap, ev ? ev[6 * k + 4] : nullptr, ev ? ev[6 * k + 5] : nullptr);
       return OIC_OK;
     };
     int rc = pass(0, c->b_probe.as<FwdTask>(), np, nullptr, np, ovf, ovf + np);
@@ -1371,8 +1370,8 @@ static int search_batch(oic_ctx *c, uint32_t s0, uint32_t ns, const std::vector<
   A.queue = c->p_queue.as<uint32_t>();
   A.stats = c->p_stats.as<unsigned long long>();
   double ms = 0;
-  const uint32_t waves = (uint32_t)c->ncu * 8;
-  int rc = run_pairs<kCapSmall>(c, A, np, waves, (int64_t)1 << 20, &ms);
+  const uint32_t waves = (uint32_t)c->ncu * 16;
+  int rc = run_pairs<WR_FIRST>(c, A, np, waves, kFirstVals, &ms);
   if (rc) return rc;
   // pairs whose band outgrew the small tile: rerun with the wide tile
   std::vector<PairOut> pout(np);
@@ -1387,8 +1386,8 @@ static int search_batch(oic_ctx *c, uint32_t s0, uint32_t ns, const std::vector<
     HIPCHK(c, hipMemcpyAsync(c->p_retry.p, retry.data(), retry.size() * 4, hipMemcpyHostToDevice, c->st));
     A.order = c->p_retry.as<uint32_t>();
     const int32_t rows = c->T.error_bound[std::min<int32_t>(c->maxlen, (int32_t)oic::kMaxReadLen)] + 4;
-    const int64_t vcap = std::min<int64_t>((int64_t)rows * kCapLarge, (int64_t)1 << 25);
-    rc = run_pairs<kCapLarge>(c, A, retry.size(), std::min<uint32_t>(waves, 256), vcap, &ms);
+    const int64_t vcap = std::min<int64_t>((int64_t)rows * WR_MAX_BAND, (int64_t)1 << 25);
+    rc = run_pairs<WR_WIDE>(c, A, retry.size(), std::min<uint32_t>(waves, 256), vcap, &ms);
     if (rc) return rc;
     HIPCHK(c, hipMemcpyAsync(pout.data(), c->p_pout.p, np * sizeof(PairOut), hipMemcpyDeviceToHost, c->st));
     HIPCHK(c, hipStreamSynchronize(c->st));
@@ -1397,7 +1396,7 @@ static int search_batch(oic_ctx *c, uint32_t s0, uint32_t ns, const std::vector<
         PairRec pr;
         HIPCHK(c, hipMemcpy(&pr, c->p_pairs.as<PairRec>() + p, sizeof pr, hipMemcpyDeviceToHost));
         return fail(c, OIC_EUNSUPPORTED, "pair S %u (%s) x T %u needs a DP band wider than the widest tile (%d cells)", pr.s_id,
-                    pr.dir ? "reverse" : "forward", pr.t_id, kCapLarge);
+                    pr.dir ? "reverse" : "forward", pr.t_id, WR_MAX_BAND + 2);
       }
   }
   c->ctr.ms_dp_kernel += ms;
@@ -1685,6 +1684,10 @@ struct BatchArgs {
   const oic_dp_task *dtasks;
   const oic_ext_task *etasks;
   uint32_t n;
+  const uint32_t *todo;     // if not null: the tasks to run (ntodo of them), left by the first level
+  const uint32_t *ntodo;
+  uint32_t *retry;          // if not null: tasks whose band or rows outgrew this level go here
+  uint32_t *nretry;
   oic_dp_result *dres;
   oic_ext_result *eres;
   int32_t *delta;
@@ -1694,12 +1697,9 @@ struct BatchArgs {
   int64_t row_stride, val_stride, delta_stride_sc;
 };
 
-template <int CAP>
 __device__ __forceinline__ DPScratch batch_scratch(const BatchArgs &A, uint32_t w) {
   DPScratch s = A.sc0;
-  s.rowL = A.sc0.rowL + (int64_t)w * A.row_stride;
-  s.rowR = A.sc0.rowR + (int64_t)w * A.row_stride;
-  s.rowOff = A.sc0.rowOff + (int64_t)w * A.row_stride;
+  s.rowm = A.sc0.rowm + (int64_t)w * A.row_stride;
   s.rowVal = A.sc0.rowVal + (int64_t)w * A.val_stride;
   s.dbuf = A.sc0.dbuf + (int64_t)w * A.delta_stride_sc;
   s.ldelta = A.sc0.ldelta + (int64_t)w * A.delta_stride_sc;
@@ -1707,17 +1707,31 @@ __device__ __forceinline__ DPScratch batch_scratch(const BatchArgs &A, uint32_t 
   return s;
 }
 
-template <int CAP>
+// the next of a launch's `total` tasks for a persistent wavefront, or A.n when none is left
+__device__ __forceinline__ uint32_t next_task(const BatchArgs &A, uint32_t total) {
+  uint32_t i = 0;
+  if (lane_id() == 0) i = atomicAdd(A.queue, 1u);
+  i = (uint32_t)__builtin_amdgcn_readfirstlane((int32_t)i);
+  if (i >= total) return A.n;
+  return A.todo ? A.todo[i] : i;
+}
+
+// true when a task that outgrew this level goes on to the next one
+__device__ __forceinline__ bool to_next_level(const BatchArgs &A, uint32_t i) {
+  if (!A.retry) return false;
+  if (lane_id() == 0) A.retry[atomicAdd(A.nretry, 1u)] = i;
+  return true;
+}
+
+// Two levels (oic_wdp.h): WR_FIRST leaves the few tasks whose band or rows outgrow it to WR_WIDE.
+template <int RING>
 __global__ void __launch_bounds__(OIC_WAVE) k_dp_batch(BatchArgs A) {
-  __shared__ int32_t bufA[CAP], bufB[CAP];
-  __shared__ uint32_t item;
+  __shared__ WaveBand<RING> band;
   const int lane = lane_id();
-  const DPScratch sc = batch_scratch<CAP>(A, blockIdx.x);
+  const DPScratch sc = batch_scratch(A, blockIdx.x);
+  const uint32_t total = A.todo ? *A.ntodo : A.n;
   while (true) {
-    if (lane == 0) item = atomicAdd(A.queue, 1u);
-    __syncthreads();
-    const uint32_t i = item;
-    __syncthreads();
+    const uint32_t i = next_task(A, total);
     if (i >= A.n) break;
     const oic_dp_task t = A.dtasks[i];
     SeqV a, b;
@@ -1729,7 +1743,9 @@ __global__ void __launch_bounds__(OIC_WAVE) k_dp_batch(BatchArgs A) {
       b = read_view(A.R, t.b_id, 1 - t.b_strand); b.b0 += A.R.len[t.b_id] - 1 - t.b_pos;
     }
     uint64_t cells = 0, slots = 0, lb = 0;
-    DPOut o = wave_prefix_dp<CAP>(a, t.m, b, t.n, t.error_limit, t.dir == 0, true, A.tb, bufA, bufB, sc, cells, slots, lb);
+    uint32_t rows = 0;
+    const DPOut o = wave_prefix_dp<RING, true>(a, t.m, b, t.n, t.error_limit, t.dir == 0, true, false, A.tb, band, sc, cells, slots, lb, rows);
+    if (o.overflow && to_next_level(A, i)) continue;
     const int32_t *src = (t.dir == 0) ? sc.rdelta : sc.ldelta;
     if (A.delta && !o.overflow) {
       const int32_t nd = o.ndelta < (int32_t)A.delta_stride ? o.ndelta : (int32_t)A.delta_stride;
@@ -1745,25 +1761,23 @@ __global__ void __launch_bounds__(OIC_WAVE) k_dp_batch(BatchArgs A) {
   }
 }
 
-template <int CAP>
-__global__ void __launch_bounds__(OIC_WAVE) k_ext_batch(BatchArgs A) {
-  __shared__ int32_t bufA[CAP], bufB[CAP];
-  __shared__ uint32_t item;
+template <int RING>
+__global__ void __launch_bounds__(OIC_WAVE) __attribute__((amdgpu_waves_per_eu(4, 8))) k_ext_batch(BatchArgs A) {
+  __shared__ WaveBand<RING> band;
   const int lane = lane_id();
-  const DPScratch sc = batch_scratch<CAP>(A, blockIdx.x);
+  const DPScratch sc = batch_scratch(A, blockIdx.x);
+  const uint32_t total = A.todo ? *A.ntodo : A.n;
   while (true) {
-    if (lane == 0) item = atomicAdd(A.queue, 1u);
-    __syncthreads();
-    const uint32_t i = item;
-    __syncthreads();
+    const uint32_t i = next_task(A, total);
     if (i >= A.n) break;
     const oic_ext_task t = A.etasks[i];
     const SeqV S = read_view(A.R, t.s_id, t.s_dir), Src = read_view(A.R, t.s_id, 1 - t.s_dir);
     const SeqV T = read_view(A.R, t.t_id, 0), Trc = read_view(A.R, t.t_id, 1);
     uint64_t cells = 0, slots = 0, lb = 0;
     uint32_t calls = 0;
-    ExtOut x = wave_extend<CAP>(t.start, t.offset, t.len, S, Src, A.R.len[t.s_id], T, Trc, A.R.len[t.t_id], A.C, bufA, bufB, sc, cells, slots,
-                                calls, lb);
+    ExtOut x = wave_extend<RING>(t.start, t.offset, t.len, S, Src, A.R.len[t.s_id], T, Trc, A.R.len[t.t_id], A.C, band, sc, cells, slots, calls,
+                                lb);
+    if (x.overflow && to_next_level(A, i)) continue;
     if (A.delta && !x.overflow) {
       const int32_t nd = x.ndelta < (int32_t)A.delta_stride ? x.ndelta : (int32_t)A.delta_stride;
       for (int32_t j = lane; j < nd; j += OIC_WAVE) A.delta[(uint64_t)i * A.delta_stride + j] = sc.ldelta[j];
@@ -1778,18 +1792,57 @@ __global__ void __launch_bounds__(OIC_WAVE) k_ext_batch(BatchArgs A) {
   }
 }
 
-template <int CAP>
-static int launch_batch(oic_ctx *c, BatchArgs A, bool ext, uint32_t waves, int64_t vcap) {
-  int rc = ensure_wave_scratch(c, waves, CAP, vcap);
+// the queue of the first level, the count of tasks left to the second, and the second's queue
+constexpr uint32_t kBatchCounters = 3;
+
+// Both levels on the stream; the second is launched only when some task could need it (its error limit
+// allows a band wider than the first level; the first level's store then holds every row too) and reads its count there.
+template <bool EXT>
+static int launch_batch(oic_ctx *c, BatchArgs A, int32_t max_limit) {
+  const int32_t rows = c->T.error_bound[std::min<int32_t>(c->maxlen, (int32_t)oic::kMaxReadLen)] + 4;
+  const bool two = 2 * (int64_t)max_limit + 1 > wr_band<WR_FIRST>();
+  // a band of at most 2e + 1 cells a row
+  const int64_t need = std::min<int64_t>((int64_t)max_limit * (max_limit + 2) + 2, (int64_t)rows * wr_band<WR_FIRST>());
+  const int64_t vcap = std::max<int64_t>(4096, std::min<int64_t>(need, kFirstVals));
+  const uint32_t waves = std::min<uint32_t>(A.n, (uint32_t)c->ncu * 16);
+  DevBuf list;
+  if (two) {
+    ALLOC(c, list, (size_t)A.n * 4);
+    A.retry = list.as<uint32_t>();
+    A.nretry = A.queue + 1;
+  }
+  auto level = [&](uint32_t w, int64_t vc) -> int {
+    int rc = ensure_wave_scratch(c, w, vc);
+    if (rc) return rc;
+    A.sc0 = scratch0(c);
+    A.row_stride = c->sc_rows;
+    A.val_stride = c->sc_stride;
+    A.delta_stride_sc = c->sc_rows + 4;
+      return OIC_OK;
+  };
+  int rc = level(waves, vcap);
   if (rc) return rc;
-  A.sc0 = scratch0(c);
-  A.row_stride = c->sc_rows;
-  A.val_stride = c->sc_val;
-  A.delta_stride_sc = c->sc_rows + 4;
-  HIPCHK(c, hipMemsetAsync(A.queue, 0, 4, c->st));
-  if (ext) hipLaunchKernelGGL(k_ext_batch<CAP>, dim3(waves), dim3(OIC_WAVE), 0, c->st, A);
-  else     hipLaunchKernelGGL(k_dp_batch<CAP>, dim3(waves), dim3(OIC_WAVE), 0, c->st, A);
+  hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, c->st, A.queue, (uint64_t)kBatchCounters, 0u);
+  if (EXT) hipLaunchKernelGGL(k_ext_batch<WR_FIRST>, dim3(waves), dim3(OIC_WAVE), 0, c->st, A);
+  else     hipLaunchKernelGGL(k_dp_batch<WR_FIRST>, dim3(waves), dim3(OIC_WAVE), 0, c->st, A);
   HIPCHK(c, hipGetLastError());
+  if (two) {
+    uint32_t left = 0;
+    HIPCHK(c, hipMemcpyAsync(&left, A.queue + 1, 4, hipMemcpyDeviceToHost, c->st));
+    HIPCHK(c, hipStreamSynchronize(c->st));
+    if (left) {
+      const uint32_t w2 = std::min<uint32_t>(left, (uint32_t)c->ncu);
+      rc = level(w2, std::min<int64_t>((int64_t)rows * WR_MAX_BAND, (int64_t)1 << 24));
+      if (rc) return rc;
+      A.todo = list.as<uint32_t>();
+      A.ntodo = A.queue + 1;
+      A.retry = nullptr;
+      A.queue += 2;
+      if (EXT) hipLaunchKernelGGL(k_ext_batch<WR_WIDE>, dim3(w2), dim3(OIC_WAVE), 0, c->st, A);
+      else     hipLaunchKernelGGL(k_dp_batch<WR_WIDE>, dim3(w2), dim3(OIC_WAVE), 0, c->st, A);
+      HIPCHK(c, hipGetLastError());
+    }
+  }
   HIPCHK(c, hipStreamSynchronize(c->st));
   return OIC_OK;
 }
@@ -1825,9 +1878,9 @@ extern "C" int oic_prefix_dp_batch(oic_ctx *c, const oic_dp_task *tasks, uint32_
   A.delta = delta ? dd.as<int32_t>() : nullptr;
   A.delta_stride = stride;
   A.queue = q.as<uint32_t>();
-  const uint32_t waves = std::min<uint32_t>(n, (uint32_t)c->ncu * 4);
-  const int32_t rows = c->T.error_bound[std::min<int32_t>(c->maxlen, (int32_t)oic::kMaxReadLen)] + 4;
-  int rc = launch_batch<kCapLarge>(c, A, false, waves, std::min<int64_t>((int64_t)rows * kCapLarge, (int64_t)1 << 24));
+  int32_t max_limit = 0;
+  for (uint32_t i = 0; i < n; i++) max_limit = std::max(max_limit, tasks[i].error_limit);
+  int rc = launch_batch<false>(c, A, max_limit);
   if (rc) return rc;
   HIPCHK(c, hipMemcpy(res, dr.p, (size_t)n * sizeof(oic_dp_result), hipMemcpyDeviceToHost));
   if (delta) HIPCHK(c, hipMemcpy(delta, dd.p, (size_t)n * stride * 4, hipMemcpyDeviceToHost));
@@ -1855,14 +1908,14 @@ constexpr size_t kQueueOff = 0;
 constexpr size_t kTaskOff = 256;
 constexpr size_t kResOff = kTaskOff + up256((size_t)kMaxTasks * sizeof(oic_dp_task));
 constexpr size_t kDeltaOff = kResOff + up256((size_t)kMaxTasks * sizeof(oic_dp_result));
-constexpr size_t kRowLOff = kDeltaOff + up256((size_t)kMaxDeltaInts * 4);
-constexpr size_t kRowROff = kRowLOff + up256((size_t)kWaves * kRows * 4);
-constexpr size_t kRowOffOff = kRowROff + up256((size_t)kWaves * kRows * 4);
-constexpr size_t kRowValOff = kRowOffOff + up256((size_t)kWaves * kRows * 8);
-constexpr size_t kDbufOff = kRowValOff + up256((size_t)kWaves * kVals * 4);
+constexpr size_t kRetryOff = kDeltaOff + up256((size_t)kMaxDeltaInts * 4);
+constexpr size_t kRowmOff = kRetryOff + up256((size_t)kMaxTasks * 4);
+constexpr size_t kRowValOff = kRowmOff + up256((size_t)kWaves * kRows * 4);
+constexpr int64_t kValStride = kVals + WR_VAL_SLACK(kRows);
+constexpr size_t kDbufOff = kRowValOff + up256((size_t)kWaves * kValStride * 4);
 constexpr size_t kLdOff = kDbufOff + up256((size_t)kWaves * (kRows + 4) * 4);
 constexpr size_t kRdOff = kLdOff + up256((size_t)kWaves * (kRows + 4) * 4);
-constexpr size_t kBytes = kRdOff + up256((size_t)kWaves * (kRows + 4) * 4);   // about 41 MB
+constexpr size_t kBytes = kRdOff + up256((size_t)kWaves * (kRows + 4) * 4);   // about 42 MB
 }  // namespace na
 
 __device__ __align__(256) uint8_t scratch[na::kBytes];
@@ -1913,7 +1966,7 @@ extern "C" int oic_prefix_dp_batch_noalloc(oic_ctx *c, const oic_dp_task *tasks,
   int32_t *dd = (int32_t *)(base + na::kDeltaOff);
   uint32_t *queue = (uint32_t *)(base + na::kQueueOff);
   HIPCHK(c, hipMemcpyAsync(dt, tasks, (size_t)n * sizeof(oic_dp_task), hipMemcpyHostToDevice, c->st));
-  hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, c->st, queue, (uint64_t)1, 0u);
+  hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, c->st, queue, (uint64_t)kBatchCounters, 0u);
   if (delta) {
     const uint64_t nd = (uint64_t)n * stride;
     hipLaunchKernelGGL(k_fill_u32, dim3((unsigned)((nd + 255) / 256)), dim3(256), 0, c->st, (uint32_t *)dd, nd, 0u);
@@ -1927,9 +1980,7 @@ extern "C" int oic_prefix_dp_batch_noalloc(oic_ctx *c, const oic_dp_task *tasks,
   A.delta = delta ? dd : nullptr;
   A.delta_stride = stride;
   A.queue = queue;
-  A.sc0.rowL = (int32_t *)(base + na::kRowLOff);
-  A.sc0.rowR = (int32_t *)(base + na::kRowROff);
-  A.sc0.rowOff = (int64_t *)(base + na::kRowOffOff);
+  A.sc0.rowm = (int32_t *)(base + na::kRowmOff);
   A.sc0.rowVal = (int32_t *)(base + na::kRowValOff);
   A.sc0.val_cap = na::kVals;
   A.sc0.max_rows = na::kRows - 2;
@@ -1937,10 +1988,24 @@ extern "C" int oic_prefix_dp_batch_noalloc(oic_ctx *c, const oic_dp_task *tasks,
   A.sc0.ldelta = (int32_t *)(base + na::kLdOff);
   A.sc0.rdelta = (int32_t *)(base + na::kRdOff);
   A.row_stride = na::kRows;
-  A.val_stride = na::kVals;
+  A.val_stride = na::kValStride;
   A.delta_stride_sc = na::kRows + 4;
   const uint32_t waves = std::min<uint32_t>(n, na::kWaves);
-  hipLaunchKernelGGL(k_dp_batch<kCapLarge>, dim3(waves), dim3(OIC_WAVE), 0, c->st, A);
+  int32_t max_limit = 0;
+  for (uint32_t i = 0; i < n; i++) max_limit = std::max(max_limit, tasks[i].error_limit);
+  const bool two = 2 * max_limit + 1 > wr_band<WR_FIRST>();   // some band may outgrow the first level
+  if (two) {
+    A.retry = (uint32_t *)(base + na::kRetryOff);
+    A.nretry = queue + 1;
+  }
+  hipLaunchKernelGGL(k_dp_batch<WR_FIRST>, dim3(waves), dim3(OIC_WAVE), 0, c->st, A);
+  if (two) {
+    A.todo = A.retry;
+    A.ntodo = queue + 1;
+    A.retry = nullptr;
+    A.queue = queue + 2;
+    hipLaunchKernelGGL(k_dp_batch<WR_WIDE>, dim3(waves), dim3(OIC_WAVE), 0, c->st, A);
+  }
   HIPCHK(c, hipGetLastError());
   HIPCHK(c, hipMemcpyAsync(res, dr, (size_t)n * sizeof(oic_dp_result), hipMemcpyDeviceToHost, c->st));
   if (delta) HIPCHK(c, hipMemcpyAsync(delta, dd, (size_t)n * stride * 4, hipMemcpyDeviceToHost, c->st));
@@ -1974,9 +2039,10 @@ extern "C" int oic_extend_batch(oic_ctx *c, const oic_ext_task *tasks, uint32_t 
   A.delta = delta ? dd.as<int32_t>() : nullptr;
   A.delta_stride = stride;
   A.queue = q.as<uint32_t>();
-  const uint32_t waves = std::min<uint32_t>(n, (uint32_t)c->ncu * 4);
-  const int32_t rows = c->T.error_bound[std::min<int32_t>(c->maxlen, (int32_t)oic::kMaxReadLen)] + 4;
-  int rc = launch_batch<kCapLarge>(c, A, true, waves, std::min<int64_t>((int64_t)rows * kCapLarge, (int64_t)1 << 24));
+  // an extension's error limit is that of its overlap, which is no longer than the shorter read
+  int32_t longest = 0;
+  for (uint32_t i = 0; i < n; i++) longest = std::max(longest, std::min(c->h_len[tasks[i].s_id], c->h_len[tasks[i].t_id]));
+  int rc = launch_batch<true>(c, A, c->T.error_bound[longest]);
   if (rc) return rc;
   HIPCHK(c, hipMemcpy(res, dr.p, (size_t)n * sizeof(oic_ext_result), hipMemcpyDeviceToHost));
   if (delta) HIPCHK(c, hipMemcpy(delta, dd.p, (size_t)n * stride * 4, hipMemcpyDeviceToHost));

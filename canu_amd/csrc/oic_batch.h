@@ -441,6 +441,77 @@ __global__ void __launch_bounds__(OIC_WAVE) k_fwd_tasks(FwdArgs A) {
   }
 }
 
+// The same tasks one to a wavefront (oic_wdp.h): the packed kernels' tasks whose band outgrew their tile, then
+// those whose band outgrew the first level.
+template <int RING, bool STATS>
+__global__ void __launch_bounds__(OIC_WAVE) k_fwd_wave(FwdArgs A) {
+  __shared__ WaveBand<RING> band;
+  const int lane = lane_id();
+  const uint32_t ntasks = (uint32_t)uni((int32_t)(A.ntasks_dev ? *A.ntasks_dev : (uint32_t)A.ntasks));
+  const DPScratch sc = {};
+  uint64_t cells_acc = 0, slots_acc = 0, bases_acc = 0;
+  uint32_t rows_acc = 0;
+  while (true) {
+    uint32_t f = 0;
+    if (lane == 0) f = atomicAdd(A.queue, 1u);
+    const uint32_t ti = (uint32_t)uni((int32_t)f);
+    if (ti >= ntasks) break;
+    const FwdTask tk = A.tasks[ti];
+    const PairRec pr = A.pairs[tk.pair];
+    const uint64_t gnode = pr.hb + tk.node;
+    const int4 nd = A.nodes[gnode];
+    const int32_t S_Len = A.R.len[pr.s_id], T_Len = A.R.len[pr.t_id];
+    const int32_t Start = nd.z, Offset = nd.x, Len = nd.y;
+    const int32_t S_Right_Begin = Start + Len, S_Right_Len = S_Len - S_Right_Begin;
+    const int32_t T_Right_Begin = Offset + Len, T_Right_Len = T_Len - T_Right_Begin;
+    const int32_t Total_Olap = (Start < Offset ? Start : Offset) + Len + (S_Right_Len < T_Right_Len ? S_Right_Len : T_Right_Len);
+    const int32_t limit = A.tb.error_bound[Total_Olap];
+    int32_t exit_d = T_Right_Begin - S_Right_Begin, right_e = 0;
+    bool mte[2] = {true, true}, overflow = false;
+    uint64_t cells = 0, slots = 0, bases = 0;
+    uint32_t rows = 0;
+    // the right tails (prefixEditDistance-extend.C:81-99), then, when their DP reached the end, the left ones (:112-132)
+    for (int side = 0; side < 2; side++) {
+      const bool right = side == 0;
+      if (right ? (S_Right_Len == 0 || T_Right_Len == 0) : (Start < 1 || Offset < 1)) continue;
+      // left tails are read rightwards on the reverse-complement strands
+      const bool s_first = right ? S_Right_Len <= T_Right_Len : S_Right_Begin <= T_Right_Begin;
+      SeqV s = read_view(A.R, pr.s_id, right ? pr.dir : 1 - pr.dir), t = read_view(A.R, pr.t_id, right ? 0 : 1);
+      s.b0 += right ? S_Right_Begin : S_Len - Start;
+      t.b0 += right ? T_Right_Begin : T_Len - Offset;
+      const int32_t sl = right ? S_Right_Len : Start, tl = right ? T_Right_Len : Offset;
+      const DPOut o = wave_prefix_dp<RING, false>(s_first ? s : t, s_first ? sl : tl, s_first ? t : s, s_first ? tl : sl, limit - right_e, true,
+                                                false, false, A.tb, band, sc, cells, slots, bases, rows);
+      if (o.overflow) { overflow = true; break; }
+      mte[side] = o.mte;
+      if (right) {
+        right_e = o.e;
+        const int32_t d = o.t_end - o.a_end;
+        exit_d += s_first ? d : -d;
+        if (!o.mte) break;
+      }
+    }
+    if (lane == 0) {
+      A.outc[gnode] = pack_outcome(overflow ? 0 : ((mte[0] && mte[1]) ? 2 : 1), exit_d, (uint32_t)cells);
+      if (overflow && A.ovf) A.ovf[atomicAdd(A.novf, 1u)] = tk;
+    }
+    if (!overflow) cells_acc += cells;
+    rows_acc += rows;
+    slots_acc += slots;
+    bases_acc += bases;
+  }
+  for (int o = 32; o > 0; o >>= 1) bases_acc += __shfl_xor(bases_acc, o);
+  if (lane == 0 && A.stats) {
+    atomicAdd(&A.stats[0], (unsigned long long)cells_acc);
+    atomicAdd(&A.stats[4], (unsigned long long)bases_acc);
+    if (STATS) {
+      atomicAdd(&A.stats[1], (unsigned long long)rows_acc);
+      atomicAdd(&A.stats[2], (unsigned long long)slots_acc);
+      atomicAdd(&A.stats[3], (unsigned long long)rows_acc);
+    }
+  }
+}
+
 // ---------------------------------------------------------------- state-machine form
 //
 // The same tasks and results as k_fwd_tasks, with the wavefront's loop turned inside out: each

@@ -50,19 +50,6 @@ struct FlatLDS {
   int32_t start[OIC_WAVE];
 };
 
-// inclusive prefix sum over the wavefront's lanes: within each row of 16 lanes by row shifts
-// (lanes whose source lies before the row start add 0), then each row's total carried into the
-// rows after it by the row broadcasts of lane 15 (into rows 1 and 3) and lane 31 (into rows 2, 3)
-__device__ __forceinline__ int32_t wave_incl_scan(int32_t v) {
-  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);   // row_shr:1
-  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);   // row_shr:2
-  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);   // row_shr:4
-  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);   // row_shr:8
-  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);   // row_bcast:15
-  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);   // row_bcast:31
-  return v;
-}
-
 // Wavefronts per SIMD the flat kernel's LDS allows, at most 4: registers are held to that
 // occupancy (128 VGPRs), which the cell loop's per-lane DP copy needs without spilling.
 // (4 x 64: 10 KB of LDS per wavefront, 16 per CU.)

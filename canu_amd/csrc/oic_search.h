@@ -15,7 +15,7 @@
 //   nodes     : per pair, Match_Node_t list in list order (Offset, Len, Start, removed).
 #pragma once
 
-#include "oic_dp.h"
+#include "oic_wdp.h"
 
 #define OIC_MAX_DISTINCT 3       // MAX_DISTINCT_OLAPS (overlapInCore.H:107)
 #define OIC_HOPELESS     90      // HOPELESS_MATCH (overlapInCore.H:78)
@@ -1086,12 +1086,12 @@ struct SearchConst {
 };
 
 // Extend_Alignment (prefixEditDistance-extend.C:35-183) for one wave.  Deltas land in sc.ldelta
-// (merged Left_Delta) when needed.
-template <int CAP>
+// (merged Left_Delta) when needed.  RING: the widest band's level (oic_wdp.h).
+template <int RING>
 __device__ ExtOut wave_extend(int32_t Start, int32_t Offset, int32_t Len, const SeqV S, const SeqV Src, int32_t S_Len,
-                              const SeqV T, const SeqV Trc, int32_t T_Len, const SearchConst &C, int32_t *bufA,
-                              int32_t *bufB, const DPScratch &sc, uint64_t &cells, uint64_t &slots, uint32_t &dpcalls,
-                              uint64_t &lane_bases, bool known_dovetail = false) {
+                              const SeqV T, const SeqV Trc, int32_t T_Len, const SearchConst &C, WaveBand<RING> &band,
+                              const DPScratch &sc, uint64_t &cells, uint64_t &slots, uint32_t &dpcalls, uint64_t &lane_bases,
+                              bool known_dovetail = false) {
   const int lane = lane_id();
   ExtOut r = {};
   const int32_t S_Left_Begin = Start - 1, S_Right_Begin = Start + Len, S_Right_Len = S_Len - S_Right_Begin;
@@ -1101,159 +1101,126 @@ __device__ ExtOut wave_extend(int32_t Start, int32_t Offset, int32_t Len, const 
   // With elision, deltas only after both sides end, by a second run with row storage; an extension
   // known to be a dovetail (its forward DPs already ran ahead) keeps rows in its only run.
   const bool need_delta = !C.elide || C.partial || known_dovetail;
+  const bool ends_only = C.elide && !C.partial;   // a side that does not end needs no delta
+  const bool no_right = S_Right_Len == 0 || T_Right_Len == 0, no_left = S_Left_Begin < 0 || T_Left_Begin < 0;
+  const bool s_right = S_Right_Len <= T_Right_Len;       // S's right tail is the shorter one: A
+  const bool s_left = S_Right_Begin <= T_Right_Begin;    // S's left tail is
 
   int32_t Right_Errors = 0, Left_Errors = 0, Leftover = 0, nr = 0, nl = 0;
   bool rmte = true, lmte = true;
-  int32_t S_Hi, T_Hi, S_Lo, T_Lo;
-  bool right_negate = false;
-
-  if (S_Right_Len == 0 || T_Right_Len == 0) {
-    S_Hi = 0; T_Hi = 0; rmte = true;
-  } else {
-    SeqV a = S, b = T;
-    int32_t am, bn;
-    if (S_Right_Len <= T_Right_Len) {
-      a.b0 += S_Right_Begin; am = S_Right_Len; b.b0 += T_Right_Begin; bn = T_Right_Len; right_negate = true;
-    } else {
-      a = T; b = S; a.b0 += T_Right_Begin; am = T_Right_Len; b.b0 += S_Right_Begin; bn = S_Right_Len;
-    }
-    DPOut o = wave_prefix_dp<CAP>(a, am, b, bn, Error_Limit, true, need_delta, C.tb, bufA, bufB, sc, cells, slots, lane_bases);
-    dpcalls++;
-    if (o.overflow) { r.overflow = 1; return r; }
-    Right_Errors = o.e; rmte = o.mte; nr = o.ndelta;
-    if (right_negate) { S_Hi = o.a_end; T_Hi = o.t_end; } else { T_Hi = o.a_end; S_Hi = o.t_end; }
-    if (!need_delta && !rmte) {
-      // Process_Matches only distinguishes DOVETAIL from the rest when not doing partials
-      r.kind = 0; r.fwd_e = Right_Errors;
-      r.s_hi = S_Hi + S_Right_Begin - 1; r.t_hi = T_Hi + T_Right_Begin - 1;
-      r.errors = Right_Errors;
-      return r;
-    }
-  }
-  r.fwd_e = Right_Errors;
-  S_Hi += S_Right_Begin - 1;
-  T_Hi += T_Right_Begin - 1;
-
-  // with elision the right side matched to the end here; its delta is needed if the left side
-  // also does: recompute it lazily below (rows of the right DP were not kept)
-  if (S_Left_Begin < 0 || T_Left_Begin < 0) {
-    S_Lo = 0; T_Lo = 0; lmte = true;
-  } else {
+  int32_t S_Hi = 0, T_Hi = 0, S_Lo = 0, T_Lo = 0;
+  // passes 0 and 1: the right and the left tails; 2 and 3: both again with row storage, for the deltas
+  // of an extension whose two sides turned out to end (their cells repeat work already counted)
+  for (int pass = 0; pass < 4; pass++) {
+    const bool again = pass >= 2, right = !(pass & 1), rows = need_delta || again;
+    if (pass == 2 && (need_delta || !rmte || !lmte)) break;
+    if (right ? no_right : no_left) continue;
     SeqV a, b;
     int32_t am, bn;
-    bool swapped;
-    if (S_Right_Begin <= T_Right_Begin) {
-      a = Src; a.b0 += S_Len - 1 - S_Left_Begin; am = S_Left_Begin + 1;
-      b = Trc; b.b0 += T_Len - 1 - T_Left_Begin; bn = T_Left_Begin + 1;
-      swapped = false;
+    bool s_first;
+    if (right) {
+      s_first = s_right;
+      a = s_first ? S : T;
+      b = s_first ? T : S;
+      a.b0 += s_first ? S_Right_Begin : T_Right_Begin;
+      b.b0 += s_first ? T_Right_Begin : S_Right_Begin;
+      am = s_first ? S_Right_Len : T_Right_Len;
+      bn = s_first ? T_Right_Len : S_Right_Len;
     } else {
-      a = Trc; a.b0 += T_Len - 1 - T_Left_Begin; am = T_Left_Begin + 1;
-      b = Src; b.b0 += S_Len - 1 - S_Left_Begin; bn = S_Left_Begin + 1;
-      swapped = true;
+      s_first = s_left;
+      a = s_first ? Src : Trc;
+      b = s_first ? Trc : Src;
+      a.b0 += s_first ? S_Len - 1 - S_Left_Begin : T_Len - 1 - T_Left_Begin;
+      b.b0 += s_first ? T_Len - 1 - T_Left_Begin : S_Len - 1 - S_Left_Begin;
+      am = (s_first ? S_Left_Begin : T_Left_Begin) + 1;
+      bn = (s_first ? T_Left_Begin : S_Left_Begin) + 1;
     }
-    DPOut o = wave_prefix_dp<CAP>(a, am, b, bn, Error_Limit - Right_Errors, false, need_delta, C.tb, bufA, bufB, sc, cells, slots, lane_bases);
-    dpcalls++;
+    uint64_t rc = 0, rs = 0, rb = 0;
+    uint32_t nrows = 0;
+    const DPOut o = wave_prefix_dp<RING, true>(a, am, b, bn, right ? Error_Limit : Error_Limit - Right_Errors, right, rows, ends_only, C.tb, band,
+                                               sc, rc, rs, rb, nrows);
+    if (!again) {
+      cells += rc; slots += rs; lane_bases += rb;
+      dpcalls++;
+    }
     if (o.overflow) { r.overflow = 1; return r; }
-    Left_Errors = o.e; lmte = o.mte; nl = o.ndelta; Leftover = o.leftover;
-    if (!swapped) { S_Lo = o.a_end; T_Lo = o.t_end; } else { T_Lo = o.a_end; S_Lo = o.t_end; }
-    if (need_delta && swapped && lane == 0)
-      for (int32_t i = 0; i < nl; i++) sc.ldelta[i] = -sc.ldelta[i];
+    if (right) {
+      nr = o.ndelta;
+      if (again) continue;
+      Right_Errors = o.e; rmte = o.mte;
+      S_Hi = s_first ? o.a_end : o.t_end;
+      T_Hi = s_first ? o.t_end : o.a_end;
+      if (ends_only && !rmte) {
+        // Process_Matches only distinguishes DOVETAIL from the rest when not doing partials
+        r.kind = 0; r.fwd_e = Right_Errors;
+        r.s_hi = S_Hi + S_Right_Begin - 1; r.t_hi = T_Hi + T_Right_Begin - 1;
+        r.errors = Right_Errors;
+        return r;
+      }
+    } else {
+      nl = o.ndelta; Leftover = o.leftover;
+      // Set_Left_Delta may move T_End by one (reverse.C:76-92): the coordinates are the last run's
+      S_Lo = s_first ? o.a_end : o.t_end;
+      T_Lo = s_first ? o.t_end : o.a_end;
+      if (!again) { Left_Errors = o.e; lmte = o.mte; }
+      if (rows && !s_first)
+        for (int32_t i = lane; i < nl; i += OIC_WAVE) sc.ldelta[i] = -sc.ldelta[i];
+    }
   }
-  S_Lo += S_Left_Begin + 1;
-  T_Lo += T_Left_Begin + 1;
-
+  if (no_left) { Leftover = 0; nl = 0; }
+  r.fwd_e = Right_Errors;
   r.errors = Left_Errors + Right_Errors;
   r.kind = (!rmte) ? (!lmte ? 0 : 2) : (!lmte ? 1 : 3);
-  r.s_lo = S_Lo; r.s_hi = S_Hi; r.t_lo = T_Lo; r.t_hi = T_Hi;
+  r.s_hi = S_Hi + S_Right_Begin - 1;
+  r.t_hi = T_Hi + T_Right_Begin - 1;
+  r.s_lo = S_Lo + S_Left_Begin + 1;
+  r.t_lo = T_Lo + T_Left_Begin + 1;
 
-  if (!need_delta && r.kind == 3) {
-    // both sides matched to the end: rerun the two DPs with row storage for the deltas (their
-    // cells repeat work already counted)
-    uint64_t rc_cells = 0, rc_slots = 0;
-    int32_t re_e = 0, rr = 0;
-    {
-      SeqV a = S, b = T;
-      int32_t am, bn;
-      if (S_Right_Len == 0 || T_Right_Len == 0) { am = 0; bn = 0; }
-      else if (S_Right_Len <= T_Right_Len) { a.b0 += S_Right_Begin; am = S_Right_Len; b.b0 += T_Right_Begin; bn = T_Right_Len; }
-      else { a = T; b = S; a.b0 += T_Right_Begin; am = T_Right_Len; b.b0 += S_Right_Begin; bn = S_Right_Len; }
-      if (am > 0) {
-        uint64_t lb = 0;
-        DPOut o = wave_prefix_dp<CAP>(a, am, b, bn, Error_Limit, true, true, C.tb, bufA, bufB, sc, rc_cells, rc_slots, lb);
-        if (o.overflow) { r.overflow = 1; return r; }
-        rr = o.ndelta; re_e = o.e;
-      }
-      // keep Right_Delta aside in dbuf while the left DP reuses the row storage
-      __syncthreads();
-      if (lane == 0) for (int32_t i = 0; i < rr; i++) sc.dbuf[i] = sc.rdelta[i];
-      __syncthreads();
-    }
-    (void)re_e;
-    if (!(S_Left_Begin < 0 || T_Left_Begin < 0)) {
-      SeqV a, b;
-      int32_t am, bn;
-      bool swapped;
-      if (S_Right_Begin <= T_Right_Begin) {
-        a = Src; a.b0 += S_Len - 1 - S_Left_Begin; am = S_Left_Begin + 1;
-        b = Trc; b.b0 += T_Len - 1 - T_Left_Begin; bn = T_Left_Begin + 1;
-        swapped = false;
-      } else {
-        a = Trc; a.b0 += T_Len - 1 - T_Left_Begin; am = T_Left_Begin + 1;
-        b = Src; b.b0 += S_Len - 1 - S_Left_Begin; bn = S_Left_Begin + 1;
-        swapped = true;
-      }
-      uint64_t lb = 0;
-      DPOut o = wave_prefix_dp<CAP>(a, am, b, bn, Error_Limit - Right_Errors, false, true, C.tb, bufA, bufB, sc, rc_cells, rc_slots, lb);
-      if (o.overflow) { r.overflow = 1; return r; }
-      nl = o.ndelta; Leftover = o.leftover;
-      // Set_Left_Delta may move T_End by one (reverse.C:76-92): take the coordinates from this run
-      if (!swapped) { r.s_lo = o.a_end + S_Left_Begin + 1; r.t_lo = o.t_end + T_Left_Begin + 1; }
-      else          { r.t_lo = o.a_end + T_Left_Begin + 1; r.s_lo = o.t_end + S_Left_Begin + 1; }
-      if (swapped && lane == 0)
-        for (int32_t i = 0; i < nl; i++) sc.ldelta[i] = -sc.ldelta[i];
-    } else {
-      nl = 0; Leftover = 0;
-    }
-    __syncthreads();
-    if (lane == 0) for (int32_t i = 0; i < rr; i++) sc.rdelta[i] = sc.dbuf[i];
-    __syncthreads();
-    nr = rr;
-  }
-
-  // merge deltas (extend.C:164-175); Right_Delta was negated when S was the shorter right tail
+  // merge deltas (extend.C:164-175); Right_Delta is negated when S was the shorter right tail
   if (need_delta || r.kind == 3) {
-    __syncthreads();
-    if (lane == 0) {
-      int32_t n = nl;
-      if (nr > 0) {
-        const int32_t r0 = right_negate ? -sc.rdelta[0] : sc.rdelta[0];
-        sc.ldelta[n++] = (r0 > 0) ? -(r0 + Leftover + Len) : -(r0 - Leftover - Len);
-      }
-      for (int32_t i = 1; i < nr; i++) {
-        const int32_t ri = right_negate ? -sc.rdelta[i] : sc.rdelta[i];
-        sc.ldelta[n++] = -ri;
-      }
-      nl = n;
+    for (int32_t i = lane; i < nr; i += OIC_WAVE) {
+      const int32_t ri = s_right ? -sc.rdelta[i] : sc.rdelta[i];
+      sc.ldelta[nl + i] = i > 0 ? -ri : (ri > 0) ? -(ri + Leftover + Len) : -(ri - Leftover - Len);
     }
-    r.ndelta = __shfl(nl, 0);
+    r.ndelta = nl + nr;
+    __threadfence_block();
     __syncthreads();
   }
   return r;
 }
 
-// Lies_On_Alignment (overlapInCore-Process_String_Overlaps.C:260-281)
-__device__ __forceinline__ bool lies_on_alignment(int32_t start, int32_t offset, int32_t s_lo, int32_t t_lo,
-                                                  const int32_t *__restrict__ delta, int32_t nd) {
-  int32_t diag = t_lo - s_lo;
-  const int32_t new_diag = offset - start;
-  for (int32_t i = 0; i < nd; i++) {
-    const int32_t dl = delta[i];
-    s_lo += dl < 0 ? -dl : dl;
-    if (start < s_lo) return abs(new_diag - diag) <= OIC_SHIFT_SLACK;
-    if (dl < 0) diag++;
-    else { s_lo++; diag--; }
+// Lies_On_Alignment (overlapInCore-Process_String_Overlaps.C:260-281) walks the delta from the alignment's
+// start: the first entry whose run ends past the node's start on S decides, by the diagonal before it.  The
+// runs' ends never fall, so for the many nodes of a pair the walk is taken once, as prefix sums over the
+// delta (run ends to thr, the diagonal before each entry to diag), and a node finds its entry by binary search.
+__device__ __forceinline__ int32_t alignment_runs(int32_t s_lo, int32_t t_lo, const int32_t *__restrict__ delta, int32_t nd,
+                                                  int32_t *__restrict__ thr, int32_t *__restrict__ diag) {
+  const int lane = lane_id();
+  int32_t s = s_lo, g = t_lo - s_lo;
+  for (int32_t b = 0; b < nd; b += OIC_WAVE) {
+    const int32_t i = b + lane;
+    const int32_t dl = i < nd ? delta[i] : 0, len = dl < 0 ? -dl : dl;
+    const int32_t ds = i < nd ? len + (dl < 0 ? 0 : 1) : 0, dg = i < nd ? (dl < 0 ? 1 : -1) : 0;
+    const int32_t is = wave_incl_scan(ds), ig = wave_incl_scan(dg);
+    if (i < nd) {
+      thr[i] = s + is - ds + len;
+      diag[i] = g + ig - dg;
+    }
+    s += __builtin_amdgcn_readlane(is, OIC_WAVE - 1);
+    g += __builtin_amdgcn_readlane(ig, OIC_WAVE - 1);
   }
-  return abs(new_diag - diag) <= OIC_SHIFT_SLACK;
+  return g;   // the diagonal after the last entry
+}
+
+__device__ __forceinline__ bool lies_on_runs(int32_t start, int32_t offset, const int32_t *__restrict__ thr, const int32_t *__restrict__ diag,
+                                             int32_t nd, int32_t last_diag) {
+  int32_t lo = 0, hi = nd;   // the first entry with start < thr
+  while (lo < hi) {
+    const int32_t mid = (lo + hi) >> 1;
+    if (start < thr[mid]) hi = mid;
+    else lo = mid + 1;
+  }
+  return abs(offset - start - (lo < nd ? diag[lo] : last_diag)) <= OIC_SHIFT_SLACK;
 }
 
 // Add_Overlap (Process_String_Overlaps.C:175-244), executed by lane 0 on the LDS copy
@@ -1452,12 +1419,9 @@ struct PairKernelArgs {
   int64_t row_stride, val_stride, delta_stride;
 };
 
-template <int CAP>
 __device__ __forceinline__ DPScratch wave_scratch(const PairKernelArgs &A, uint32_t w) {
   DPScratch s = A.sc0;
-  s.rowL = A.sc0.rowL + (int64_t)w * A.row_stride;
-  s.rowR = A.sc0.rowR + (int64_t)w * A.row_stride;
-  s.rowOff = A.sc0.rowOff + (int64_t)w * A.row_stride;
+  s.rowm = A.sc0.rowm + (int64_t)w * A.row_stride;
   s.rowVal = A.sc0.rowVal + (int64_t)w * A.val_stride;
   s.dbuf = A.sc0.dbuf + (int64_t)w * A.delta_stride;
   s.ldelta = A.sc0.ldelta + (int64_t)w * A.delta_stride;
@@ -1465,17 +1429,67 @@ __device__ __forceinline__ DPScratch wave_scratch(const PairKernelArgs &A, uint3
   return s;
 }
 
+// hopeless check for a singleton match (Process_String_Overlaps.C:384-415)
+__device__ __forceinline__ bool hopeless_pair(const SearchConst &C, const PairRec &pr, const int4 *nodes, int32_t nn, int32_t S_Len,
+                                              int32_t T_Len) {
+  if (!C.hopeless || nn != 1 || C.partial) return false;
+  const int4 nd = nodes[0];
+  const int32_t s_head = nd.z, t_head = nd.x;
+  const uint32_t ss = C.sscreen ? C.sscreen[2 * (pr.s_id - C.s0) + pr.dir] : 0u;
+  const uint32_t ts = C.tscreen ? C.tscreen[pr.t_id - C.hbgn] : 0u;
+  bool hopeless = false;
+  if (s_head <= t_head) { if (s_head > OIC_HOPELESS && !(ss & 1u)) hopeless = true; }
+  else                  { if (t_head > OIC_HOPELESS && !(ts & 1u)) hopeless = true; }
+  const int32_t s_tail = S_Len - s_head - nd.y + 1, t_tail = T_Len - t_head - nd.y + 1;
+  if (s_tail <= t_tail) { if (s_tail > OIC_HOPELESS && !(ss & 2u)) hopeless = true; }
+  else                  { if (t_tail > OIC_HOPELESS && !(ts & 2u)) hopeless = true; }
+  return hopeless;
+}
+
+// a pair's end, on one lane: the selection among its distinct overlaps, its records and counts
+__device__ __forceinline__ void finish_pair(const SearchConst &C, const PairRec &pr, int32_t S_Len, int32_t T_Len, OlapDev *olap, int32_t ct,
+                                            PairOut po, OutRec *recs, PairOut *pout, unsigned long long *stats) {
+  int32_t deleted[OIC_MAX_DISTINCT] = {0, 0, 0};
+  select_distinct(C, olap, ct, deleted);
+  int32_t nout = 0;
+  uint32_t cont = 0, dove = 0;
+  for (int32_t i = 0; i < ct; i++) {
+    if (deleted[i]) continue;
+    OutRec rr;
+    if (C.partial) output_partial(pr.s_id, pr.t_id, pr.dir, olap[i], S_Len, T_Len, &rr);
+    else {
+      if (output_overlap(pr.s_id, S_Len, pr.dir, pr.t_id, T_Len, olap[i], &rr)) cont++; else dove++;
+    }
+    recs[nout] = rr;
+    nout++;
+  }
+  po.nout = nout;
+  po.contained = cont;
+  po.dovetail = dove;
+  *pout = po;
+  if (nout == 0) atomicAdd(&stats[STAT_WITHOUT], 1ull);
+  else {
+    atomicAdd(&stats[STAT_WITH], 1ull);
+    if (nout > 1) atomicAdd(&stats[STAT_MULTI], 1ull);
+  }
+  atomicAdd(&stats[STAT_TOTAL], (unsigned long long)nout);
+  if (!C.partial) {
+    atomicAdd(&stats[STAT_CONT], (unsigned long long)cont);
+    atomicAdd(&stats[STAT_DOVE], (unsigned long long)dove);
+  }
+}
+
 // Process_Matches (overlapInCore-Process_String_Overlaps.C:353-547) for one candidate pair per
 // wavefront.  Persistent: each wave pulls the next pair index from a global counter.
-template <int CAP>
-__global__ void __launch_bounds__(OIC_WAVE) k_process_pairs(PairKernelArgs A) {
-  __shared__ int32_t bufA[CAP], bufB[CAP];
+template <int RING>
+__global__ void __launch_bounds__(OIC_WAVE) __attribute__((amdgpu_waves_per_eu(4, 8))) k_process_pairs(PairKernelArgs A) {
+  __shared__ WaveBand<RING> band;
   __shared__ OlapDev olap[OIC_MAX_DISTINCT];
   __shared__ int32_t olap_ct;
   __shared__ uint32_t next_item;
   const int lane = lane_id();
   const uint32_t w = blockIdx.x;
-  const DPScratch sc = wave_scratch<CAP>(A, w);
+  const DPScratch sc = wave_scratch(A, w);
   const SearchConst &C = A.C;
 
   uint64_t cells = 0, slots = 0, lane_bases = 0, own_cells = 0;
@@ -1495,7 +1509,9 @@ __global__ void __launch_bounds__(OIC_WAVE) k_process_pairs(PairKernelArgs A) {
     const SeqV S = read_view(A.R, S_ID, pr.dir), Src = read_view(A.R, S_ID, 1 - pr.dir);
     const SeqV T = read_view(A.R, T_ID, 0), Trc = read_view(A.R, T_ID, 1);
     PairOut po = {};
-    const uint64_t cells0 = cells;
+    // what an abandoned pair (its band outgrew the tile) counted is taken back: the rerun counts it whole
+    const uint64_t cells0 = cells, own0 = own_cells, slots0 = slots, bases0 = lane_bases;
+    const uint32_t dpcalls0 = dpcalls, exts0 = exts;
 
     // --minkmers filter (Process_String_Overlaps.C:618-621); the threshold per diagonal span is a
     // host-computed table (computeMinimumKmers, :22-33)
@@ -1507,26 +1523,13 @@ __global__ void __launch_bounds__(OIC_WAVE) k_process_pairs(PairKernelArgs A) {
       }
     }
 
-    // hopeless check for a singleton match (Process_String_Overlaps.C:384-415)
-    if (C.hopeless && nn == 1 && !C.partial) {
-      const int4 nd = nodes[0];
-      const int32_t s_head = nd.z, t_head = nd.x;
-      const uint32_t ss = C.sscreen ? C.sscreen[2 * (S_ID - C.s0) + pr.dir] : 0u;
-      const uint32_t ts = C.tscreen ? C.tscreen[T_ID - C.hbgn] : 0u;
-      bool hopeless = false;
-      if (s_head <= t_head) { if (s_head > OIC_HOPELESS && !(ss & 1u)) hopeless = true; }
-      else                  { if (t_head > OIC_HOPELESS && !(ts & 1u)) hopeless = true; }
-      const int32_t s_tail = S_Len - s_head - nd.y + 1, t_tail = T_Len - t_head - nd.y + 1;
-      if (s_tail <= t_tail) { if (s_tail > OIC_HOPELESS && !(ss & 2u)) hopeless = true; }
-      else                  { if (t_tail > OIC_HOPELESS && !(ts & 2u)) hopeless = true; }
-      if (hopeless) {
-        if (lane == 0) {
-          po.status = 2;
-          A.pout[p] = po;
-          atomicAdd(&A.stats[STAT_WITHOUT], 1ull);
-        }
-        continue;
+    if (hopeless_pair(C, pr, nodes, nn, S_Len, T_Len)) {
+      if (lane == 0) {
+        po.status = 2;
+        A.pout[p] = po;
+        atomicAdd(&A.stats[STAT_WITHOUT], 1ull);
       }
+      continue;
     }
 
     if (lane == 0) olap_ct = 0;
@@ -1541,7 +1544,7 @@ __global__ void __launch_bounds__(OIC_WAVE) k_process_pairs(PairKernelArgs A) {
         const int4 nd = nodes[i];
         if (!nd.w && nd.y > bl) { bl = nd.y; bi = i; }
       }
-      wave_argmax_first(bl, bi);
+      wave_pick(bl, bi);
       if (bl < 0) break;
       if (outc && outcome_kind(outc[bi]) == 1) {
         // A node whose extension is known not to be a dovetail is only removed (:473-490); so are
@@ -1551,7 +1554,7 @@ __global__ void __launch_bounds__(OIC_WAVE) k_process_pairs(PairKernelArgs A) {
           const int4 nd = nodes[i];
           if (!nd.w && outcome_kind(outc[i]) != 1 && nd.y > ul) { ul = nd.y; ui = i; }
         }
-        wave_argmax_first(ul, ui);
+        wave_pick(ul, ui);
         uint64_t cnt = 0, cs = 0;
         if (pr.consistent) {
           if (lane == 0) { cnt = 1; cs = outcome_cells(outc[bi]); nodes[bi].w = 1; }
@@ -1578,8 +1581,8 @@ __global__ void __launch_bounds__(OIC_WAVE) k_process_pairs(PairKernelArgs A) {
       }
       const int4 lm = nodes[bi];
       const uint64_t cx = cells;
-      ExtOut x = wave_extend<CAP>(lm.z, lm.x, lm.y, S, Src, S_Len, T, Trc, T_Len, C, bufA, bufB, sc, cells, slots, dpcalls, lane_bases,
-                                  outc && outcome_kind(outc[bi]) == 2);
+      ExtOut x = wave_extend<RING>(lm.z, lm.x, lm.y, S, Src, S_Len, T, Trc, T_Len, C, band, sc, cells, slots, dpcalls,
+                                  lane_bases, outc && outcome_kind(outc[bi]) == 2);
       own_cells += cells - cx;
       exts++;
       po.n_ext++;
@@ -1600,11 +1603,13 @@ __global__ void __launch_bounds__(OIC_WAVE) k_process_pairs(PairKernelArgs A) {
       // remove the longest match and, after a dovetail, every match on the alignment (:476-490)
       if (lane == 0) nodes[bi].w = 1;
       if (x.kind == 3 || C.partial) {
+        const int32_t gl = alignment_runs(x.s_lo, x.t_lo, sc.ldelta, x.ndelta, sc.dbuf, sc.rdelta);
+        __threadfence_block();
         for (int32_t i = lane; i < nn; i += OIC_WAVE) {
           const int4 nd = nodes[i];
           if (nd.w || i == bi) continue;
           if (x.s_lo - OIC_SHIFT_SLACK <= nd.z && nd.z + nd.y <= (x.s_hi + 1) + OIC_SHIFT_SLACK - 1 &&
-              lies_on_alignment(nd.z, nd.x, x.s_lo, x.t_lo, sc.ldelta, x.ndelta))
+              lies_on_runs(nd.z, nd.x, sc.dbuf, sc.rdelta, x.ndelta, gl))
             nodes[i].w = 1;
         }
       }
@@ -1615,43 +1620,16 @@ __global__ void __launch_bounds__(OIC_WAVE) k_process_pairs(PairKernelArgs A) {
     if (overflow) {
       // leave the node list untouched for the retry: clear removal marks
       for (int32_t i = lane; i < nn; i += OIC_WAVE) nodes[i].w = 0;
+      cells = cells0; own_cells = own0; slots = slots0; lane_bases = bases0;
+      dpcalls = dpcalls0; exts = exts0;
+      po = PairOut{};
       if (lane == 0) { po.status = 1; A.pout[p] = po; }
       __syncthreads();
       continue;
     }
 
-    if (lane == 0) {
-      const int32_t ct = olap_ct;
-      int32_t deleted[OIC_MAX_DISTINCT] = {0, 0, 0};
-      select_distinct(C, olap, ct, deleted);
-      int32_t nout = 0;
-      uint32_t cont = 0, dove = 0;
-      for (int32_t i = 0; i < ct; i++) {
-        if (deleted[i]) continue;
-        OutRec rr;
-        if (C.partial) output_partial(S_ID, T_ID, pr.dir, olap[i], S_Len, T_Len, &rr);
-        else {
-          if (output_overlap(S_ID, S_Len, pr.dir, T_ID, T_Len, olap[i], &rr)) cont++; else dove++;
-        }
-        A.recs[(uint64_t)p * OIC_MAX_DISTINCT + nout] = rr;
-        nout++;
-      }
-      po.nout = nout;
-      po.contained = cont;
-      po.dovetail = dove;
-      po.cells = cells - cells0;
-      A.pout[p] = po;
-      if (nout == 0) atomicAdd(&A.stats[STAT_WITHOUT], 1ull);
-      else {
-        atomicAdd(&A.stats[STAT_WITH], 1ull);
-        if (nout > 1) atomicAdd(&A.stats[STAT_MULTI], 1ull);
-      }
-      atomicAdd(&A.stats[STAT_TOTAL], (unsigned long long)nout);
-      if (!C.partial) {
-        atomicAdd(&A.stats[STAT_CONT], (unsigned long long)cont);
-        atomicAdd(&A.stats[STAT_DOVE], (unsigned long long)dove);
-      }
-    }
+    po.cells = cells - cells0;
+    if (lane == 0) finish_pair(C, pr, S_Len, T_Len, olap, olap_ct, po, A.recs + (uint64_t)p * OIC_MAX_DISTINCT, A.pout + p, A.stats);
     __syncthreads();
   }
   for (int o = 32; o > 0; o >>= 1) lane_bases += __shfl_xor(lane_bases, o);
