@@ -246,9 +246,11 @@ def main():
     else:
         form = {0: "k_fwd_sm", 1: "k_fwd_tasks", 2: "k_fwd_flat"}[tuning.get("fwd_loop", 0)]
         fwd_name = f"{form}<{lanes}, {tile}, {stats_flag}>"
-    kernels = [dict(kernel="k_process_pairs<512>", ms=d["ms_pp_kernel"], cells=d["pp_cells"], bases=d["pp_bases"],
+    # Process_Matches: in rounds of extensions, or (plain) one pair per wavefront
+    kernels = [dict(kernel="k_process_pairs<1024>" if args.schedule == "plain" else "k_extend_nodes", ms=d["ms_pp_kernel"], cells=d["pp_cells"], bases=d["pp_bases"],
                     launches=d["pp_launches"],
-                    timing="HIP events around each launch on its stream")]
+                    timing="HIP events around each launch on its stream" if args.schedule == "plain" else
+                           "HIP events around each batch's rounds (k_resolve_pairs and k_extend_nodes launches)")]
     if args.schedule != "plain":
         kernels.append(dict(kernel=fwd_name, ms=d["ms_fwd_narrow"], cells=d["fwd_cells"], bases=d["fwd_bases"],
                             launches=d["fwd_launches"],

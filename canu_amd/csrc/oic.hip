@@ -24,6 +24,7 @@
 #include "oic_batch.h"
 #include "oic_flat.h"
 #include "oic_lane.h"
+#include "oic_rounds.h"
 #include "oic_mlp.h"
 #include <random>
 #include <numeric>
@@ -73,6 +74,15 @@ int ceil_log2(uint64_t x) {
 
 constexpr int64_t kFirstVals = (int64_t)1 << 19;        // band cells a wavefront keeps for its traceback at the first level
 constexpr uint64_t kPassBytesPerHit = 140;   // device bytes a search pass holds per seed hit (hits, sort, lists, nodes, outcomes)
+// rounds of Process_Matches (oic_rounds.h): extensions and node-mask words a batch may hold; how many extensions a
+// pair may ask for in one round: as many as give each resident wavefront kAheadFill, within the limits.  Measured
+// at 2, 4, 8, 16, 32 per wavefront: 755 low-error reads 42, 37, 31, 29, 29 ms, 37 reads 6.8, 6.3, 5.6, 6.1, 5.9 ms,
+// 146 reads under -partial 12.5, 10.4, 9.8, 10.6, 12.9 ms; fewer rounds end fewer launches on their longest
+// extension, and past 8 the extensions that turn out to be removed cost more than that.
+constexpr uint64_t kRoundTasks = (uint64_t)1 << 24;
+constexpr uint64_t kRoundWords = (uint64_t)1 << 27, kRoundWordsMin = (uint64_t)1 << 16;
+constexpr uint32_t kAheadMin = 2, kAheadMax = 64, kAheadFill = 8;
+
 }  // namespace
 
 struct oic_ctx {
@@ -108,6 +118,7 @@ struct oic_ctx {
   uint64_t h_alloc = 0;                 // seed hits the per-hit pass buffers are sized for
   int wallclock_khz = 0;                // rate of wall_clock64()
   DevBuf p_pairs, p_tmp, p_nodes, p_recs, p_pout, p_order, p_queue, p_stats, p_nout, p_noff, p_outrec, p_retry;
+  DevBuf r_state, r_open, r_tasks, r_recs, r_masks, r_cnt;   // Process_Matches in rounds
   DevBuf sc_rowm, sc_rowVal, sc_dbuf, sc_ld, sc_rd;
   DevBuf b_outc, b_probe, b_spec, b_cnt, b_off, b_stats, b_order, b_ovf, b_novf;
   // learned cost model
@@ -915,16 +926,18 @@ static int run_forward_passes(oic_ctx *c, uint64_t np, uint64_t H) {
   FA.tasks = c->b_probe.as<FwdTask>();
   int rc = run_fwd_binned(c, FA, np, &ms);
   if (rc) return rc;
-  hipLaunchKernelGGL(k_spec_count, dim3(g), dim3(256), 0, c->st, c->p_pairs.as<PairRec>(), np, c->b_probe.as<FwdTask>(),
-                     c->b_outc.as<uint64_t>(), spec_pred(c), c->p_order.as<uint32_t>(),
-                     c->b_cnt.as<uint32_t>());
+  const unsigned gw = (unsigned)((np + 3) / 4);   // one wavefront per pair
+  hipLaunchKernelGGL(k_spec_count, dim3(gw), dim3(256), 0, c->st, c->p_pairs.as<PairRec>(), np, c->b_probe.as<FwdTask>(),
+                     c->b_outc.as<uint64_t>(), spec_pred(c), c->p_order.as<uint32_t>(), c->p_nodes.as<int4>(), c->d_len.as<int32_t>(),
+                     c->d_eb.as<int32_t>(), c->b_cnt.as<uint32_t>());
   uint64_t nt = 0;
   ALLOC(c, c->s_scan, scan_scratch_words(np) * 8);
   HIPCHK(c, scan_excl<uint32_t>(c->b_cnt.as<uint32_t>(), c->b_off.as<uint64_t>(), np, c->s_scan.as<uint64_t>(), c->st, &nt));
   if (nt) {
     ALLOC(c, c->b_spec, nt * sizeof(FwdTask));
-    hipLaunchKernelGGL(k_spec_write, dim3(g), dim3(256), 0, c->st, c->p_pairs.as<PairRec>(), np, c->b_probe.as<FwdTask>(),
-                       c->p_order.as<uint32_t>(), c->b_cnt.as<uint32_t>(), c->b_off.as<uint64_t>(), c->b_spec.as<FwdTask>());
+    hipLaunchKernelGGL(k_spec_write, dim3(gw), dim3(256), 0, c->st, c->p_pairs.as<PairRec>(), np, c->b_probe.as<FwdTask>(),
+                       c->p_order.as<uint32_t>(), c->p_nodes.as<int4>(), c->d_len.as<int32_t>(), c->d_eb.as<int32_t>(),
+                       c->b_cnt.as<uint32_t>(), c->b_off.as<uint64_t>(), c->b_spec.as<FwdTask>());
     FA.tasks = c->b_spec.as<FwdTask>();
     if (c->tune.fwd_order == 1) {
       // the hit buffers are free once the match lists exist
@@ -1038,13 +1051,15 @@ static int run_forward_passes_graph(oic_ctx *c, uint64_t np, uint64_t H, uint64_
     };
     int rc = pass(0, c->b_probe.as<FwdTask>(), np, nullptr, np, ovf, ovf + np);
     if (rc) return rc;
-    hipLaunchKernelGGL(k_spec_count, dim3(g), dim3(256), 0, c->st, c->p_pairs.as<PairRec>(), np, c->b_probe.as<FwdTask>(),
-                       c->b_outc.as<uint64_t>(), spec_pred(c), c->p_order.as<uint32_t>(),
-                       c->b_cnt.as<uint32_t>());
+    const unsigned gw = (unsigned)((np + 3) / 4);   // one wavefront per pair
+    hipLaunchKernelGGL(k_spec_count, dim3(gw), dim3(256), 0, c->st, c->p_pairs.as<PairRec>(), np, c->b_probe.as<FwdTask>(),
+                       c->b_outc.as<uint64_t>(), spec_pred(c), c->p_order.as<uint32_t>(), c->p_nodes.as<int4>(), c->d_len.as<int32_t>(),
+                       c->d_eb.as<int32_t>(), c->b_cnt.as<uint32_t>());
     HIPCHK(c, scan_excl<uint32_t>(c->b_cnt.as<uint32_t>(), c->b_off.as<uint64_t>(), np, c->s_scan.as<uint64_t>(), c->st, nullptr));
     hipLaunchKernelGGL(k_scan_total, dim3(1), dim3(64), 0, c->st, c->b_cnt.as<uint32_t>(), c->b_off.as<uint64_t>(), np, cnt + 6);
-    hipLaunchKernelGGL(k_spec_write, dim3(g), dim3(256), 0, c->st, c->p_pairs.as<PairRec>(), np, c->b_probe.as<FwdTask>(),
-                       c->p_order.as<uint32_t>(), c->b_cnt.as<uint32_t>(), c->b_off.as<uint64_t>(), c->b_spec.as<FwdTask>());
+    hipLaunchKernelGGL(k_spec_write, dim3(gw), dim3(256), 0, c->st, c->p_pairs.as<PairRec>(), np, c->b_probe.as<FwdTask>(),
+                       c->p_order.as<uint32_t>(), c->p_nodes.as<int4>(), c->d_len.as<int32_t>(), c->d_eb.as<int32_t>(),
+                       c->b_cnt.as<uint32_t>(), c->b_off.as<uint64_t>(), c->b_spec.as<FwdTask>());
     rc = pass(1, c->b_spec.as<FwdTask>(), 0, cnt + 6, nnodes, ovf + 2 * np, ovf + 2 * np + nnodes);
     if (rc) return rc;
     HIPCHK(c, hipGetLastError());
@@ -1124,6 +1139,83 @@ static int run_forward_passes_graph(oic_ctx *c, uint64_t np, uint64_t H, uint64_
   for (float x : f) ms += x;
   c->ctr.ms_fwd_kernel += ms;
   c->ctr.ms_dp_kernel += ms;
+  return OIC_OK;
+}
+
+// Process_Matches of the batch's pairs in rounds (oic_rounds.h).  list (np pairs, processing order) may be
+// overwritten.  Pairs that the rounds' arrays could not hold run one to a wavefront at the end.
+static int run_rounds(oic_ctx *c, const PairKernelArgs &PA, uint64_t np, uint64_t nnodes, double *ms) {
+  RoundArgs A{};
+  A.R = PA.R;
+  A.C = PA.C;
+  A.pairs = PA.pairs;
+  A.nodes = PA.nodes;
+  A.outc = c->b_outc.as<uint64_t>();
+  A.pred = spec_pred(c);
+  A.out = PA.recs;
+  A.pout = PA.pout;
+  A.stats = PA.stats;
+  // every node is extended at most once; a mask is a bit per node of the task's pair
+  A.task_cap = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(nnodes, 1), kRoundTasks);
+  A.word_cap = std::max<uint64_t>(kRoundWordsMin, std::min<uint64_t>(4 * nnodes, kRoundWords));
+  ALLOC(c, c->r_state, np * sizeof(PairState));
+  ALLOC(c, c->r_open, 2 * np * 4);
+  ALLOC(c, c->r_tasks, (size_t)A.task_cap * sizeof(ExtNode));
+  ALLOC(c, c->r_recs, (size_t)A.task_cap * sizeof(ExtRec));
+  ALLOC(c, c->r_masks, A.word_cap * 8);
+  ALLOC(c, c->r_cnt, sizeof(RoundCount));
+  A.state = c->r_state.as<PairState>();
+  A.tasks = c->r_tasks.as<ExtNode>();
+  A.recs = c->r_recs.as<ExtRec>();
+  A.masks = c->r_masks.as<uint64_t>();
+  A.cnt = c->r_cnt.as<RoundCount>();
+  const uint32_t ewaves = (uint32_t)c->ncu * 16;
+  HIPCHK(c, hipEventRecord(c->ev0, c->st));
+  hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, c->st, (uint32_t *)A.cnt, (uint64_t)(sizeof(RoundCount) / 4), 0u);
+  A.list = PA.order;
+  A.n = (uint32_t)np;
+  uint32_t *open[2] = {c->r_open.as<uint32_t>(), c->r_open.as<uint32_t>() + np};
+  RoundCount rc{};
+  uint32_t left = 0;
+  for (int round = 0;; round++) {
+    A.open = open[round & 1];
+    A.ahead = (int32_t)std::max<uint32_t>(kAheadMin, std::min<uint32_t>(kAheadMax, kAheadFill * ewaves / std::max<uint32_t>(A.n, 1)));
+    A.resume = round > 0 ? 1 : 0;
+    hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, c->st, (uint32_t *)A.cnt, (uint64_t)4, 0u);
+    hipLaunchKernelGGL(k_resolve_pairs, dim3(std::min<uint32_t>(A.n, (uint32_t)c->ncu * 32)), dim3(OIC_WAVE), 0, c->st, A);
+    HIPCHK(c, hipGetLastError());
+    c->ctr.pp_launches++;
+    HIPCHK(c, hipMemcpyAsync(&rc, A.cnt, sizeof rc, hipMemcpyDeviceToHost, c->st));
+    HIPCHK(c, hipStreamSynchronize(c->st));
+    const uint32_t nt = std::min(rc.ntasks, A.task_cap);
+    if (rc.nopen == 0) break;
+    if (nt == A.task0) { left = rc.nopen; break; }   // nothing more fits
+    A.task1 = nt;
+    const uint32_t waves = std::min<uint32_t>(ewaves, nt - A.task0);
+    int e = ensure_wave_scratch(c, waves, kFirstVals);
+    if (e) return e;
+    A.sc0 = scratch0(c);
+    A.row_stride = c->sc_rows;
+    A.val_stride = c->sc_stride;
+    A.delta_stride = c->sc_rows + 4;
+    hipLaunchKernelGGL(k_extend_nodes, dim3(waves), dim3(OIC_WAVE), 0, c->st, A);
+    HIPCHK(c, hipGetLastError());
+    c->ctr.spec_tasks += nt - A.task0;
+    A.task0 = nt;
+    A.list = A.open;
+    A.n = rc.nopen;
+  }
+  HIPCHK(c, hipEventRecord(c->ev1, c->st));
+  HIPCHK(c, hipEventSynchronize(c->ev1));
+  float f = 0;
+  hipEventElapsedTime(&f, c->ev0, c->ev1);
+  *ms += f;
+  if (left) {
+    hipLaunchKernelGGL(k_reopen_pairs, dim3(left), dim3(OIC_WAVE), 0, c->st, A.pairs, A.open, A.nodes);
+    PairKernelArgs B = PA;
+    B.order = A.open;
+    return run_pairs<WR_FIRST>(c, B, left, (uint32_t)c->ncu * 16, kFirstVals, ms);
+  }
   return OIC_OK;
 }
 
@@ -1348,7 +1440,13 @@ static int search_batch(oic_ctx *c, uint32_t s0, uint32_t ns, const std::vector<
   HIPCHK(c, hipMemcpyAsync(c->p_order.p, order.data(), np * 4, hipMemcpyHostToDevice, c->st));
 
   // batched schedules: forward DPs of probe and speculative nodes, packed 4 per wavefront
-  const bool batched = c->P.schedule != OIC_SCHED_PLAIN && !c->P.partial;
+  // Under -partial every extension's delta is needed and none runs ahead; the rounds find no outcomes.
+  const bool in_rounds = c->P.schedule != OIC_SCHED_PLAIN;
+  const bool batched = in_rounds && !c->P.partial;
+  if (in_rounds && !batched) {
+    ALLOC(c, c->b_outc, std::max<uint64_t>(H, 1) * 8);
+    hipLaunchKernelGGL(k_fill_u32, dim3((unsigned)((2 * H + 255) / 256)), dim3(256), 0, c->st, (uint32_t *)c->b_outc.p, 2 * H, 0u);
+  }
   if (batched) {
     int rc = (c->tune.fwd_order == 0) ? run_forward_passes_graph(c, np, H, batch_nodes) : run_forward_passes(c, np, H);
     if (rc) return rc;
@@ -1361,7 +1459,7 @@ static int search_batch(oic_ctx *c, uint32_t s0, uint32_t ns, const std::vector<
     A.C.sscreen = c->g_sscreen.as<uint32_t>();
     A.C.s0 = s0;
   }
-  A.outc = batched ? c->b_outc.as<uint64_t>() : nullptr;
+  A.outc = in_rounds ? c->b_outc.as<uint64_t>() : nullptr;
   A.pairs = c->p_pairs.as<PairRec>();
   A.order = c->p_order.as<uint32_t>();
   A.nodes = c->p_nodes.as<int4>();
@@ -1371,7 +1469,7 @@ static int search_batch(oic_ctx *c, uint32_t s0, uint32_t ns, const std::vector<
   A.stats = c->p_stats.as<unsigned long long>();
   double ms = 0;
   const uint32_t waves = (uint32_t)c->ncu * 16;
-  int rc = run_pairs<WR_FIRST>(c, A, np, waves, kFirstVals, &ms);
+  int rc = in_rounds ? run_rounds(c, A, np, batch_nodes, &ms) : run_pairs<WR_FIRST>(c, A, np, waves, kFirstVals, &ms);
   if (rc) return rc;
   // pairs whose band outgrew the small tile: rerun with the wide tile
   std::vector<PairOut> pout(np);
@@ -1426,6 +1524,10 @@ static int search_batch(oic_ctx *c, uint32_t s0, uint32_t ns, const std::vector<
   c->ctr.dp_bases += stats[STAT_BASES];
   c->ctr.pp_cells += stats[STAT_PPCELLS];
   c->ctr.pp_bases += stats[STAT_BASES];
+  if (in_rounds) {
+    c->ctr.spec_cells += stats[STAT_PPCELLS];
+    c->ctr.spec_bases += stats[STAT_BASES];
+  }
   // records that fit go straight into the caller's sink, the rest are held by the context
   // (oic_fetch_pending hands them over without searching again)
   const uint64_t room = (sink->records && sink->capacity > sink->count) ? sink->capacity - sink->count : 0;

@@ -11,9 +11,8 @@
 //   0  not computed (band outgrew the tile),
 // with the run's DP cells and right-end diagonal, so that a finished task makes a single store.
 // Tasks run 64/G to a wavefront (G lanes each, a T-cell band tile in LDS; the autotuner picks G and
-// T, 8 x 64 on repeat-rich reads); those whose band outgrows the tile are queued and re-run one to a
-// wavefront with a 512-cell tile, then an 8192-cell one, which holds any band the error limit
-// allows (2 x 2700 + 3 cells at 60 kbp and 4.5 %).
+// T); those whose band outgrows the tile are queued and re-run one to a wavefront (oic_wdp.h), up to 960 cells,
+// then up to 8190, which holds any band the error limit allows (2 x 2700 + 3 cells at 60 kbp and 4.5 %).
 // The DP is wave_prefix_dp's row loop without row storage or traceback, on a G-lane group, with the
 // first 1024 bases of both tails staged in LDS.  When the forward DP reaches the end, the reverse DP
 // on the left tails runs too, so the cached outcome is the extension's kind.  Two loop forms:
@@ -982,46 +981,92 @@ __global__ void k_probe_tasks(const PairRec *__restrict__ pairs, uint64_t np, Fw
   tasks[p].node = (uint32_t)pairs[p].first_longest;   // found by the list builders
 }
 
-// Pairs whose other nodes are all worth a forward DP ahead of Process_Matches: those whose probe
-// was not a dovetail (each later node is reached unless it is itself the next one removed), and
-// some of those with a dovetail probe, whose nodes on the probe's alignment Process_Matches will
-// remove without extending them (overlapInCore-Process_String_Overlaps.C:476-490) while repeat
-// copies on shifted diagonals survive.  For a dovetail probe the static rule speculates when the
-// pair has at least SPEC_DOVE_MIN nodes; with a cost model (pred: its log(1 + DP cells) of the
-// pair's Process_Matches, per pair) it speculates when the model expects more than SPEC_DOVE_GAIN
-// times the probe's own cells, i.e. further extensions beyond the probe.  Counts are written in
-// processing order.  Which nodes run ahead never changes a result.
+// Nodes worth a forward DP ahead of Process_Matches: all others of a pair whose probe was not a dovetail (each
+// is reached unless it is itself the next one removed), and some of a pair with a dovetail probe.  There,
+// Process_Matches removes the nodes on the probe's alignment without extending them
+// (overlapInCore-Process_String_Overlaps.C:476-490), and what it extends of those near it is a dovetail too,
+// whose delta it needs (oic_rounds.h runs those once, with rows); repeat copies on shifted diagonals survive and
+// mostly are none.  So only nodes whose diagonal lies further from the probe's than its alignment drifts run
+// here: SPEC_NEAR + limit / 8 diagonals, limit the errors the pair's longest overlap may have (8 kbp at 4.5 %:
+// 77; the drift of 3 % indels there is about 13, at most 40).  On 755 low-error reads, 662 thousand nodes, the forward
+// kernels of a batch go from 61 to 7 ms.  The static rule takes such a pair when it has at least SPEC_DOVE_MIN
+// nodes; with a cost model (pred: its log(1 + DP cells) of the pair's
+// Process_Matches, per pair) when the model expects more than SPEC_DOVE_GAIN times the probe's own cells,
+// i.e. further extensions beyond the probe.  Which nodes run ahead never changes a result.
 #define SPEC_DOVE_MIN 16
 #define SPEC_DOVE_GAIN 2.0f
-__global__ void k_spec_count(const PairRec *__restrict__ pairs, uint64_t np, const FwdTask *__restrict__ probe,
-                             const uint64_t *__restrict__ outc, const float *__restrict__ pred,
-                             const uint32_t *__restrict__ order, uint32_t *__restrict__ cnt) {
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= np) return;
-  const uint32_t p = order[i];
-  const PairRec pr = pairs[p];
-  const uint64_t po = outc[pr.hb + probe[p].node];
+#define SPEC_NEAR 32
+
+// whether the pair's nodes run ahead: 0 none, 1 all but the probe, 2 those far from the probe's diagonal
+__device__ __forceinline__ int spec_rule(const PairRec &pr, uint64_t po, const float *__restrict__ pred, uint32_t p) {
   const int pc = outcome_kind(po);
+  if (pr.consistent || pr.nnodes <= 1) return 0;
+  if (pc == 1) return 1;
   bool dove_spec = pr.nnodes >= SPEC_DOVE_MIN;
   if (pred) dove_spec = expm1f(pred[2 * (uint64_t)p]) > SPEC_DOVE_GAIN * (float)outcome_cells(po);
-  const bool spec = !pr.consistent && pr.nnodes > 1 && (pc == 1 || (pc == 2 && dove_spec));
-  cnt[i] = spec ? (uint32_t)(pr.nnodes - 1) : 0u;
+  return (pc == 2 && dove_spec) ? 2 : 0;
 }
 
-__global__ void k_spec_write(const PairRec *__restrict__ pairs, uint64_t np, const FwdTask *__restrict__ probe,
-                             const uint32_t *__restrict__ order, const uint32_t *__restrict__ cnt, const uint64_t *__restrict__ off,
-                             FwdTask *__restrict__ tasks) {
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= np || cnt[i] == 0) return;
+__device__ __forceinline__ int32_t spec_reach(const PairRec &pr, const int32_t *__restrict__ len, const int32_t *__restrict__ error_bound) {
+  const int32_t a = len[pr.s_id], b = len[pr.t_id];
+  return SPEC_NEAR + error_bound[a < b ? a : b] / 8;
+}
+
+// one wavefront per pair (a repeat pair holds up to 10^5 nodes); counts are written in processing order
+__global__ void __launch_bounds__(256) k_spec_count(const PairRec *__restrict__ pairs, uint64_t np, const FwdTask *__restrict__ probe,
+                                                    const uint64_t *__restrict__ outc, const float *__restrict__ pred,
+                                                    const uint32_t *__restrict__ order, const int4 *__restrict__ nodes,
+                                                    const int32_t *__restrict__ len, const int32_t *__restrict__ error_bound,
+                                                    uint32_t *__restrict__ cnt) {
+  const uint64_t i = (uint64_t)blockIdx.x * (blockDim.x / OIC_WAVE) + threadIdx.x / OIC_WAVE;
+  if (i >= np) return;
+  const int lane = lane_id();
   const uint32_t p = order[i];
-  const int32_t nn = pairs[p].nnodes;
-  const uint32_t skip = probe[p].node;
+  const PairRec pr = pairs[p];
+  const int32_t pn = (int32_t)probe[p].node;
+  const int rule = spec_rule(pr, outc[pr.hb + pn], pred, p);
+  int32_t n = rule == 1 ? pr.nnodes - 1 : 0;
+  if (rule == 2) {
+    const int32_t reach = spec_reach(pr, len, error_bound);
+    const int4 pd = nodes[pr.hb + pn];
+    for (int32_t j0 = 0; j0 < pr.nnodes; j0 += OIC_WAVE) {
+      const int32_t j = j0 + lane;
+      bool far = false;
+      if (j < pr.nnodes) {
+        const int4 nd = nodes[pr.hb + j];
+        far = j != pn && abs((nd.x - nd.z) - (pd.x - pd.z)) > reach;
+      }
+      n += (int32_t)__builtin_popcountll(__ballot(far));
+    }
+  }
+  if (lane == 0) cnt[i] = (uint32_t)n;
+}
+
+__global__ void __launch_bounds__(256) k_spec_write(const PairRec *__restrict__ pairs, uint64_t np, const FwdTask *__restrict__ probe,
+                                                    const uint32_t *__restrict__ order, const int4 *__restrict__ nodes,
+                                                    const int32_t *__restrict__ len, const int32_t *__restrict__ error_bound,
+                                                    const uint32_t *__restrict__ cnt, const uint64_t *__restrict__ off,
+                                                    FwdTask *__restrict__ tasks) {
+  const uint64_t i = (uint64_t)blockIdx.x * (blockDim.x / OIC_WAVE) + threadIdx.x / OIC_WAVE;
+  if (i >= np || cnt[i] == 0) return;
+  const int lane = lane_id();
+  const uint32_t p = order[i];
+  const PairRec pr = pairs[p];
+  const int32_t pn = (int32_t)probe[p].node;
+  const bool all = cnt[i] == (uint32_t)(pr.nnodes - 1);
+  const int32_t reach = spec_reach(pr, len, error_bound);
+  const int4 pd = nodes[pr.hb + pn];
   uint64_t w = off[i];
-  for (int32_t i = 0; i < nn; i++) {
-    if ((uint32_t)i == skip) continue;
-    tasks[w].pair = (uint32_t)p;
-    tasks[w].node = (uint32_t)i;
-    w++;
+  for (int32_t j0 = 0; j0 < pr.nnodes; j0 += OIC_WAVE) {
+    const int32_t j = j0 + lane;
+    bool take = j < pr.nnodes && j != pn;
+    if (take && !all) {
+      const int4 nd = nodes[pr.hb + j];
+      take = abs((nd.x - nd.z) - (pd.x - pd.z)) > reach;
+    }
+    const uint64_t b = __ballot(take);
+    if (take) tasks[w + __builtin_popcountll(b & ((1ull << lane) - 1))] = FwdTask{p, (uint32_t)j};
+    w += (uint64_t)__builtin_popcountll(b);
   }
 }
 

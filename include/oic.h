@@ -116,7 +116,8 @@ typedef struct oic_counters {
   uint64_t dp_lane_slots;      /* lane-cells issued (cells plus idle lanes of partial chunks) */
   uint64_t dp_bases;           /* bases compared in slides, plus one terminating compare per cell */
   uint64_t overflow_retries;   /* DP tasks re-run with a wider band tile */
-  uint64_t spec_tasks;         /* forward DPs run ahead of Process_Matches (batched schedules) */
+  uint64_t spec_tasks;         /* forward DPs and whole extensions run ahead of their pair's Process_Matches
+                                  (batched and learned schedules) */
   uint64_t spec_cells;         /* cells of those runs, used or not */
   uint64_t spec_rows;          /* DP rows (e >= 1) of those runs (with tuning.fwd_counters) */
   uint64_t spec_lane_slots;    /* lane-cells issued by those runs (with tuning.fwd_counters) */
@@ -140,11 +141,12 @@ typedef struct oic_counters {
                                   or, inside a forward-pass graph, the span from its first wavefront's
                                   start to its last one's end (device wall clock) */
   double   ms_fwd_graph;       /* forward-pass graphs, HIP events around their launches */
-  double   ms_pp_kernel;       /* the Process_Matches kernel (k_process_pairs), HIP events around its launches */
-  uint64_t pp_cells;           /* DP cells that kernel computes itself (full extensions with row storage) */
+  double   ms_pp_kernel;       /* Process_Matches (k_process_pairs, or the rounds of k_resolve_pairs and
+                                  k_extend_nodes), HIP events around its launches */
+  uint64_t pp_cells;           /* DP cells it computes itself (full extensions with row storage) */
   uint64_t pp_bases;           /* bases it compares in their slides, plus one per cell */
   uint64_t learned_pairs;      /* pairs the learned cost model ordered (OIC_SCHED_LEARNED with a model) */
-  uint64_t pp_launches;        /* launches of the Process_Matches kernel */
+  uint64_t pp_launches;        /* launches of k_process_pairs or k_resolve_pairs */
   uint64_t spec_wave_chunks;   /* band chunk iterations wavefronts of the row-stepped kernel executed (with tuning.fwd_counters) */
   uint64_t allocs;             /* device work-buffer allocations the context made (first use or growth) */
   double   ms_alloc;           /* host time those allocations took, with the free of the smaller buffer */
@@ -160,8 +162,8 @@ typedef struct oic_tuning {
                                    DPs per wavefront, rows spread over the group; default 4) */
   uint32_t fwd_tile;            /* band cells a packed forward DP holds in LDS: 16, 32 or 64 with one
                                    lane per DP; 32 or 64 (8 or 16 lanes), 128, 256 or 512 otherwise;
-                                   wider bands re-run one per wavefront, with a 512-cell tile and then
-                                   an 8192-cell one (default 64) */
+                                   wider bands re-run one per wavefront, up to 960 cells and then up to
+                                   8190 (default 64) */
   uint32_t fwd_order;          /* speculative DP tasks in pair order (0) or by seed length,
                                    longest first (1); the autotuner picks */
   uint32_t fwd_graph;           /* 1 (default): each search batch's probe and speculation passes run
