@@ -1336,7 +1336,7 @@ static int search_batch(oic_ctx *c, uint32_t s0, uint32_t ns, const std::vector<
     LS.sA = b; LS.sB = b + H; LS.oA = b + 2 * H; LS.oB = b + 3 * H; LS.fr = b + 4 * H; LS.dq = b + 5 * H; LS.db = b + 6 * H;
     LS.pos = b + 7 * H;
     LS.fl = (uint8_t *)(b + 8 * H);
-    // pairs with many hits: one wavefront each; the rest (and any handed back): one thread each
+    // one wavefront per pair, at a level by its hits; pairs that one hands back: one thread each
     ALLOC(c, c->l_done, np);
     ALLOC(c, c->l_big, np * 4 * (LW_BUCKETS + 2));
     ALLOC(c, c->l_crowd, np);
@@ -1352,6 +1352,7 @@ static int search_batch(oic_ctx *c, uint32_t s0, uint32_t ns, const std::vector<
                        c->l_crowd.as<uint8_t>(), lists + LW_BUCKETS * np, cnt + 8);
     BigListArgs BA;
     BA.pairs = c->p_pairs.as<PairRec>();
+    BA.np = np;
     BA.big = c->l_big.as<uint32_t>();
     BA.nbig = cnt;
     BA.bcnt = cnt + 12;
@@ -1374,15 +1375,23 @@ static int search_batch(oic_ctx *c, uint32_t s0, uint32_t ns, const std::vector<
     B2.next = cnt + 9;
     B2.up = nullptr;
     B2.nup = nullptr;
-    // Second stream, beside the 128-hit level: the one-thread builder for the pairs no wavefront
-    // takes, then (when there are any) the crowded pairs at 512 hits, one wavefront each.
+    // Second stream, beside the 128-hit level: the pairs with fewer hits, at 64 hits per offset, then (when
+    // there are any) the crowded pairs at 512 hits, one wavefront each.
     uint32_t ncrowd = 0;
     HIPCHK(c, hipMemcpyAsync(&ncrowd, cnt + 8, 4, hipMemcpyDeviceToHost, c->st));
     HIPCHK(c, hipStreamSynchronize(c->st));
     HIPCHK(c, hipEventRecord(c->evl[0], c->st));
     HIPCHK(c, hipStreamWaitEvent(c->st2, c->evl[0], 0));
-    hipLaunchKernelGGL(k_build_lists, dim3((unsigned)((np + 127) / 128)), dim3(128), 0, c->st2, c->p_pairs.as<PairRec>(), np, hv,
-                       c->p_tmp.as<int4>(), c->p_nodes.as<int4>(), K, LS, c->l_done.as<uint8_t>(), (uint8_t)0, BA.nnodes_total);
+    BigListArgs BS = BA;
+    BS.np = np;
+    BS.big = nullptr;
+    BS.bcnt = nullptr;
+    BS.next = cnt + 6;
+    BS.handed_back = cnt + 7;
+    BS.up = nullptr;
+    BS.nup = nullptr;
+    hipLaunchKernelGGL(k_build_lists_wave<LW_CAP_SMALL>, dim3((unsigned)std::min<uint64_t>((np + LW_TAKE - 1) / LW_TAKE, 32 * ncu)), dim3(64),
+                       0, c->st2, BS);
     if (ncrowd)
       hipLaunchKernelGGL(k_build_lists_wave<LW_CAP>, dim3((unsigned)std::min<uint64_t>(ncrowd, 4 * ncu)), dim3(64), 0, c->st2, B2);
     HIPCHK(c, hipEventRecord(c->evl[1], c->st2));
@@ -1396,7 +1405,7 @@ static int search_batch(oic_ctx *c, uint32_t s0, uint32_t ns, const std::vector<
     B3.next = cnt + 11;
     hipLaunchKernelGGL(k_build_lists_wave<LW_CAP>, dim3((unsigned)std::min<uint64_t>(np, 4 * ncu)), dim3(64), 0, c->st, B3);
     HIPCHK(c, hipStreamWaitEvent(c->st, c->evl[1], 0));
-    // pairs a wavefront handed back (an offset of more than 512 hits)
+    // pairs a wavefront handed back (an offset of more than 512 hits, or 64 at the level of few hits)
     hipLaunchKernelGGL(k_build_lists, dim3((unsigned)((np + 127) / 128)), dim3(128), 0, c->st, c->p_pairs.as<PairRec>(), np, hv,
                        c->p_tmp.as<int4>(), c->p_nodes.as<int4>(), K, LS, c->l_done.as<uint8_t>(), (uint8_t)2, BA.nnodes_total);
   }

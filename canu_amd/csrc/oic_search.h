@@ -396,7 +396,8 @@ __global__ void k_pair_ends(PairRec *__restrict__ pairs, uint64_t np, uint64_t n
 }
 
 // Add_Ref + Add_Match (overlapInCore-Find_Overlaps.C:24-96, :104-163), one thread per candidate
-// pair, in O(1) per hit.
+// pair, in O(1) per hit: for the pairs that the wavefront builders below hand back (an offset of more hits
+// than they hold).
 //
 // Add_Match walks the match list from its head.  With hits in (S offset asc, T offset desc) order,
 // the list at S offset o is [nodes touched at o] ++ [nodes touched at o-1, in list order] ++ [dead
@@ -418,7 +419,7 @@ struct ListScratch {
   uint8_t *fl;
 };
 
-// Pairs with done[p] == want: 0 for pairs never given to a wavefront, 2 for pairs a wavefront handed back.
+// Pairs with done[p] == want (2: handed back).
 __global__ void k_build_lists(PairRec *__restrict__ pairs, uint64_t np, const uint64_t *__restrict__ hval, int4 *__restrict__ tmp,
                               int4 *__restrict__ nodes, int32_t K, ListScratch X, const uint8_t *__restrict__ done, uint8_t want,
                               unsigned long long *__restrict__ nnodes_total) {
@@ -519,9 +520,12 @@ __global__ void k_build_lists(PairRec *__restrict__ pairs, uint64_t np, const ui
   pairs[p] = pr;
 }
 
-// The same list, built by one wavefront per pair for pairs with many hits (satellite and repeat
-// pairs reach millions).  Offsets are still taken in order, but the hits of one offset are handled
-// by all lanes at once, with the live nodes in LDS:
+// The same list, built by one wavefront per pair.  Offsets that hold one hit each (nearly all of a plain
+// overlap's) are taken up to 64 at once while at most one node is live: the nodes are then the runs of hits that
+// continue one another on a diagonal.  One thread per pair, the form above, took 2 us a hit, a chain of dependent
+// loads: the list stage of a batch lasted 4 ms or more however few its pairs, 17 ms for 83 thousand pairs of
+// 4 %-error reads; this way 0.2 and 4.7 ms.  Other offsets are taken in order, the hits of one offset by all lanes
+// at once, with the live nodes in LDS:
 //   - a hit's node is found by binary search over the live diagonals (descending);
 //   - with t(k) = index of the hit touching the node at list position k (INF if none), the node
 //     of hit j moves to the front iff max(t(0..k-1)) > j, i.e. some node before it is not yet
@@ -537,6 +541,8 @@ __global__ void k_build_lists(PairRec *__restrict__ pairs, uint64_t np, const ui
 // (the 512-hit kernel), or, from the last level, back to the one-thread builder (done[p] = 2).
 #define LW_CAP 512        // hits per offset of the last wavefront level
 #define LW_CAP_FIRST 128  // of the first: a quarter of the LDS, four times the wavefronts per CU
+#define LW_CAP_SMALL 64   // of the level for pairs with few hits in all
+#define LW_TAKE 4         // pairs a wavefront of that level takes from the queue at once
 
 __device__ __forceinline__ int32_t wave_incl_max_i32(int32_t v) {
   const int lane = threadIdx.x & 63;
@@ -562,6 +568,7 @@ __device__ __forceinline__ int32_t wave_min_i32(int32_t v) {
 
 struct BigListArgs {
   PairRec *pairs;
+  uint64_t np;              // if big is null: all pairs p < np with done[p] == 0, LW_TAKE at a time
   const uint32_t *big;      // indices of pairs with many hits
   const uint32_t *nbig;
   const uint32_t *bcnt;     // if not null: big holds LW_BUCKETS lists of bstride entries, bcnt[b]
@@ -570,7 +577,7 @@ struct BigListArgs {
   uint32_t *handed_back;    // pairs left to the one-thread builder
   uint32_t *up;             // if not null: pairs too crowded for this level go here, for the next one
   uint32_t *nup;
-  uint8_t *done;            // per pair: 0 = one-thread builder, 1 = a wavefront builds it, 2 = handed back
+  uint8_t *done;            // per pair: 0 = level of few hits, 1 = level of many hits, 2 = handed back
   unsigned long long *nnodes_total;
   const uint64_t *hval;
   int4 *tmp;
@@ -630,28 +637,38 @@ __global__ void __launch_bounds__(64) k_build_lists_wave(BigListArgs A) {
   __shared__ int32_t sQ[CAP > LW_CAP_FIRST ? CAP : 1];    // per hit: live index of its node, or -1 (512-hit level)
   __shared__ int32_t sRk[CAP > LW_CAP_FIRST ? CAP : 1];   // per hit: 2 x rank among created / moved hits, +1 if it is one
   __shared__ int32_t sIp[CAP];      // per list position: rank among nodes extended in place
-  __shared__ uint64_t sW[128];      // hit values [wb, wb + 128) of the pair, refilled every 64 hits
+  __shared__ uint64_t sW[128];      // hit values [wb, wb + 128) of the pair, hit hh at (hh - hb) mod 128
   __shared__ uint32_t sWork;
   const int lane = threadIdx.x;
   const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
   const int32_t INF = 0x7fffffff;
   const int32_t K = A.K;
-  const uint32_t nbig = *A.nbig;
+  const uint32_t nbig = A.big ? *A.nbig : (uint32_t)((A.np + LW_TAKE - 1) / LW_TAKE);
+  uint32_t work = 0, more = 0;      // pairs of a queue entry still to do (the small level)
   for (;;) {
-    if (lane == 0) sWork = atomicAdd(A.next, 1u);
-    __syncthreads();
-    const uint32_t w = sWork;
-    __syncthreads();
-    if (w >= nbig) break;
     uint32_t p;
-    if (A.bcnt) {
-      uint32_t r = w;
-      int k = 0;
-      while (k < LW_BUCKETS - 1 && r >= A.bcnt[k]) r -= A.bcnt[k++];
-      p = A.big[(uint64_t)k * A.bstride + r];
+    if (more) {
+      p = ++work;
+      more--;
     } else {
-      p = A.big[w];
+      if (lane == 0) sWork = atomicAdd(A.next, 1u);
+      __syncthreads();
+      const uint32_t w = sWork;
+      __syncthreads();
+      if (w >= nbig) break;
+      if (!A.big) {
+        p = work = w * LW_TAKE;
+        more = LW_TAKE - 1;
+      } else if (A.bcnt) {
+        uint32_t r = w;
+        int k = 0;
+        while (k < LW_BUCKETS - 1 && r >= A.bcnt[k]) r -= A.bcnt[k++];
+        p = A.big[(uint64_t)k * A.bstride + r];
+      } else {
+        p = A.big[w];
+      }
     }
+    if (!A.big && (p >= A.np || A.done[p] != 0)) continue;
     PairRec pr = A.pairs[p];
     const uint64_t hb = pr.hb, he = pr.he;
     int4 *dq = A.tmp + hb;
@@ -659,46 +676,90 @@ __global__ void __launch_bounds__(64) k_build_lists_wave(BigListArgs A) {
     int32_t nA = 0, nnode = 0, ndq = 0, maxm = 0, prev_o = -2;
     bool consistent = true, over = false;
     int4 head = make_int4(0, 0, 0, 0);
-    uint64_t h = hb, wb = hb;
-    auto fill = [&]() {   // the window from wb (hits past the pair's end read as 0, never used)
-      for (int i = lane; i < 128; i += 64) sW[i] = (wb + (uint64_t)i < he) ? A.hval[wb + i] : 0ull;
+    uint64_t h = hb, wb = hb, ahead = 0;   // ahead: this lane's hit of [wb + 128, wb + 192), on its way
+    auto load = [&](uint64_t hh) -> uint64_t { return hh < he ? A.hval[hh] : 0ull; };   // past the pair's end: 0, never used
+    auto fill = [&]() {
+      sW[(wb - hb + lane) & 127] = load(wb + lane);
+      sW[(wb - hb + 64 + lane) & 127] = load(wb + 64 + lane);
+      ahead = load(wb + 128 + lane);
       __syncthreads();
     };
     // hit value hh of the pair: from the window when it holds it
-    auto hit = [&](uint64_t hh) -> uint64_t { return (hh - wb < 128) ? sW[hh - wb] : A.hval[hh]; };
+    auto hit = [&](uint64_t hh) -> uint64_t { return (hh - wb < 128) ? sW[(hh - hb) & 127] : A.hval[hh]; };
     fill();
     while (h < he) {
       if (h - wb >= 64) {   // keep [h, h + 64) in the window
         __syncthreads();
-        wb = h;
-        fill();
-      }
-      if (nA == 1) {
-        // The next offsets, each holding one hit on the live node's diagonal, only extend that node
-        // (the one-hit step below, with nothing dying and nothing created): take up to 64 at once.
-        // Hit h + lane and h + lane + 1 lie in the window ([h, h + 64) is held, the window is 128).
-        const uint64_t hh = h + (uint64_t)lane;
-        bool ext = false;
-        uint64_t v = 0;
-        if (hh < he) {
-          v = sW[hh - wb];
-          const int32_t oi = (int32_t)(v & 0x1fffff);
-          const int32_t gi = (int32_t)((v >> 21) & 0x1fffff) - oi;
-          const bool single = hh + 1 >= he || (int32_t)(sW[hh + 1 - wb] & 0x1fffff) != oi;
-          ext = oi == prev_o + 1 + lane && gi == sLd[cur][0] && single;
-        }
-        const uint64_t b = __ballot(ext);
-        const int32_t r = (b == ~0ull) ? 64 : __builtin_ctzll(~b);
-        if (r > 0) {
-          if (lane < r) maxm = max(maxm, (int32_t)(v >> 42));
-          if (lane == 0) sR[cur][0].y += r;
+        if (h - wb >= 128) {
+          wb = hb + ((h - hb) & ~63ull);
+          fill();
+        } else {
+          sW[(wb - hb + lane) & 127] = ahead;   // the 64 hits after the window take the place of its first 64
+          wb += 64;
+          ahead = load(wb + 128 + lane);
           __syncthreads();
+        }
+      }
+      if (nA <= 1) {
+        // The next offsets that hold one hit each, up to 64 of them at once.  With at most one node live, such
+        // a hit either extends it (the next offset, the same diagonal) or makes a node, the live one dying; so
+        // the nodes are the runs of hits between those that do not continue the hit before.
+        const uint64_t hh = h + (uint64_t)lane;
+        const bool in = hh < he;
+        const uint64_t v = in ? sW[(hh - hb) & 127] : 0ull;
+        const int32_t oi = (int32_t)(v & 0x1fffff), gi = (int32_t)((v >> 21) & 0x1fffff) - oi;
+        int32_t op = __shfl_up(oi, 1), gp = __shfl_up(gi, 1);
+        const int32_t on = hh + 1 < he ? (int32_t)(sW[(hh + 1 - hb) & 127] & 0x1fffff) : -1;
+        if (lane == 0) { op = prev_o; gp = nA ? sLd[cur][0] : 0; }
+        const uint64_t bs = __ballot(in && on != oi);          // single: hit h starts an offset, as the invariant
+        const int32_t r = (bs == ~0ull) ? 64 : __builtin_ctzll(~bs);
+        if (r > 0) {
+          const bool mine = lane < r;
+          const bool cont = mine && oi == op + 1 && gi == gp && (lane > 0 || nA > 0);
+          const uint64_t M = __ballot(mine && !cont);           // hits that make a node
+          if (mine) maxm = max(maxm, (int32_t)(v >> 42));
+          // a node made with one live, or (none live) away from the last one's end, ends consistency
+          const bool first = nnode == 0 && lane == 0;
+          const bool bad = mine && !cont && !first && (oi == op + 1 || abs(gp - gi) > 3 || oi < op + 1 + K - 2);
+          if (__ballot(bad)) consistent = false;
+          const int32_t nb = (int32_t)__popcll(M), ext = M ? __builtin_ctzll(M) : r;   // ext: hits that extend the live node
+          const int32_t died = nA == 1 && nb > 0 ? 1 : 0;
+          int4 live = make_int4(0, 0, 0, 0);
+          if (nA == 1) {
+            live = sR[cur][0];
+            live.y += ext;
+          }
+          if (lane == 0 && died) {
+            int4 rec = live;
+            rec.w = ndq + 1;
+            dq[ndq] = rec;
+          }
+          if ((M >> lane) & 1) {
+            const uint64_t after = lane == 63 ? 0ull : (M >> (lane + 1)) << (lane + 1);
+            const int32_t end = after ? __builtin_ctzll(after) : r;
+            const int32_t at = ndq + died + (int32_t)__popcll(M & lt);
+            int4 rec = make_int4(gi + oi, K + end - lane - 1, oi, at + 1);
+            if (after) {
+              dq[at] = rec;
+            } else {
+              rec.w = 0;
+              sR[cur][0] = rec;
+              sLd[cur][0] = gi;
+              sLq[cur][0] = 0;
+            }
+          } else if (lane == 0 && nb == 0) {
+            sR[cur][0] = live;
+          }
+          __syncthreads();
+          ndq += died + (nb > 0 ? nb - 1 : 0);
+          nnode += nb;
+          prev_o = __shfl(oi, r - 1);
+          nA = 1;
           h += (uint64_t)r;
-          prev_o += r;
           continue;
         }
       }
-      const int32_t o = (int32_t)(sW[h - wb] & 0x1fffff);
+      const int32_t o = (int32_t)(sW[(h - hb) & 127] & 0x1fffff);
       int32_t c = 0;
       for (;;) {
         const uint64_t hh = h + (uint64_t)c + (uint64_t)lane;

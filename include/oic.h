@@ -130,7 +130,7 @@ typedef struct oic_counters {
   uint64_t fwd_cells;          /* cells and bases of those launches */
   uint64_t fwd_bases;
   uint64_t graphs_launched;    /* forward-pass hipGraphs launched */
-  uint64_t list_wave_pairs;    /* pairs whose match list one wavefront built */
+  uint64_t list_wave_pairs;    /* pairs whose match list the 128-hit wavefront level built */
   uint64_t list_handed_back;   /* of those, pairs with an offset of more hits than the wavefront holds */
   uint64_t list_second_level;  /* of those, pairs taken on by the 512-hit wavefront level (an offset
                                   with more than 128 hits) */
@@ -155,8 +155,8 @@ typedef struct oic_counters {
 /* Launch-shape knobs.  No setting changes a result; the defaults suit MI355X.  No reference
  * counterpart: overlapInCore has no device work to shape. */
 typedef struct oic_tuning {
-  uint32_t list_wave_min_hits;  /* pairs with at least this many seed hits build their match list
-                                   with one wavefront, smaller ones with one thread (default 2048) */
+  uint32_t list_wave_min_hits;  /* pairs with at least this many seed hits build their match list at the
+                                   128-hit wavefront level, smaller ones at a 64-hit one (default 2048) */
   uint32_t fwd_lanes;           /* lanes per packed forward DP: 1 (64 DPs per wavefront, each lane
                                    walking its own band cell by cell), or 4, 8, 16 or 32 (64/fwd_lanes
                                    DPs per wavefront, rows spread over the group; default 4) */
