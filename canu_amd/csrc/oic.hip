@@ -110,7 +110,7 @@ struct oic_ctx {
   DevBuf s_k1, s_v1, s_k2, s_v2, s_scan, s_flag, s_idx, s_small, s_rp;
   // search
   DevBuf g_cnt, g_off, g_pbase, g_searched, g_sdsum, g_phi, g_pval;
-  DevBuf l_scr, l_done, l_big, l_cnt, l_crowd;
+  DevBuf l_scr, l_done, l_big, l_cnt, l_split, l_items;
   std::vector<uint64_t> skip;           // -k skip k-mers, both strands, sorted, unique
   DevBuf d_skip, x_tscreen, g_sscreen;
   oic_tuning tune{};
@@ -1336,27 +1336,31 @@ static int search_batch(oic_ctx *c, uint32_t s0, uint32_t ns, const std::vector<
     LS.sA = b; LS.sB = b + H; LS.oA = b + 2 * H; LS.oB = b + 3 * H; LS.fr = b + 4 * H; LS.dq = b + 5 * H; LS.db = b + 6 * H;
     LS.pos = b + 7 * H;
     LS.fl = (uint8_t *)(b + 8 * H);
-    // one wavefront per pair, at a level by its hits; pairs that one hands back: one thread each
+    // one wavefront per pair, at a level by its hits, and several for a long one; pairs that one hands back: one
+    // thread each
+    const uint64_t ntile = (H + LW_SPLIT - 1) / LW_SPLIT;
+    const uint64_t nlong = H / LW_LONG + 1;              // long pairs at most
     ALLOC(c, c->l_done, np);
-    ALLOC(c, c->l_big, np * 4 * (LW_BUCKETS + 2));
-    ALLOC(c, c->l_crowd, np);
-    hipLaunchKernelGGL(k_fill_u8, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, c->st, c->l_crowd.as<uint8_t>(), np);
-    hipLaunchKernelGGL(k_crowded_pairs, dim3((unsigned)((H + 255) / 256)), dim3(256), 0, c->st, hk, hv, c->s_flag.as<uint32_t>(),
-                       c->s_idx.as<uint64_t>(), H, c->l_crowd.as<uint8_t>());
+    ALLOC(c, c->l_big, (2 * np + ntile + 4 * nlong) * 4);       // big, up (pairs and parts), long pairs and their parts
+    ALLOC(c, c->l_split, ntile * 8);
+    ALLOC(c, c->l_items, (ntile + nlong) * sizeof(ListItem));   // at most one part begins in a tile, and one at a pair's start
     ALLOC(c, c->l_cnt, 64);
     HIPCHK(c, hipMemsetAsync(c->l_cnt.p, 0, 64, c->st));
+    // cnt: [0] big pairs, [1] their queue, [2] handed back, [4..5] nodes, [6] queue of few hits, [7] handed back
+    // there, [8] long pairs, [9] parts, [10] pairs and parts with over 128 hits at an offset, [11] their queue
     uint32_t *cnt = c->l_cnt.as<uint32_t>();
-    uint32_t *lists = c->l_big.as<uint32_t>();
+    uint32_t *big = c->l_big.as<uint32_t>(), *up = big + np, *lng = up + np + ntile + nlong, *lfirst = lng + nlong, *lcount = lfirst + nlong;
     hipLaunchKernelGGL(k_big_select, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, c->st, c->p_pairs.as<PairRec>(), np,
-                       (uint64_t)c->tune.list_wave_min_hits, c->l_done.as<uint8_t>(), lists, cnt, cnt + 12,
-                       c->l_crowd.as<uint8_t>(), lists + LW_BUCKETS * np, cnt + 8);
-    BigListArgs BA;
+                       (uint64_t)c->tune.list_wave_min_hits, c->l_done.as<uint8_t>(), big, cnt, lng, cnt + 8);
+    hipLaunchKernelGGL(k_list_splits, dim3((unsigned)((ntile + 3) / 4)), dim3(256), 0, c->st, c->p_pairs.as<PairRec>(), c->s_flag.as<uint32_t>(),
+                       c->s_idx.as<uint64_t>(), c->l_done.as<uint8_t>(), hv, H, c->l_split.as<uint64_t>());
+    BigListArgs BA{};
     BA.pairs = c->p_pairs.as<PairRec>();
     BA.np = np;
-    BA.big = c->l_big.as<uint32_t>();
+    BA.big = big;
     BA.nbig = cnt;
-    BA.bcnt = cnt + 12;
-    BA.bstride = np;
+    BA.items = c->l_items.as<ListItem>();
+    BA.nitems = cnt + 9;
     BA.next = cnt + 1;
     BA.handed_back = cnt + 2;
     BA.done = c->l_done.as<uint8_t>();
@@ -1366,44 +1370,43 @@ static int search_batch(oic_ctx *c, uint32_t s0, uint32_t ns, const std::vector<
     BA.nodes = c->p_nodes.as<int4>();
     BA.K = K;
     const uint64_t ncu = (uint64_t)std::max(c->ncu, 1);
-    // crowded pairs (an offset of more than 128 hits): the 512-hit level, on the second stream,
-    // beside the first level; the two take disjoint pairs
-    BigListArgs B2 = BA;
-    B2.big = lists + LW_BUCKETS * np;
-    B2.nbig = cnt + 8;
-    B2.bcnt = nullptr;
-    B2.next = cnt + 9;
-    B2.up = nullptr;
-    B2.nup = nullptr;
-    // Second stream, beside the 128-hit level: the pairs with fewer hits, at 64 hits per offset, then (when
-    // there are any) the crowded pairs at 512 hits, one wavefront each.
-    uint32_t ncrowd = 0;
-    HIPCHK(c, hipMemcpyAsync(&ncrowd, cnt + 8, 4, hipMemcpyDeviceToHost, c->st));
-    HIPCHK(c, hipStreamSynchronize(c->st));
-    HIPCHK(c, hipEventRecord(c->evl[0], c->st));
-    HIPCHK(c, hipStreamWaitEvent(c->st2, c->evl[0], 0));
+    // Second stream, beside the others: the pairs with fewer hits, at 64 hits per offset.
     BigListArgs BS = BA;
-    BS.np = np;
     BS.big = nullptr;
-    BS.bcnt = nullptr;
+    BS.nitems = nullptr;
     BS.next = cnt + 6;
     BS.handed_back = cnt + 7;
-    BS.up = nullptr;
-    BS.nup = nullptr;
+    HIPCHK(c, hipEventRecord(c->evl[0], c->st));
+    HIPCHK(c, hipStreamWaitEvent(c->st2, c->evl[0], 0));
     hipLaunchKernelGGL(k_build_lists_wave<LW_CAP_SMALL>, dim3((unsigned)std::min<uint64_t>((np + LW_TAKE - 1) / LW_TAKE, 32 * ncu)), dim3(64),
                        0, c->st2, BS);
-    if (ncrowd)
-      hipLaunchKernelGGL(k_build_lists_wave<LW_CAP>, dim3((unsigned)std::min<uint64_t>(ncrowd, 4 * ncu)), dim3(64), 0, c->st2, B2);
     HIPCHK(c, hipEventRecord(c->evl[1], c->st2));
-    // first level: up to 128 hits per offset; a pair it still finds crowded runs at 512 hits after it
-    BA.up = lists + (LW_BUCKETS + 1) * np;
+    uint32_t nl = 0;
+    HIPCHK(c, hipMemcpyAsync(&nl, cnt + 8, 4, hipMemcpyDeviceToHost, c->st));
+    HIPCHK(c, hipStreamSynchronize(c->st));
+    uint32_t nit = 0;
+    if (nl) {
+      hipLaunchKernelGGL(k_list_items, dim3(nl), dim3(OIC_WAVE), 0, c->st, BA.pairs, lng, c->l_split.as<uint64_t>(), BA.items, cnt + 9, lfirst,
+                         lcount);
+      HIPCHK(c, hipMemcpyAsync(&nit, cnt + 9, 4, hipMemcpyDeviceToHost, c->st));
+    }
+    // first level: up to 128 hits per offset; what it finds more crowded runs at 512 hits after it
+    BA.up = up;
     BA.nup = cnt + 10;
-    hipLaunchKernelGGL(k_build_lists_wave<LW_CAP_FIRST>, dim3((unsigned)std::min<uint64_t>(np, 16 * ncu)), dim3(64), 0, c->st, BA);
-    BigListArgs B3 = B2;
-    B3.big = BA.up;
-    B3.nbig = BA.nup;
+    hipLaunchKernelGGL(k_build_lists_wave<LW_CAP_FIRST>, dim3((unsigned)std::min<uint64_t>(np + ntile, 16 * ncu)), dim3(64), 0, c->st, BA);
+    BigListArgs B3 = BA;
+    B3.big = up;
+    B3.nbig = cnt + 10;
+    B3.nitems = nullptr;
     B3.next = cnt + 11;
-    hipLaunchKernelGGL(k_build_lists_wave<LW_CAP>, dim3((unsigned)std::min<uint64_t>(np, 4 * ncu)), dim3(64), 0, c->st, B3);
+    B3.up = nullptr;
+    B3.nup = nullptr;
+    hipLaunchKernelGGL(k_build_lists_wave<LW_CAP>, dim3((unsigned)std::min<uint64_t>(np + ntile, 4 * ncu)), dim3(64), 0, c->st, B3);
+    if (nl) {
+      HIPCHK(c, hipStreamSynchronize(c->st));   // nit
+      hipLaunchKernelGGL(k_list_join, dim3(nl), dim3(OIC_WAVE), 0, c->st, BA, lng, lfirst, lcount);
+      hipLaunchKernelGGL(k_list_copy, dim3((nit + 3) / 4), dim3(256), 0, c->st, BA, nit);
+    }
     HIPCHK(c, hipStreamWaitEvent(c->st, c->evl[1], 0));
     // pairs a wavefront handed back (an offset of more than 512 hits, or 64 at the level of few hits)
     hipLaunchKernelGGL(k_build_lists, dim3((unsigned)((np + 127) / 128)), dim3(128), 0, c->st, c->p_pairs.as<PairRec>(), np, hv,
@@ -1414,9 +1417,9 @@ static int search_batch(oic_ctx *c, uint32_t s0, uint32_t ns, const std::vector<
     uint32_t lc[16];
     HIPCHK(c, hipMemcpyAsync(lc, c->l_cnt.p, 64, hipMemcpyDeviceToHost, c->st));
     HIPCHK(c, hipStreamSynchronize(c->st));
-    c->ctr.list_wave_pairs += lc[0];
+    c->ctr.list_wave_pairs += lc[0] + lc[8];
     c->ctr.list_handed_back += lc[2];
-    c->ctr.list_second_level += lc[8] + lc[10];
+    c->ctr.list_second_level += lc[10];
     memcpy(&batch_nodes, lc + 4, 8);
     c->ctr.nodes += batch_nodes;
   }

@@ -543,6 +543,8 @@ __global__ void k_build_lists(PairRec *__restrict__ pairs, uint64_t np, const ui
 #define LW_CAP_FIRST 128  // of the first: a quarter of the LDS, four times the wavefronts per CU
 #define LW_CAP_SMALL 64   // of the level for pairs with few hits in all
 #define LW_TAKE 4         // pairs a wavefront of that level takes from the queue at once
+#define LW_SPLIT 1024     // hits per part of a long pair, or up to the next gap
+#define LW_LONG 8192      // hits from which a pair is built in parts: below, one wavefront takes 0.2 ms at most
 
 __device__ __forceinline__ int32_t wave_incl_max_i32(int32_t v) {
   const int lane = threadIdx.x & 63;
@@ -566,16 +568,29 @@ __device__ __forceinline__ int32_t wave_min_i32(int32_t v) {
   return v;
 }
 
+// A part of a long pair's hits, from one gap in its S offsets to another.  At a gap every live node dies, so a
+// part's list is built on its own; the pair's list is its parts' lists, the last part's first.  One wavefront per
+// pair, 92 thousand pairs of repeat-rich reads took 18.8 ms of which the largest, a satellite pair of some
+// thousand crowded offsets, took nearly all; in parts 6.2 ms.
+struct ListItem {
+  uint64_t b, e;            // its hits
+  uint64_t dst;             // its list's place in the pair's
+  uint32_t pair;
+  int32_t nn, consistent, longest, first_longest, dmin, dmax, maxm;
+  int4 head;                // its list's first node
+};
+#define LW_ITEM 0x80000000u   // marks a part's index in a list of work
+
 struct BigListArgs {
   PairRec *pairs;
   uint64_t np;              // if big is null: all pairs p < np with done[p] == 0, LW_TAKE at a time
-  const uint32_t *big;      // indices of pairs with many hits
+  const uint32_t *big;      // pairs, or parts (LW_ITEM), to build
   const uint32_t *nbig;
-  const uint32_t *bcnt;     // if not null: big holds LW_BUCKETS lists of bstride entries, bcnt[b]
-  uint64_t bstride;         //   of them used, taken in bucket order (largest pairs first)
+  ListItem *items;
+  const uint32_t *nitems;   // if not null: parts 0 .. *nitems follow the list's entries
   uint32_t *next;           // work counter, starts at 0
   uint32_t *handed_back;    // pairs left to the one-thread builder
-  uint32_t *up;             // if not null: pairs too crowded for this level go here, for the next one
+  uint32_t *up;             // if not null: pairs and parts too crowded for this level go here, for the next one
   uint32_t *nup;
   uint8_t *done;            // per pair: 0 = level of few hits, 1 = level of many hits, 2 = handed back
   unsigned long long *nnodes_total;
@@ -585,46 +600,150 @@ struct BigListArgs {
   int32_t K;
 };
 
-__global__ void k_fill_u8(uint8_t *__restrict__ p, uint64_t n) {
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = 0;
-}
-
-// Pairs with an S offset of more than LW_CAP_FIRST hits (crowded[p] = 1).  Within a pair, hits are in
-// S-offset order, so an offset holds more than LW_CAP_FIRST of them exactly when some hit i and hit
-// i + LW_CAP_FIRST have the same pair key and the same offset.  keys are the pair-grouped hit keys,
-// flag marks each pair's first hit and idx is the exclusive scan of flag.
-__global__ void k_crowded_pairs(const uint64_t *__restrict__ keys, const uint64_t *__restrict__ hval,
-                                const uint32_t *__restrict__ flag, const uint64_t *__restrict__ idx, uint64_t n,
-                                uint8_t *__restrict__ crowded) {
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i + LW_CAP_FIRST >= n) return;
-  const uint64_t v = hval[i];
-  if ((v >> 42) <= LW_CAP_FIRST) return;   // a k-mer with no more occurrences cannot crowd an offset
-  const uint64_t j = i + LW_CAP_FIRST;
-  if (keys[j] == keys[i] && (hval[j] & 0x1fffff) == (v & 0x1fffff)) crowded[idx[i] + flag[i] - 1] = 1;
-}
-
-// Pairs for the wavefront builder, bucketed by hit count (>= 2^17, 2^14, 2^11, the rest) so that
-// the largest, whose offsets run one after another, start first and do not end the launch late.
-// Crowded pairs go to the 512-hit level's list (up) directly.
-#define LW_BUCKETS 4
+// Pairs by level: fewer than min_hits hits (done 0), whole (big), or in parts (long).
 __global__ void k_big_select(const PairRec *__restrict__ pairs, uint64_t np, uint64_t min_hits, uint8_t *__restrict__ done,
-                             uint32_t *__restrict__ big, uint32_t *__restrict__ nbig, uint32_t *__restrict__ bcnt,
-                             const uint8_t *__restrict__ crowded, uint32_t *__restrict__ up, uint32_t *__restrict__ nup) {
+                             uint32_t *__restrict__ big, uint32_t *__restrict__ nbig, uint32_t *__restrict__ lng,
+                             uint32_t *__restrict__ nlng) {
   const uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= np) return;
   const uint64_t nh = pairs[p].he - pairs[p].hb;
   const bool b = nh >= min_hits;
   done[p] = b ? 1 : 0;
   if (!b) return;
-  if (crowded[p]) {
-    up[atomicAdd(nup, 1u)] = (uint32_t)p;
-    return;
+  if (nh >= LW_LONG) lng[atomicAdd(nlng, 1u)] = (uint32_t)p;
+  else big[atomicAdd(nbig, 1u)] = (uint32_t)p;
+}
+
+// One wavefront per LW_SPLIT hits (tile t: hits from t LW_SPLIT on): the first hit in the tile at which a part of
+// a long pair can begin, an S offset after a gap; ~0 where there is none.  flag marks each pair's first hit, idx
+// is the exclusive scan of flag.
+__global__ void __launch_bounds__(256) k_list_splits(const PairRec *__restrict__ pairs, const uint32_t *__restrict__ flag,
+                                                     const uint64_t *__restrict__ idx, const uint8_t *__restrict__ done,
+                                                     const uint64_t *__restrict__ hval, uint64_t n, uint64_t *__restrict__ split) {
+  const uint64_t t = (uint64_t)blockIdx.x * (blockDim.x / OIC_WAVE) + threadIdx.x / OIC_WAVE, B = t * LW_SPLIT;
+  if (B >= n) return;
+  const int lane = lane_id();
+  const uint64_t p = idx[B] + flag[B] - 1;
+  const uint64_t hb = pairs[p].hb, he = pairs[p].he;
+  uint64_t at = ~0ull;
+  if (done[p] == 1 && he - hb >= LW_LONG) {
+    const uint64_t lo = B > hb ? B : hb + 1, hi = B + LW_SPLIT < he ? B + LW_SPLIT : he;
+    for (uint64_t i0 = lo; i0 < hi; i0 += OIC_WAVE) {
+      const uint64_t i = i0 + lane;
+      const bool gap = i < hi && (hval[i] & 0x1fffff) > (hval[i - 1] & 0x1fffff) + 1;
+      const uint64_t b = __ballot(gap);
+      if (b) { at = i0 + __builtin_ctzll(b); break; }
+    }
   }
-  const int k = nh >= (1u << 17) ? 0 : nh >= (1u << 14) ? 1 : nh >= (1u << 11) ? 2 : 3;
-  big[(uint64_t)k * np + atomicAdd(&bcnt[k], 1u)] = (uint32_t)p;
-  atomicAdd(nbig, 1u);
+  if (lane == 0) split[t] = at;
+}
+
+// One wavefront per long pair: its parts, numbered in order from first[j]; count[j] of them.
+__global__ void __launch_bounds__(OIC_WAVE) k_list_items(const PairRec *__restrict__ pairs, const uint32_t *__restrict__ lng,
+                                                         const uint64_t *__restrict__ split, ListItem *__restrict__ items,
+                                                         uint32_t *__restrict__ nitems, uint32_t *__restrict__ first,
+                                                         uint32_t *__restrict__ count) {
+  const int lane = lane_id();
+  const uint32_t j = blockIdx.x, p = lng[j];
+  const uint64_t hb = pairs[p].hb, he = pairs[p].he;
+  const uint64_t t0 = (hb + LW_SPLIT - 1) / LW_SPLIT, t1 = (he - 1) / LW_SPLIT + 1;
+  uint32_t n = 1;
+  for (uint64_t t = t0; t < t1; t += OIC_WAVE)
+    n += (uint32_t)__builtin_popcountll(__ballot(t + lane < t1 && split[t + lane] != ~0ull));
+  uint32_t id = 0;
+  if (lane == 0) {
+    id = atomicAdd(nitems, n);
+    first[j] = id;
+    count[j] = n;
+    items[id].b = hb;
+    items[id].pair = p;
+    items[id + n - 1].e = he;
+  }
+  id = (uint32_t)uni((int32_t)id);
+  for (uint64_t t = t0; t < t1; t += OIC_WAVE) {
+    const uint64_t at = t + lane < t1 ? split[t + lane] : ~0ull;
+    const uint64_t b = __ballot(at != ~0ull);
+    if (at != ~0ull) {
+      const uint32_t k = id + (uint32_t)__builtin_popcountll(b & ((1ull << lane) - 1));
+      items[k].e = at;
+      items[k + 1].b = at;
+      items[k + 1].pair = p;
+    }
+    id += (uint32_t)__builtin_popcountll(b);
+  }
+}
+
+// One wavefront per long pair: its parts' places in its list, and its record.  A part's first node is made with no
+// node live: the pair stays consistent there if the head of the list so far, the part before's first node, lies
+// within 3 diagonals and ends near (Add_Match's test, overlapInCore-Find_Overlaps.C:104-163).
+__global__ void __launch_bounds__(OIC_WAVE) k_list_join(BigListArgs A, const uint32_t *__restrict__ lng, const uint32_t *__restrict__ first,
+                                                        const uint32_t *__restrict__ count) {
+  const int lane = lane_id();
+  const uint32_t j = blockIdx.x, p = lng[j];
+  if (A.done[p] == 2) return;
+  PairRec pr = A.pairs[p];
+  ListItem *it = A.items + first[j];
+  const int32_t n = (int32_t)count[j];
+  uint64_t at = 0, key = 0;                     // key: Len << 32 | ~position, its maximum the first longest node
+  int32_t dmin = 0x7fffffff, dmax = -0x7fffffff, maxm = 0;
+  bool consistent = true;
+  for (int32_t i0 = 0; i0 < n; i0 += OIC_WAVE) {
+    const int32_t k = n - 1 - (i0 + lane);      // list order: the last part first
+    int32_t nn = 0;
+    ListItem x;
+    if (k >= 0) { x = it[k]; nn = x.nn; }
+    const int32_t inc = wave_incl_scan(nn);
+    if (k >= 0) {
+      const uint64_t dst = at + (uint64_t)(inc - nn);
+      it[k].dst = dst;
+      const uint64_t f = ((uint64_t)(uint32_t)x.longest << 32) | (uint32_t)~(uint32_t)(dst + x.first_longest);
+      key = f > key ? f : key;
+      dmin = x.dmin < dmin ? x.dmin : dmin;
+      dmax = x.dmax > dmax ? x.dmax : dmax;
+      maxm = x.maxm > maxm ? x.maxm : maxm;
+      bool bad = !x.consistent;
+      if (k > 0) {
+        const int4 hd = it[k - 1].head;
+        const uint64_t v = A.hval[x.b];
+        const int32_t o = (int32_t)(v & 0x1fffff), g = (int32_t)((v >> 21) & 0x1fffff) - o;
+        const int32_t es = hd.z + hd.y - A.K + 1, dg = hd.x - hd.z;
+        if (abs(dg - g) > 3 || o < es + A.K - 2) bad = true;
+      }
+      if (bad) consistent = false;
+    }
+    at += (uint64_t)(uint32_t)__builtin_amdgcn_readlane(inc, OIC_WAVE - 1);
+  }
+  for (int o = 32; o > 0; o >>= 1) {
+    const uint64_t f = __shfl_xor(key, o);
+    key = f > key ? f : key;
+  }
+  dmin = wave_min_i32(dmin);
+  dmax = wave_max_i32(dmax);
+  maxm = wave_max_i32(maxm);
+  const bool all = __ballot(!consistent) == 0;
+  if (lane == 0) {
+    pr.nnodes = (int32_t)at;
+    atomicAdd(A.nnodes_total, (unsigned long long)at);
+    pr.consistent = all ? 1 : 0;
+    pr.diag_bgn = (int32_t)(A.hval[pr.hb] & 0x1fffff);
+    pr.diag_end = (int32_t)(A.hval[pr.he - 1] & 0x1fffff);
+    pr.max_mult = maxm;
+    pr.longest = (int32_t)(key >> 32);
+    pr.first_longest = (int32_t)~(uint32_t)key;
+    pr.dmin = dmin;
+    pr.dmax = dmax;
+    A.pairs[p] = pr;
+  }
+}
+
+// the parts' lists, from tmp to their places; one wavefront per part
+__global__ void __launch_bounds__(256) k_list_copy(BigListArgs A, uint32_t n) {
+  const uint32_t i = blockIdx.x * (blockDim.x / OIC_WAVE) + threadIdx.x / OIC_WAVE;
+  if (i >= n) return;
+  const ListItem x = A.items[i];
+  if (A.done[x.pair] == 2) return;
+  int4 *out = A.nodes + A.pairs[x.pair].hb + x.dst;
+  for (int32_t k = lane_id(); k < x.nn; k += OIC_WAVE) out[k] = A.tmp[x.b + k];
 }
 
 template <int CAP>
@@ -643,7 +762,8 @@ __global__ void __launch_bounds__(64) k_build_lists_wave(BigListArgs A) {
   const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
   const int32_t INF = 0x7fffffff;
   const int32_t K = A.K;
-  const uint32_t nbig = A.big ? *A.nbig : (uint32_t)((A.np + LW_TAKE - 1) / LW_TAKE);
+  const uint32_t nlist = A.big ? *A.nbig : (uint32_t)((A.np + LW_TAKE - 1) / LW_TAKE);
+  const uint32_t nbig = nlist + (A.nitems ? *A.nitems : 0u);
   uint32_t work = 0, more = 0;      // pairs of a queue entry still to do (the small level)
   for (;;) {
     uint32_t p;
@@ -659,19 +779,19 @@ __global__ void __launch_bounds__(64) k_build_lists_wave(BigListArgs A) {
       if (!A.big) {
         p = work = w * LW_TAKE;
         more = LW_TAKE - 1;
-      } else if (A.bcnt) {
-        uint32_t r = w;
-        int k = 0;
-        while (k < LW_BUCKETS - 1 && r >= A.bcnt[k]) r -= A.bcnt[k++];
-        p = A.big[(uint64_t)k * A.bstride + r];
       } else {
-        p = A.big[w];
+        p = w < nlist ? A.big[w] : (w - nlist) | LW_ITEM;
       }
     }
     if (!A.big && (p >= A.np || A.done[p] != 0)) continue;
+    const bool part = A.big && (p & LW_ITEM);
+    const uint32_t entry = p;
+    ListItem item = {};
+    if (part) { item = A.items[p & ~LW_ITEM]; p = item.pair; }
     PairRec pr = A.pairs[p];
-    const uint64_t hb = pr.hb, he = pr.he;
-    int4 *dq = A.tmp + hb;
+    const uint64_t hb = part ? item.b : pr.hb, he = part ? item.e : pr.he;
+    // a part's list goes to tmp first: its place in the pair's list depends on the parts after it
+    int4 *dq = (part ? A.nodes : A.tmp) + hb;
     int cur = 0;
     int32_t nA = 0, nnode = 0, ndq = 0, maxm = 0, prev_o = -2;
     bool consistent = true, over = false;
@@ -1062,7 +1182,7 @@ __global__ void __launch_bounds__(64) k_build_lists_wave(BigListArgs A) {
     if (over) {
       if (lane == 0) {
         if (A.up) {
-          A.up[atomicAdd(A.nup, 1u)] = p;
+          A.up[atomicAdd(A.nup, 1u)] = entry;
         } else {
           A.done[p] = 2;
           atomicAdd(A.handed_back, 1u);
@@ -1072,7 +1192,7 @@ __global__ void __launch_bounds__(64) k_build_lists_wave(BigListArgs A) {
     }
     __threadfence();
     __syncthreads();
-    int4 *out = A.nodes + hb;
+    int4 *out = (part ? A.tmp : A.nodes) + hb;
     const int4 *R = sR[cur];
     const int32_t *Lq = sLq[cur];
     int32_t longest = 0, dmin = 0x7fffffff, dmax = -0x7fffffff;
@@ -1101,7 +1221,17 @@ __global__ void __launch_bounds__(64) k_build_lists_wave(BigListArgs A) {
     dmin = wave_min_i32(dmin);
     dmax = wave_max_i32(dmax);
     maxm = wave_max_i32(maxm);
-    if (lane == 0) {
+    if (lane == 0 && part) {
+      item.nn = nA + ndq;
+      item.consistent = consistent ? 1 : 0;
+      item.longest = longest;
+      item.first_longest = (int32_t)~(uint32_t)lkey;
+      item.dmin = dmin;
+      item.dmax = dmax;
+      item.maxm = maxm;
+      item.head = R[Lq[0]];
+      A.items[entry & ~LW_ITEM] = item;
+    } else if (lane == 0) {
       pr.nnodes = nA + ndq;
       atomicAdd(A.nnodes_total, (unsigned long long)(nA + ndq));
       pr.consistent = consistent ? 1 : 0;

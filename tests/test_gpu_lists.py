@@ -62,3 +62,24 @@ def test_offsets_of_several_hits_between_blocks(gap, min_hits):
     t = left + unit + rand_seq(rng, gap) + unit + rand_seq(rng, gap) + unit + right
     u = left + unit + other_base(unit[0]) + unit[1:] + right
     check(readsim.from_strings([s, t, u, t[10:]]), min_hits)
+
+
+@pytest.mark.parametrize("min_hits", [None, 0, 16384])
+@pytest.mark.parametrize("copies,errors", [(20, 0), (20, 4), (60, 30), (150, 12), (560, 3)])
+def test_long_pairs_in_parts(copies, errors, min_hits):
+    """Tandem units: an S of 24 copies with errors (gaps in its offsets) against a T of many (that many hits at
+    an offset: below and above 64, 128 and 512), and a plain overlap of 9 kbp, with one gap."""
+    rng = np.random.default_rng(900 + copies + errors)
+    unit, left, right = rand_seq(rng, 33), rand_seq(rng, 300), rand_seq(rng, 300)
+    s = list(left + unit * 24 + right)
+    for p in rng.integers(0, len(s), errors):
+        s[p] = other_base(s[p])
+    t = left + unit * copies + right
+    plain = rand_seq(rng, 9000)
+    spot = 4500 + int(rng.integers(0, 300))
+    R = readsim.from_strings(["".join(s), t, plain, plain[:spot] + other_base(plain[spot]) + plain[spot + 1:]])
+    c = check(R, min_hits)
+    assert c["hits"] > 8192 + 8900
+    if min_hits == 0:
+        assert c["list_wave_pairs"] == c["pairs"]
+        assert (c["list_second_level"] > 0) == (copies > 128) and (c["list_handed_back"] > 0) == (copies > 512)
