@@ -1839,7 +1839,7 @@ __device__ __forceinline__ bool to_next_level(const BatchArgs &A, uint32_t i) {
 
 // Two levels (oic_wdp.h): WR_FIRST leaves the few tasks whose band or rows outgrow it to WR_WIDE.
 template <int RING>
-__global__ void __launch_bounds__(OIC_WAVE) k_dp_batch(BatchArgs A) {
+__global__ void __launch_bounds__(OIC_WAVE) __attribute__((amdgpu_waves_per_eu(4, 8))) k_dp_batch(BatchArgs A) {
   __shared__ WaveBand<RING> band;
   const int lane = lane_id();
   const DPScratch sc = batch_scratch(A, blockIdx.x);

@@ -443,7 +443,7 @@ __global__ void __launch_bounds__(OIC_WAVE) k_fwd_tasks(FwdArgs A) {
 // The same tasks one to a wavefront (oic_wdp.h): the packed kernels' tasks whose band outgrew their tile, then
 // those whose band outgrew the first level.
 template <int RING, bool STATS>
-__global__ void __launch_bounds__(OIC_WAVE) k_fwd_wave(FwdArgs A) {
+__global__ void __launch_bounds__(OIC_WAVE) __attribute__((amdgpu_waves_per_eu(4, 8))) k_fwd_wave(FwdArgs A) {
   __shared__ WaveBand<RING> band;
   const int lane = lane_id();
   const uint32_t ntasks = (uint32_t)uni((int32_t)(A.ntasks_dev ? *A.ntasks_dev : (uint32_t)A.ntasks));

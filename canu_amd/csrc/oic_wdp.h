@@ -14,8 +14,13 @@
 // (barriers between a row's steps, one chunk's slides after another's, two passes for the pruned range, a
 // 12-step shuffle maximum) took about 8000 cycles for the row of a 140-cell band, and its traceback followed
 // the path through HBM, three dependent loads a row on one lane.  Here
-//   * lane l of chunk c holds diagonal 64 c - 32 + l for as long as the DP runs, so a narrow band around
-//     diagonal 0 is one chunk, a chunk's place in the LDS ring is uniform and ballots give diagonals at once;
+//   * a row of up to 64 diagonals stays in one register per lane: neighbours come over DPP shifts, the pruned
+//     range and who slides on are 64-bit scalar masks, and the row never touches LDS.  Most rows of most calls
+//     are such rows (a read pair of 9 % difference keeps about 40 diagonals).  The band moves to the middle of
+//     the lanes when one of its ends reaches lane 0 or 63; from 52 diagonals on it moves to the wide form
+//     instead, and comes back below 40, so that a band near 64 doesn't move at each row;
+//   * in the wide form lane l of chunk c holds diagonal 64 c - 32 + l, so a chunk's place in the LDS ring is
+//     uniform and ballots give diagonals at once;
 //   * the loads of up to WR_GROUP chunks (four words of each tail in one load each: 48 bases or more) are
 //     issued before the first is compared;
 //   * a slide past 48 bases is finished by the whole wavefront, 1024 bases at a time, unless many lanes slide on;
@@ -24,10 +29,11 @@
 //   * a stored cell carries the traceback's choice at that cell in its low two bits.  The traceback loads 32
 //     rows of the 64 diagonals around its own at once and walks them in scalar registers.
 // One wavefront per workgroup: its LDS operations complete in order, so fences only keep the compiler's order.
-// About 105 vector instructions a chunk (64 cells) and 80 a row; bound by their issue, one wavefront's chain when
-// calls are few.  Measured against the first form, whole calls: 12 DPs of 600 bases 150 -> 95 us, 400 of 12 kbp
-// 1.32 -> 0.97 ms, 600 extensions of 8 kbp 4.7 -> 2.7 ms, a search with one candidate pair per wavefront (951
-// thousand extensions of 4 %-error reads) 101 -> 51 ms.
+// wave_rows is not inlined: the kernels' other live values would otherwise be spilled around its loops.
+// Bound by the issue of a wavefront's instructions, one wavefront's chain when calls are few.  Measured as whole
+// calls, first form -> wide rows only -> both: 12 DPs of 600 bases 150 -> 95 -> 75 us, 400 of 12 kbp 1.43 -> 0.97
+// -> 0.90 ms, 600 extensions of 8 kbp 4.7 -> 2.7 -> 1.9 ms, a search with one candidate pair per wavefront (951
+// thousand extensions of 4 %-error reads) 101 -> 51 -> 37 ms.
 #pragma once
 
 #include "oic_dp.h"
@@ -78,6 +84,11 @@ struct DPOut {
 };
 
 struct __attribute__((packed, aligned(4))) Words4 { uint32_t x, y, z, w; };
+
+// pointers of a function that is not inlined carry their address space (a plain one compiles to flat accesses)
+typedef const __attribute__((address_space(1))) uint32_t *g_words;
+typedef __attribute__((address_space(1))) int32_t *g_ints;
+typedef __attribute__((address_space(3))) int32_t *l_ints;
 
 __device__ __forceinline__ int32_t uni(int32_t v) { return __builtin_amdgcn_readfirstlane(v); }
 __device__ __forceinline__ int64_t uni64(int64_t v) {
@@ -144,8 +155,13 @@ __device__ __forceinline__ uint32_t lowest_bit(uint32_t x) {
 }
 
 // the four words holding position p (p >= 0) of a tail: a 32-bit byte offset from the uniform base
-__device__ __forceinline__ Words4 words_at(const uint32_t *__restrict__ w, int32_t p) {
-  return *(const Words4 *)((const uint8_t *)w + (uint32_t)(((uint32_t)p >> 2) & ~3u));
+__device__ __forceinline__ Words4 words_at(g_words w, int32_t p) {
+  typedef const __attribute__((address_space(1))) uint8_t *g_bytes;
+  typedef const __attribute__((address_space(1))) Words4 *g_words4;
+  const g_words4 x = (g_words4)((g_bytes)w + (uint32_t)(((uint32_t)p >> 2) & ~3u));
+  Words4 r;
+  r.x = x->x; r.y = x->y; r.z = x->z; r.w = x->w;
+  return r;
 }
 
 // both bits of every N base among 16 from position p of the N mask
@@ -156,12 +172,26 @@ __device__ __forceinline__ uint32_t nspread16(const uint32_t *__restrict__ nm, i
 
 // The two tails of a DP, uniform: words from the one holding base 0, and base 0's place in it
 struct WTails {
-  const uint32_t *wa, *wt;
+  g_words wa, wt;
   const uint32_t *nm;        // N mask with absolute base indexing (read only for the tails that hold N)
   int64_t a0, t0;
   int32_t ra, rt;
   bool na, nt;
 };
+
+__device__ __forceinline__ WTails make_tails(const uint32_t *words, const uint32_t *nm, int64_t a0, int64_t t0, bool na, bool nt) {
+  WTails W;
+  W.a0 = a0;
+  W.t0 = t0;
+  W.wa = (g_words)words + (a0 >> 4);
+  W.wt = (g_words)words + (t0 >> 4);
+  W.nm = nm;
+  W.ra = (int32_t)(a0 & 15);
+  W.rt = (int32_t)(t0 & 15);
+  W.na = na;
+  W.nt = nt;
+  return W;
+}
 
 // equal bases from positions p of A and q of T on, at most rem, all arguments uniform: 1024 a step
 template <bool HASN>
@@ -171,7 +201,7 @@ __device__ __forceinline__ int32_t wave_run(const WTails &W, int32_t p, int32_t 
     const int32_t off = base + 16 * lane, r = rem - off;
     const int32_t o = r > 0 ? off : 0;          // lanes past the end read the first window again
     const int32_t ia = W.ra + p + o, it = W.rt + q + o;
-    const uint32_t *a = W.wa + (uint32_t)(ia >> 4), *b = W.wt + (uint32_t)(it >> 4);
+    const g_words a = W.wa + (uint32_t)(ia >> 4), b = W.wt + (uint32_t)(it >> 4);
     uint32_t x = __builtin_amdgcn_alignbit(a[1], a[0], (uint32_t)ia * 2u) ^ __builtin_amdgcn_alignbit(b[1], b[0], (uint32_t)it * 2u);
     if (HASN && W.na) x &= ~nspread16(W.nm, W.a0 + p + o);
     if (HASN && W.nt) x &= ~nspread16(W.nm, W.t0 + q + o);
@@ -253,6 +283,13 @@ __device__ __forceinline__ int32_t wave_traceback(const DPScratch &sc, int32_t e
   return nev;
 }
 
+// wave_rows' flags
+#define WR_NA      1u    // A's read holds N
+#define WR_NT      2u    // T's
+#define WR_FORWARD 4u
+#define WR_STORE   8u    // rows are stored
+#define WR_PARTIAL 16u
+
 // a DP's rows: where it ended and what the traceback starts from
 struct WRows {
   int32_t e, d, last;        // traceback start: row, diagonal, the cell's value (< 0: the stored one)
@@ -263,33 +300,109 @@ struct WRows {
   bool mte, overflow;
 };
 
-// Rows 1 .. limit of a DP whose row 0 reached row0.  All values but the cells are uniform.
-template <int RING, bool ROWS, bool HASN>
-__device__ __forceinline__ WRows wave_rows(const WTails &W, const int32_t m, const int32_t n, const int32_t limit, const int32_t row0,
-                                           const bool is_forward, const bool store, const DPTables &tb, WaveBand<RING> &band,
-                                           const DPScratch &sc) {
+// Equal bases of a chunk's lanes from their positions p of A and q = p + d of T on, at most rem each (0 for lanes
+// without a cell): lane l's diagonal is d0 + l, wa and wt hold its words there.
+template <bool HASN>
+__device__ __forceinline__ int32_t chunk_slide(const WTails &W, const Words4 &wa, const Words4 &wt, int32_t p, int32_t q, int32_t rem,
+                                               int32_t d0) {
   const int lane = lane_id();
+  const uint32_t sa = (uint32_t)(W.ra + p) * 2u, st = (uint32_t)(W.rt + q) * 2u;   // alignbit takes them modulo 32
+  uint32_t y0 = __builtin_amdgcn_alignbit(wa.y, wa.x, sa) ^ __builtin_amdgcn_alignbit(wt.y, wt.x, st);
+  uint32_t y1 = __builtin_amdgcn_alignbit(wa.z, wa.y, sa) ^ __builtin_amdgcn_alignbit(wt.z, wt.y, st);
+  uint32_t y2 = __builtin_amdgcn_alignbit(wa.w, wa.z, sa) ^ __builtin_amdgcn_alignbit(wt.w, wt.z, st);
+  if (HASN && W.na) {
+    y0 &= ~nspread16(W.nm, W.a0 + p);
+    y1 &= ~nspread16(W.nm, W.a0 + p + 16);
+    y2 &= ~nspread16(W.nm, W.a0 + p + 32);
+  }
+  if (HASN && W.nt) {
+    y0 &= ~nspread16(W.nm, W.t0 + q);
+    y1 &= ~nspread16(W.nm, W.t0 + q + 16);
+    y2 &= ~nspread16(W.nm, W.t0 + q + 32);
+  }
+  // the first differing base: lowest set bit (two bits a base); all-ones where a word has none
+  const uint32_t f0 = lowest_bit(y0), f1 = lowest_bit(y1) | 32u, f2 = lowest_bit(y2) | 64u;
+  uint32_t f = f0 < f1 ? f0 : f1;
+  f = f < f2 ? f : f2;
+  f >>= 1;                                    // 48 and more: no difference among the 48 bases
+  int32_t adv = (int32_t)(f < (uint32_t)rem ? f : (uint32_t)rem);
+  uint64_t more = lanes(adv >= 48);
+  if (more) {
+    more = lanes(f >= 48u && rem > 48);
+    adv = adv < 48 ? adv : 48;
+    if (__builtin_popcountll(more) <= 4) {
+      while (more) {
+        const int l = __builtin_ctzll(more);
+        more &= more - 1;
+        const int32_t P = __builtin_amdgcn_readlane(p, l);
+        const int32_t k = wave_run<HASN>(W, P + 48, P + d0 + l + 48, __builtin_amdgcn_readlane(rem, l) - 48);
+        adv = lane == l ? 48 + k : adv;
+      }
+    } else if (f >= 48u && rem > 48) {
+      SeqV a, t;
+      a.w = t.w = (const uint32_t *)(W.wa - (W.a0 >> 4));   // all packed reads
+      a.nm = HASN && W.na ? W.nm : nullptr; a.b0 = W.a0;
+      t.nm = HASN && W.nt ? W.nm : nullptr; t.b0 = W.t0;
+      while (adv < rem) {
+        const int32_t k = match64(a, p + adv, t, q + adv);
+        adv += k;
+        if (k < 64) break;
+      }
+      adv = adv < rem ? adv : rem;
+    }
+  }
+  return adv;
+}
+
+// whether this lane's bit is set
+__device__ __forceinline__ bool lane_in(uint64_t mask) { return __builtin_amdgcn_inverse_ballot_w64(mask); }
+
+// Rows 1 .. limit of a DP whose row 0 reached row0.  All values but the cells are uniform.
+//
+// A row runs in one of two forms.  Narrow: the band lies within 64 diagonals, lane l holding diagonal base + l in a
+// register, and the row's masks (band, kept range) are single 64-bit scalars; about 75 vector and 50 scalar
+// instructions a row.  When the band reaches either end it is moved to the middle by one permute, or, past 52
+// diagonals, to LDS.  Wide: chunks of 64 in the LDS ring, WR_GROUP chunks' loads in flight; back to narrow below 40
+// diagonals.
+// Not inlined: its loops then have the registers to themselves (inlined, a kernel's own values and the N form's
+// took 150 and more, or spilled into the rows).
+template <int RING, bool ROWS, bool HASN>
+__device__ __attribute__((noinline)) WRows wave_rows(const uint32_t *words_, const uint32_t *nmask_, int64_t a0_, int64_t t0_, uint32_t flags_,
+                                                     int32_t m_, int32_t n_, int32_t limit_, int32_t row0_, const int32_t *match_limit_,
+                                                     double bmv, double slope_min, uint32_t end_dist_, int32_t *rowm_, int32_t *rowVal_,
+                                                     int32_t val_cap_, int32_t max_rows_, int32_t *band_) {
+  constexpr int32_t MASK = RING - 1;
+  const int lane = lane_id();
+  const uint32_t flags = (uint32_t)uni((int32_t)flags_), end_dist = (uint32_t)uni((int32_t)end_dist_);
+  const bool is_forward = flags & WR_FORWARD, store = ROWS && (flags & WR_STORE), partial = flags & WR_PARTIAL;
+  const WTails W = make_tails((const uint32_t *)uni64((int64_t)words_), (const uint32_t *)uni64((int64_t)nmask_), uni64(a0_), uni64(t0_),
+                              flags & WR_NA, flags & WR_NT);
+  const int32_t m = uni(m_), n = uni(n_), limit = uni(limit_), val_cap = uni(val_cap_), max_rows = uni(max_rows_);
+  const g_ints match_limit = (g_ints)(int32_t *)uni64((int64_t)match_limit_);
+  const g_ints rowm = (g_ints)(int32_t *)uni64((int64_t)rowm_), rowVal = (g_ints)(int32_t *)uni64((int64_t)rowVal_);
+  const l_ints band0 = (l_ints)band_;
   WRows o = {};
   int32_t Left = 0, Right = 0, Longest = 0, MSL = 0, MSd = 0, MSe = 0;
   double MaxScore = 0.0;
   int32_t vend = 1;                            // cells stored
-  int64_t kept = 1;                            // those of them that were kept
+  int32_t kept = 1;                            // those of them that were kept
   int32_t mlv = 0;                             // Edit_Match_Limit of 64 rows, one a lane
-  int cur = 0;
-  // row 0 and the sentinels around it (ring cells 30 .. 34)
-  if (lane < 5) band.b[0][1 + 30 + lane] = lane == 2 ? row0 : -2;
-  if (ROWS && store && lane == 0) {
-    sc.rowm[0] = 0;
-    sc.rowVal[0] = row0 << 2;
+  int cur = 0;                                 // wide: the buffer of the previous row
+  bool narrow = true;
+  int32_t base = -32, v = uni(row0_);          // narrow: the previous row, -2 outside its kept range
+  uint64_t km = 1ull << 32;                    // narrow: the kept range's lanes
+  if (store && lane == 0) {
+    rowm[0] = 0;
+    rowVal[0] = v << 2;
   }
-  wave_order();
+  v = lane == 32 ? v : -2;
   // Longest / Max_Score after row er, from each lane's first maximum of that row (forward.C:284-306).  With
   // Longest unchanged the score only falls, and MaxScore already holds the earlier row's.
   auto longest = [&](int32_t pv, int32_t pd, int32_t er) {
     const int32_t M = wave_max_dpp(pv);
     if (M > Longest) {
       Longest = M;
-      const double Score = (double)M * tb.bmv - (double)er;
+      const double Score = (double)M * bmv - (double)er;
       if (Score > MaxScore) {
         uint64_t b = lanes(pv == M);
         int32_t bd = __builtin_amdgcn_readlane(pd, __builtin_ctzll(b));
@@ -301,48 +414,125 @@ __device__ __forceinline__ WRows wave_rows(const WTails &W, const int32_t m, con
       }
     }
   };
+  // The end of A or T was reached in row e on diagonal rd: branch-point test (forward.C:172-212);
+  // -ffp-contract=off keeps the score two roundings.  after: the previous row's cell at rd + 1.
+  auto reached = [&](int32_t e, int32_t rd, int32_t rrow, int32_t after) {
+    o.cells += (uint32_t)(rd - Left + 1);
+    const double Score = (double)rrow * bmv - (double)e;
+    const int32_t Tail_Len = rrow - MSL;
+    const double slope = (double)(MaxScore - Score) / (double)Tail_Len;
+    bool abort_ = false;
+    if (partial && (Score < MaxScore)) abort_ = true;
+    if (((uint32_t)e > end_dist / 2u) && ((uint32_t)Tail_Len >= end_dist) && (slope >= slope_min))
+      abort_ = true;
+    o.mte = !abort_;
+    o.e = e;
+    o.d = (is_forward && rrow == m && 1 + after == rrow && rd < Right) ? rd + 1 : rd;
+    o.last = rrow; o.rrow = rrow;
+    if (abort_) { o.e = MSe; o.d = MSd; o.rrow = MSL; o.last = -1; }
+  };
   for (int32_t e = 1; e <= limit; e++) {
     if ((e & 63) == 0 || e == 1) {
       const int32_t i = (e & ~63) + lane;
-      mlv = tb.match_limit[i < limit ? i : limit];
+      mlv = match_limit[i < limit ? i : limit];
     }
     Left--;
     Right++;
     const int32_t width = Right - Left;
-    if (width + 1 > wr_band<RING>() || (ROWS && store && e >= sc.max_rows)) {
+    if (width + 1 > wr_band<RING>() || (store && e >= max_rows)) {
       o.overflow = true;
       return o;
     }
     const int32_t eml = __builtin_amdgcn_readlane(mlv, e & 63);
+    o.rows++;
+    if (store && lane == 0) rowm[e] = vend - Left;
+    o.end = vend + width + 1;
+    if (narrow) {
+      const uint64_t act = km | km << 1 | km >> 1;
+      const int32_t d = base + lane;
+      const int32_t x1 = v + 1, x2 = __builtin_amdgcn_update_dpp(-2, v, 0x138, 0xF, 0xF, false);      // wave_shr:1
+      const int32_t x3 = __builtin_amdgcn_update_dpp(-2, v, 0x130, 0xF, 0xF, false) + 1;              // wave_shl:1
+      const int32_t x12 = x1 > x2 ? x1 : x2;
+      const bool on = lane_in(act);
+      const int32_t Row = on ? (x12 > x3 ? x12 : x3) : 0, q = on ? Row + d : 0;
+      const Words4 wa = words_at(W.wa, W.ra + Row), wt = words_at(W.wt, W.rt + q);
+      const int32_t r1 = m - Row, r2 = n - q;
+      const int32_t rem = on ? (r1 < r2 ? r1 : r2) : 0;
+      const int32_t adv = chunk_slide<HASN>(W, wa, wt, Row, q, rem, base);
+      o.lb += (uint32_t)adv;
+      o.slots += OIC_WAVE;
+      const int32_t r = Row + adv;
+      if (store && on) {
+        // the traceback's choice (forward.C:44-56): from d unless d - 1 is larger, then d + 1 if larger still
+        const int32_t code = x3 > x12 ? 2 : (x2 > x1 ? 1 : 0);
+        rowVal[(uint32_t)(vend + (d - Left))] = (r << 2) | code;
+      }
+      const uint64_t rb = lanes(adv == rem) & act;
+      if (rb) {
+        const int l = __builtin_ctzll(rb);
+        reached(e, base + l, __builtin_amdgcn_readlane(r, l), l < 63 ? __builtin_amdgcn_readlane(v, l + 1) : -2);
+        return o;
+      }
+      o.cells += (uint32_t)(width + 1);
+      const uint64_t kb = lanes(r + (d > 0 ? d : 0) >= eml) & act;     // not pruned (forward.C:244-282)
+      if (!kb) break;
+      const int32_t lo = __builtin_ctzll(kb), hi = 63 - __builtin_clzll(kb);
+      km = (~0ull << lo) & (~0ull >> (63 - hi));
+      v = lane_in(km) ? r : -2;
+      Left = base + lo;
+      Right = base + hi;
+      longest(v, d, e);
+      if (store) {
+        kept += hi - lo + 1;
+        if (kept > val_cap) { o.overflow = true; return o; }
+        vend += width + 1;
+      }
+      if (lo == 0 || hi == 63) {
+        if (hi - lo < 52) {
+          const int32_t by = ((lo + hi) >> 1) - 32, i = lane + by;
+          const int32_t x = __builtin_amdgcn_ds_bpermute(i << 2, v);
+          v = (uint32_t)i < 64u ? x : -2;
+          base += by;
+          km = by < 0 ? km << -by : km >> by;
+        } else {
+          const l_ints nb = band0 + cur * (RING + 2);
+          const int32_t i = (d + 32) & MASK;
+          nb[1 + i] = v;
+          if (lane < 4) nb[1 + ((lane + (lane < 2 ? Left - 2 : Right - 1) + 32) & MASK)] = -2;
+          wave_order();
+          if (lane < 2) nb[lane ? RING + 1 : 0] = nb[lane ? 1 : RING];
+          wave_order();
+          narrow = false;
+        }
+      }
+      continue;
+    }
     const int32_t Lc = (Left + 32) >> 6, Hc = (Right + 32) >> 6;
-    const int32_t *pb = band.b[cur];
-    int32_t *nb = band.b[cur ^ 1];
-    int32_t nL = 0x7fffffff, nR = 0, rd = 0x7fffffff, rrow = 0;
+    const l_ints pb = band0 + cur * (RING + 2);
+    const l_ints nb = band0 + (cur ^ 1) * (RING + 2);
+    int32_t nL = 0x7fffffff, nR = 0;
+    uint64_t any = 0;
     int32_t pv = -2, pd = 0;                   // this lane's first maximum of the previous row
     for (int32_t g = Lc; g <= Hc; g += WR_GROUP) {
       Words4 wa[WR_GROUP], wt[WR_GROUP];
-      int32_t rw[WR_GROUP];
-      uint32_t cd[WR_GROUP];
+      int32_t rw[WR_GROUP], cd[WR_GROUP];
       // recurrence and loads
 #pragma unroll
       for (int i = 0; i < WR_GROUP; i++) {
         const int32_t c = g + i;
         if (c <= Hc) {
           const int32_t d = 64 * c - 32 + lane;
-          const int32_t *p3 = pb + 64 * (c & (RING / 64 - 1)) + lane;
+          const l_ints p3 = pb + 64 * (c & (RING / 64 - 1)) + lane;
           const int32_t x2 = p3[0], pc = p3[1], x1 = pc + 1, x3 = p3[2] + 1;
-          const bool act = (uint32_t)(d - Left) <= (uint32_t)width;
-          const int32_t pm = act ? pc : -2;    // only the band's own cells and the sentinels around it count
+          const bool on = (uint32_t)(d - Left) <= (uint32_t)width;
+          const int32_t pm = on ? pc : -2;     // only the band's own cells and the sentinels around it count
           pd = pm > pv ? d : pd;
           pv = pm > pv ? pm : pv;
           const int32_t x12 = x1 > x2 ? x1 : x2;
-          int32_t Row = x12 > x3 ? x12 : x3;
-          // the traceback's choice (forward.C:44-56): from d unless d - 1 is larger, then d + 1 if larger still
-          if (ROWS) cd[i] = x3 > x12 ? 2u : (x2 > x1 ? 1u : 0u);
-          Row = act ? Row : 0;
-          const int32_t pa = W.ra + Row, pt = W.rt + (act ? Row + d : 0);
-          wa[i] = words_at(W.wa, pa);
-          wt[i] = words_at(W.wt, pt);
+          if (ROWS) cd[i] = x3 > x12 ? 2 : (x2 > x1 ? 1 : 0);
+          const int32_t Row = on ? (x12 > x3 ? x12 : x3) : 0;
+          wa[i] = words_at(W.wa, W.ra + Row);
+          wt[i] = words_at(W.wt, W.rt + (on ? Row + d : 0));
           rw[i] = Row;
         }
       }
@@ -351,138 +541,81 @@ __device__ __forceinline__ WRows wave_rows(const WTails &W, const int32_t m, con
       for (int i = 0; i < WR_GROUP; i++) {
         const int32_t c = g + i;
         if (c <= Hc) {
-          const int32_t d0 = 64 * c - 32, d = d0 + lane;
-          const bool act = (uint32_t)(d - Left) <= (uint32_t)width;
-          const int32_t p = rw[i], q = act ? p + d : 0;
-          const uint32_t sa = (uint32_t)(W.ra + p) * 2u, st = (uint32_t)(W.rt + q) * 2u;   // alignbit takes them modulo 32
-          uint32_t y0 = __builtin_amdgcn_alignbit(wa[i].y, wa[i].x, sa) ^ __builtin_amdgcn_alignbit(wt[i].y, wt[i].x, st);
-          uint32_t y1 = __builtin_amdgcn_alignbit(wa[i].z, wa[i].y, sa) ^ __builtin_amdgcn_alignbit(wt[i].z, wt[i].y, st);
-          uint32_t y2 = __builtin_amdgcn_alignbit(wa[i].w, wa[i].z, sa) ^ __builtin_amdgcn_alignbit(wt[i].w, wt[i].z, st);
-          if (HASN && W.na) {
-            y0 &= ~nspread16(W.nm, W.a0 + p);
-            y1 &= ~nspread16(W.nm, W.a0 + p + 16);
-            y2 &= ~nspread16(W.nm, W.a0 + p + 32);
-          }
-          if (HASN && W.nt) {
-            y0 &= ~nspread16(W.nm, W.t0 + q);
-            y1 &= ~nspread16(W.nm, W.t0 + q + 16);
-            y2 &= ~nspread16(W.nm, W.t0 + q + 32);
-          }
-          // the first differing base: lowest set bit (two bits a base); all-ones where a word has none
-          const uint32_t f0 = lowest_bit(y0), f1 = lowest_bit(y1) | 32u, f2 = lowest_bit(y2) | 64u;
-          uint32_t f = f0 < f1 ? f0 : f1;
-          f = f < f2 ? f : f2;
-          const int32_t kk = (int32_t)(f >> 1);       // 48 and more: no difference among the 48 bases
-          const int32_t r1 = m - p, r2 = n - q;
-          const int32_t rem = act ? (r1 < r2 ? r1 : r2) : 0;
-          int32_t adv = kk < 48 ? kk : 48;
-          adv = adv < rem ? adv : rem;
-          const bool on = kk >= 48 && rem > 48;
-          uint64_t more = lanes(on);
-          if (more) {
-            if (__builtin_popcountll(more) <= 4) {
-              while (more) {
-                const int l = __builtin_ctzll(more);
-                more &= more - 1;
-                const int32_t P = __builtin_amdgcn_readlane(p, l);
-                const int32_t k = wave_run<HASN>(W, P + 48, P + d0 + l + 48, __builtin_amdgcn_readlane(rem, l) - 48);
-                adv = lane == l ? 48 + k : adv;
-              }
-            } else if (on) {
-              SeqV a, t;
-              a.w = W.wa; a.nm = nullptr; a.b0 = W.ra;
-              t.w = W.wt; t.nm = nullptr; t.b0 = W.rt;
-              if (HASN) {
-                // absolute base indexing for the N mask
-                a.w = W.wa - (W.a0 >> 4); a.nm = W.na ? W.nm : nullptr; a.b0 = W.a0;
-                t.w = W.wt - (W.t0 >> 4); t.nm = W.nt ? W.nm : nullptr; t.b0 = W.t0;
-              }
-              while (adv < rem) {
-                const int32_t k = match64(a, p + adv, t, q + adv);
-                adv += k;
-                if (k < 64) break;
-              }
-              adv = adv < rem ? adv : rem;
-            }
-          }
+          const int32_t d0 = 64 * c - 32, d = d0 + lane, p = rw[i];
+          const bool on = (uint32_t)(d - Left) <= (uint32_t)width;
+          const int32_t q = on ? p + d : 0, r1 = m - p, r2 = n - q;
+          const int32_t rem = on ? (r1 < r2 ? r1 : r2) : 0;
+          const int32_t adv = chunk_slide<HASN>(W, wa[i], wt[i], p, q, rem, d0);
           o.lb += (uint32_t)adv;
           const int32_t r = p + adv;
-          if (act) {
-            const int32_t sl = c & (RING / 64 - 1);
-            nb[64 * sl + lane + 1] = r;
-            if (sl == 0 && lane == 0) nb[RING + 1] = r;
-            if (sl == RING / 64 - 1 && lane == 63) nb[0] = r;
-            if (ROWS && store) sc.rowVal[vend + (d - Left)] = (r << 2) | (int32_t)cd[i];
+          if (on) {
+            nb[64 * (c & (RING / 64 - 1)) + lane + 1] = r;
+            if (store) rowVal[(uint32_t)(vend + (d - Left))] = (r << 2) | cd[i];
           }
-          const uint64_t rb = lanes(act && adv == rem);
-          if (rb && rd == 0x7fffffff) {
-            const int l = __builtin_ctzll(rb);
-            rd = d0 + l;
-            rrow = __builtin_amdgcn_readlane(r, l);
-          }
-          const uint64_t kb = lanes(act && r + (d > 0 ? d : 0) >= eml);   // not pruned (forward.C:244-282)
+          any |= lanes(on && adv == rem);
+          const uint64_t kb = lanes(on && r + (d > 0 ? d : 0) >= eml);   // not pruned (forward.C:244-282)
           if (kb) {
-            if (nL == 0x7fffffff) nL = d0 + __builtin_ctzll(kb);
+            const int32_t first = d0 + __builtin_ctzll(kb);
+            nL = first < nL ? first : nL;
             nR = d0 + 63 - __builtin_clzll(kb);
           }
         }
       }
     }
     wave_order();
-    o.rows++;
     o.slots += (uint32_t)(Hc - Lc + 1) * OIC_WAVE;
-    if (ROWS && store && lane == 0) sc.rowm[e] = vend - Left;
-    if (e >= 2) longest(pv, pd, e - 1);
-    if (rd != 0x7fffffff) {
-      // the end of A or T was reached: branch-point test (forward.C:172-212); -ffp-contract=off keeps the
-      // score two roundings
-      o.cells += (uint32_t)(rd - Left + 1);
-      const double Score = (double)rrow * tb.bmv - (double)e;
-      const int32_t Tail_Len = rrow - MSL;
-      const double slope = (double)(MaxScore - Score) / (double)Tail_Len;
-      bool abort_ = false;
-      if (tb.partial && (Score < MaxScore)) abort_ = true;
-      if (((uint32_t)e > tb.min_branch_end_dist / 2u) && ((uint32_t)Tail_Len >= tb.min_branch_end_dist) && (slope >= tb.slope_min))
-        abort_ = true;
-      o.end = vend + width + 1;
-      if (!abort_) {
-        int32_t d = rd;
-        if (is_forward && rrow == m && d < Right && 1 + uni(pb[1 + ((rd + 1 + 32) & (RING - 1))]) == rrow) d++;
-        o.mte = true;
-        o.e = e; o.d = d; o.last = rrow; o.rrow = rrow;
-        return o;
+    longest(pv, pd, e - 1);
+    if (any) {
+      // the lowest diagonal that reached an end
+      int32_t rd = 0x7fffffff, rrow = 0;
+      for (int32_t c = Lc; rd == 0x7fffffff; c++) {
+        const int32_t d = 64 * c - 32 + lane, r = nb[64 * (c & (RING / 64 - 1)) + lane + 1];
+        const uint64_t b = lanes((uint32_t)(d - Left) <= (uint32_t)width && (r == m || r + d == n));
+        if (b) {
+          const int l = __builtin_ctzll(b);
+          rd = 64 * c - 32 + l;
+          rrow = __builtin_amdgcn_readlane(r, l);
+        }
       }
-      o.e = MSe; o.d = MSd; o.rrow = MSL; o.last = -1;
+      reached(e, rd, rrow, uni(pb[1 + ((rd + 1 + 32) & MASK)]));
       return o;
     }
     o.cells += (uint32_t)(width + 1);
-    o.end = vend + width + 1;
     if (nL == 0x7fffffff) break;
-    if (ROWS && store) {
+    if (store) {
       kept += nR - nL + 1;
-      if (kept > sc.val_cap) { o.overflow = true; return o; }
+      if (kept > val_cap) { o.overflow = true; return o; }
       vend += width + 1;
     }
-    // the sentinels of the next row: its band's new ends and the cells past them
-    if (lane < 4) {
-      const int32_t i = (lane + (lane < 2 ? nL - 2 : nR - 1) + 32) & (RING - 1);
-      nb[1 + i] = -2;
-      if (i == 0) nb[RING + 1] = -2;
-      if (i == RING - 1) nb[0] = -2;
-    }
-    wave_order();
     Left = nL;
     Right = nR;
     cur ^= 1;
-    if (e == limit) {
-      // the last row's own maximum
+    if (nR - nL < 40 || e == limit) {
+      // narrow again, or the last row: its own maximum now
       int32_t bv = -2, bd = 0;
-      for (int32_t d = nL + lane; d <= nR; d += OIC_WAVE) {
-        const int32_t x = nb[1 + ((d + 32) & (RING - 1))];
-        bd = x > bv ? d : bd;
-        bv = x > bv ? x : bv;
+      base = ((nL + nR) >> 1) - 32;
+      if (nR - nL < 40) {
+        const int32_t d = base + lane;
+        bv = (uint32_t)(d - nL) <= (uint32_t)(nR - nL) ? nb[1 + ((d + 32) & MASK)] : -2;
+        bd = d;
+        v = bv;
+        km = (~0ull << (nL - base)) & (~0ull >> (63 - (nR - base)));
+        narrow = true;
+      } else {
+        for (int32_t d = nL + lane; d <= nR; d += OIC_WAVE) {
+          const int32_t x = nb[1 + ((d + 32) & MASK)];
+          bd = x > bv ? d : bd;
+          bv = x > bv ? x : bv;
+        }
       }
       longest(bv, bd, e);
+    }
+    if (!narrow) {
+      // the sentinels of the next row (its band's new ends and the cells past them), and the copies around the ring
+      if (lane < 4) nb[1 + ((lane + (lane < 2 ? nL - 2 : nR - 1) + 32) & MASK)] = -2;
+      wave_order();
+      if (lane < 2) nb[lane ? RING + 1 : 0] = nb[lane ? 1 : RING];
+      wave_order();
     }
   }
   // branch point, error limit exhausted or band emptied (forward.C:306-313)
@@ -505,17 +638,10 @@ __device__ __forceinline__ DPOut wave_prefix_dp(const SeqV &A, const int32_t m_,
   const int lane = lane_id();
   const int32_t m = uni(m_), n = uni(n_), limit = uni(limit_);
   const bool store = ROWS && uni((int32_t)want_delta_) != 0;
-  WTails W;
-  W.a0 = uni64(A.b0);
-  W.t0 = uni64(T.b0);
-  W.wa = A.w + (W.a0 >> 4);
-  W.wt = T.w + (W.t0 >> 4);
-  W.ra = (int32_t)(W.a0 & 15);
-  W.rt = (int32_t)(W.t0 & 15);
-  W.na = uni(A.nm != nullptr) != 0;
-  W.nt = uni(T.nm != nullptr) != 0;
-  W.nm = W.na ? A.nm : T.nm;
-  const bool has_n = W.na || W.nt;
+  // every view's words are the packed reads
+  const bool na = uni(A.nm != nullptr) != 0, nt = uni(T.nm != nullptr) != 0;
+  const WTails W = make_tails(A.w, na ? A.nm : T.nm, uni64(A.b0), uni64(T.b0), na, nt);
+  const bool has_n = na || nt;
   DPOut out;
   out.overflow = 0;
   out.ndelta = 0;
@@ -532,8 +658,12 @@ __device__ __forceinline__ DPOut wave_prefix_dp(const SeqV &A, const int32_t m_,
     out.leftover = m;
     return out;
   }
-  const WRows r = has_n ? wave_rows<RING, ROWS, true>(W, m, n, limit, row0, is_forward, store, tb, band, sc)
-                        : wave_rows<RING, ROWS, false>(W, m, n, limit, row0, is_forward, store, tb, band, sc);
+  const uint32_t flags = (na ? WR_NA : 0u) | (nt ? WR_NT : 0u) | (is_forward ? WR_FORWARD : 0u) | (store ? WR_STORE : 0u) |
+                         (tb.partial ? WR_PARTIAL : 0u);
+  const WRows r = has_n ? wave_rows<RING, ROWS, true>(A.w, W.nm, W.a0, W.t0, flags, m, n, limit, row0, tb.match_limit, tb.bmv, tb.slope_min,
+                                                      tb.min_branch_end_dist, sc.rowm, sc.rowVal, (int32_t)sc.val_cap, sc.max_rows, band.b[0])
+                        : wave_rows<RING, ROWS, false>(A.w, W.nm, W.a0, W.t0, flags, m, n, limit, row0, tb.match_limit, tb.bmv, tb.slope_min,
+                                                       tb.min_branch_end_dist, sc.rowm, sc.rowVal, (int32_t)sc.val_cap, sc.max_rows, band.b[0]);
   cells += r.cells;
   slots += r.slots;
   rows += r.rows;
