@@ -2282,26 +2282,27 @@ extern "C" int oic_model_predict(oic_ctx *c, const float *feat, uint64_t n, floa
   return OIC_OK;
 }
 
-static uint32_t grad_waves(oic_ctx *c, uint64_t n) {
-  return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((n + 63) / 64, (uint64_t)c->ncu * 2));
-}
+// workgroups of k_mlp_grad: one a chunk up to two for each CU, which its partial sums (20 KB each) are sized for
+static uint32_t grad_groups(uint64_t n) { return (uint32_t)std::min<uint64_t>((n + MLP_CHUNK - 1) / MLP_CHUNK, MLP_WG); }
+#define MLP_SUM_GRID dim3(MLP_NPARAM / 64 + 1)
 
 extern "C" int oic_model_grad(oic_ctx *c, const float *w, const float *z, const float *t, uint64_t n, float w_exit, float *loss,
                               float *grad) {
   if (!c || !w || !z || !t || !n || !grad) return OIC_EINVAL;
-  DevBuf dp, dz, dt, dg, dl;
+  DevBuf dp, dz, dt, dg, dl, part;
   ALLOC(c, dp, MLP_NPARAM * 4);
   ALLOC(c, dz, n * MLP_IN * 4);
   ALLOC(c, dt, n * MLP_OUT * 4);
   ALLOC(c, dg, MLP_NPARAM * 4);
   ALLOC(c, dl, 4);
+  ALLOC(c, part, (uint64_t)grad_groups(n) * MLP_PART * 4);
   HIPCHK(c, hipMemcpy(dp.p, w, MLP_NPARAM * 4, hipMemcpyHostToDevice));
   HIPCHK(c, hipMemcpy(dz.p, z, n * MLP_IN * 4, hipMemcpyHostToDevice));
   HIPCHK(c, hipMemcpy(dt.p, t, n * MLP_OUT * 4, hipMemcpyHostToDevice));
-  hipLaunchKernelGGL(k_fill_f, dim3((MLP_NPARAM + 255) / 256), dim3(256), 0, c->st, dg.as<float>(), (uint64_t)MLP_NPARAM, 0.f);
-  hipLaunchKernelGGL(k_fill_f, dim3(1), dim3(64), 0, c->st, dl.as<float>(), (uint64_t)1, 0.f);
-  hipLaunchKernelGGL(k_mlp_grad, dim3(grad_waves(c, n)), dim3(64), 0, c->st, dz.as<float>(), dt.as<float>(), (const uint32_t *)nullptr, n,
-                     dp.as<float>(), w_exit, 1.0f / (float)n, dg.as<float>(), dl.as<float>());
+  const uint32_t wg = grad_groups(n);
+  hipLaunchKernelGGL(k_mlp_grad, dim3(wg), dim3(256), 0, c->st, dz.as<float>(), dt.as<float>(), (const uint32_t *)nullptr, n,
+                     dp.as<float>(), w_exit, 1.0f / (float)n, part.as<float>());
+  hipLaunchKernelGGL(k_mlp_sum, MLP_SUM_GRID, dim3(256), 0, c->st, part.as<float>(), wg, dg.as<float>(), dl.as<float>());
   HIPCHK(c, hipGetLastError());
   HIPCHK(c, hipStreamSynchronize(c->st));
   HIPCHK(c, hipMemcpy(grad, dg.p, MLP_NPARAM * 4, hipMemcpyDeviceToHost));
@@ -2313,17 +2314,19 @@ extern "C" int oic_model_grad(oic_ctx *c, const float *w, const float *z, const 
 
 extern "C" int oic_model_train(oic_ctx *c, const float *feat, const float *targ, uint64_t n, const oic_train_params *tp, float *final_loss) {
   if (!c || !feat || !targ || n < 2 || !tp || tp->batch == 0 || tp->epochs == 0) return OIC_EINVAL;
-  // standardisation
+  // standardisation: the features' sums side by side, each in the samples' order
+  double s[MLP_IN] = {}, s2[MLP_IN] = {};
+  for (uint64_t r = 0; r < n; r++)
+    for (int i = 0; i < MLP_IN; i++) {
+      const double v = feat[r * MLP_IN + i];
+      s[i] += v;
+      s2[i] += v * v;
+    }
   for (int i = 0; i < MLP_IN; i++) {
-    double s = 0, s2 = 0;
-    for (uint64_t r = 0; r < n; r++) { const double v = feat[r * MLP_IN + i]; s += v; s2 += v * v; }
-    const double m = s / n, var = s2 / n - m * m;
+    const double m = s[i] / n, var = s2[i] / n - m * m;
     c->mmu[i] = (float)m;
     c->msd[i] = (float)(var > 1e-12 ? std::sqrt(var) : 1.0);
   }
-  std::vector<float> z(n * MLP_IN);
-  for (uint64_t r = 0; r < n; r++)
-    for (int i = 0; i < MLP_IN; i++) z[r * MLP_IN + i] = (feat[r * MLP_IN + i] - c->mmu[i]) / c->msd[i];
   // Glorot-uniform initial weights from a fixed seed, zero biases
   std::mt19937_64 rng(tp->seed);
   auto init = [&](int off, int fan_out, int fan_in) {
@@ -2337,43 +2340,46 @@ extern "C" int oic_model_train(oic_ctx *c, const float *feat, const float *targ,
   init(MLP_OFF_W3, MLP_OUT, MLP_H);
   int rc = upload_model(c);
   if (rc) return rc;
-  DevBuf dz, dt, dg, dm, dv, dl, didx;
+  DevBuf dz, dt, dm, dv, dl, didx, part;
+  const uint32_t most = grad_groups(std::min<uint64_t>(tp->batch, n));
   ALLOC(c, dz, n * MLP_IN * 4);
   ALLOC(c, dt, n * MLP_OUT * 4);
-  ALLOC(c, dg, MLP_NPARAM * 4);
   ALLOC(c, dm, MLP_NPARAM * 4);
   ALLOC(c, dv, MLP_NPARAM * 4);
   ALLOC(c, dl, 4);
   ALLOC(c, didx, n * 4);
-  HIPCHK(c, hipMemcpy(dz.p, z.data(), n * MLP_IN * 4, hipMemcpyHostToDevice));
+  ALLOC(c, part, (uint64_t)most * MLP_PART * 4);
+  HIPCHK(c, hipMemcpy(dz.p, feat, n * MLP_IN * 4, hipMemcpyHostToDevice));
   HIPCHK(c, hipMemcpy(dt.p, targ, n * MLP_OUT * 4, hipMemcpyHostToDevice));
-  hipLaunchKernelGGL(k_fill_f, dim3((MLP_NPARAM + 255) / 256), dim3(256), 0, c->st, dm.as<float>(), (uint64_t)MLP_NPARAM, 0.f);
-  hipLaunchKernelGGL(k_fill_f, dim3((MLP_NPARAM + 255) / 256), dim3(256), 0, c->st, dv.as<float>(), (uint64_t)MLP_NPARAM, 0.f);
-  std::vector<uint32_t> perm(n);
-  std::iota(perm.begin(), perm.end(), 0u);
+  hipLaunchKernelGGL(k_standardise, dim3((unsigned)std::min<uint64_t>((n * MLP_IN + 255) / 256, 8 * (uint64_t)c->ncu)), dim3(256), 0, c->st, dz.as<float>(), n,
+                     c->m_mu.as<float>(), c->m_sd.as<float>());
+  // Each epoch's order is drawn while the epoch before it runs; the copy's source stays as it is meanwhile.
+  std::vector<uint32_t> perm[2];
+  perm[0].resize(n);
+  std::iota(perm[0].begin(), perm[0].end(), 0u);
   int step = 0;
-  float last = 0;
   for (uint32_t ep = 0; ep < tp->epochs; ep++) {
-    std::shuffle(perm.begin(), perm.end(), rng);
-    HIPCHK(c, hipMemcpyAsync(didx.p, perm.data(), n * 4, hipMemcpyHostToDevice, c->st));
-    hipLaunchKernelGGL(k_fill_f, dim3(1), dim3(64), 0, c->st, dl.as<float>(), (uint64_t)1, 0.f);
+    std::vector<uint32_t> &order = perm[ep & 1];
+    if (ep) order = perm[(ep - 1) & 1];
+    std::shuffle(order.begin(), order.end(), rng);
+    if (ep) HIPCHK(c, hipStreamSynchronize(c->st));
+    HIPCHK(c, hipMemcpyAsync(didx.p, order.data(), n * 4, hipMemcpyHostToDevice, c->st));
     for (uint64_t b0 = 0; b0 < n; b0 += tp->batch) {
       const uint64_t nb = std::min<uint64_t>(tp->batch, n - b0);
-      hipLaunchKernelGGL(k_fill_f, dim3((MLP_NPARAM + 255) / 256), dim3(256), 0, c->st, dg.as<float>(), (uint64_t)MLP_NPARAM, 0.f);
-      hipLaunchKernelGGL(k_mlp_grad, dim3(grad_waves(c, nb)), dim3(64), 0, c->st, dz.as<float>(), dt.as<float>(),
-                         didx.as<uint32_t>() + b0, nb, c->m_param.as<float>(), tp->w_exit, 1.0f / (float)nb, dg.as<float>(),
-                         dl.as<float>());
+      const uint32_t wg = grad_groups(nb);
+      hipLaunchKernelGGL(k_mlp_grad, dim3(wg), dim3(256), 0, c->st, dz.as<float>(), dt.as<float>(), didx.as<uint32_t>() + b0, nb,
+                         c->m_param.as<float>(), tp->w_exit, 1.0f / (float)nb, part.as<float>());
       step++;
       const float c1 = 1.f - std::pow(tp->beta1, (float)step), c2 = 1.f - std::pow(tp->beta2, (float)step);
-      hipLaunchKernelGGL(k_adam, dim3((MLP_NPARAM + 255) / 256), dim3(256), 0, c->st, c->m_param.as<float>(), dg.as<float>(),
-                         dm.as<float>(), dv.as<float>(), MLP_NPARAM, tp->lr, tp->beta1, tp->beta2, tp->eps, c1, c2);
+      hipLaunchKernelGGL(k_mlp_adam, MLP_SUM_GRID, dim3(256), 0, c->st, part.as<float>(), wg, c->m_param.as<float>(), dm.as<float>(),
+                         dv.as<float>(), step == 1, tp->lr, tp->beta1, tp->beta2, tp->eps, c1, c2, dl.as<float>(), b0 != 0);
     }
     HIPCHK(c, hipGetLastError());
-    float l = 0;
-    HIPCHK(c, hipMemcpyAsync(&l, dl.p, 4, hipMemcpyDeviceToHost, c->st));
-    HIPCHK(c, hipStreamSynchronize(c->st));
-    last = l / (float)n;
   }
+  HIPCHK(c, hipStreamSynchronize(c->st));
+  float l = 0;
+  HIPCHK(c, hipMemcpy(&l, dl.p, 4, hipMemcpyDeviceToHost));
+  const float last = l / (float)n;
   HIPCHK(c, hipMemcpy(c->mparam, c->m_param.p, MLP_NPARAM * 4, hipMemcpyDeviceToHost));
   if (final_loss) *final_loss = last;
   return OIC_OK;
