@@ -478,9 +478,9 @@ static int sort_pass(oic_ctx *c, const uint64_t *ki, const uint64_t *vi, uint64_
   const uint64_t ncount = ((uint64_t)1 << BITS) * ntiles;
   uint32_t *counts = (uint32_t *)c->s_rp.p;
   uint64_t *offs = (uint64_t *)((uint8_t *)c->s_rp.p + ncount * 4);
-  hipLaunchKernelGGL(k_rs_hist<BITS>, dim3((unsigned)ntiles), dim3(RS_THREADS), 0, c->st, ki, n, shift, counts, (uint32_t)ntiles);
+  hipLaunchKernelGGL(k_rs_hist<BITS>, dim3(rs_grid((uint32_t)ntiles)), dim3(RS_THREADS), 0, c->st, ki, n, shift, counts, (uint32_t)ntiles);
   HIPCHK(c, scan_excl<uint32_t>(counts, offs, ncount, c->s_small.as<uint64_t>(), c->st, nullptr));
-  hipLaunchKernelGGL(k_rs_scatter<BITS>, dim3((unsigned)ntiles), dim3(RS_THREADS), 0, c->st, ki, vi, ko, vo, n, shift, offs,
+  hipLaunchKernelGGL(k_rs_scatter<BITS>, dim3(rs_grid((uint32_t)ntiles)), dim3(RS_THREADS), 0, c->st, ki, vi, ko, vo, n, shift, offs,
                      (uint32_t)ntiles);
   HIPCHK(c, hipGetLastError());
   return OIC_OK;
@@ -489,7 +489,7 @@ static int sort_pass(oic_ctx *c, const uint64_t *ki, const uint64_t *vi, uint64_
 static int sort_pairs(oic_ctx *c, uint64_t **k, uint64_t **v, uint64_t n, int nbits) {
   if (n < 2 || nbits <= 0) return OIC_OK;
   const uint64_t ntiles = (n + RS_TILE - 1) / RS_TILE;
-  if (ntiles > 0xffffffffull) return fail(c, OIC_EINVAL, "sort of %lu keys has too many tiles", (unsigned long)n);
+  if (ntiles > 0xfffffff0ull) return fail(c, OIC_EINVAL, "sort of %lu keys has too many tiles", (unsigned long)n);
   const int passes = (nbits + 10) / 11;
   const int bits = std::max(8, (nbits + passes - 1) / passes);
   const uint64_t ncount = ((uint64_t)1 << bits) * ntiles;
