@@ -103,9 +103,9 @@ struct oic_ctx {
   // index of the current hash block
   bool have_index = false;
   uint32_t hbgn = 0, hend = 0, nblock = 0;
-  uint64_t nu = 0, nvalid = 0, npos = 0;
+  uint64_t nu = 0;
   int dshift = 0;
-  DevBuf x_ukey, x_ustart, x_dir, x_occ;
+  DevBuf x_ukey, x_ustart, x_dir, x_occ, x_loaded, x_posbase, x_first;
   // sort / scan temporaries
   DevBuf s_k1, s_v1, s_k2, s_v2, s_scan, s_flag, s_idx, s_small, s_rp;
   // search
@@ -438,7 +438,8 @@ extern "C" int oic_load_reads(oic_ctx *c, const oic_reads *rd) {
   ALLOC(c, c->d_b0r, ((size_t)n + 1) * 8);
   ALLOC(c, c->d_len, ((size_t)n + 1) * 4);
   ALLOC(c, c->d_hasN, (size_t)n + 1);
-  DevBuf raw, dstart;
+  // the bases and their starts wait in buffers of the index build, which follows
+  DevBuf &raw = c->s_k1, &dstart = c->x_posbase;
   ALLOC(c, raw, (hi - lo) + 1);
   ALLOC(c, dstart, ((size_t)n + 1) * 8);
   HIPCHK(c, hipMemsetAsync(c->d_words.p, 0, nwords * 4, c->st));
@@ -513,8 +514,10 @@ static int sort_pairs(oic_ctx *c, uint64_t **k, uint64_t **v, uint64_t n, int nb
   return OIC_OK;
 }
 
-// builds the k-mer table over hash reads [bgn, end]; fills first_t (distinct k-mers first seen per read)
-static int build_table(oic_ctx *c, uint32_t bgn, uint32_t end, std::vector<uint32_t> *first_t) {
+// builds the k-mer table over hash reads [bgn, end]; fills first_t (distinct k-mers first seen per read) if there
+// are at least `limit` distinct k-mers: with fewer no prefix of the reads reaches it (counting them, an atomic per
+// k-mer, took 5 ms of a 150 Mbp table's 25)
+static int build_table(oic_ctx *c, uint32_t bgn, uint32_t end, uint64_t limit, std::vector<uint32_t> *first_t) {
   const int K = (int)c->P.kmer;
   const uint32_t nb = end - bgn + 1;
   std::vector<uint8_t> loaded(nb);
@@ -527,14 +530,12 @@ static int build_table(oic_ctx *c, uint32_t bgn, uint32_t end, std::vector<uint3
     if (loaded[t]) N += (uint64_t)(L - K + 1);
   }
   posbase[nb] = N;
-  c->npos = N;
-  DevBuf d_loaded, d_posbase, d_first;
-  ALLOC(c, d_loaded, nb);
-  ALLOC(c, d_posbase, (nb + 1) * 8);
-  ALLOC(c, d_first, nb * 4);
-  HIPCHK(c, hipMemcpyAsync(d_loaded.p, loaded.data(), nb, hipMemcpyHostToDevice, c->st));
-  HIPCHK(c, hipMemcpyAsync(d_posbase.p, posbase.data(), (nb + 1) * 8, hipMemcpyHostToDevice, c->st));
-  HIPCHK(c, hipMemsetAsync(d_first.p, 0, nb * 4, c->st));
+  ALLOC(c, c->x_loaded, nb);
+  ALLOC(c, c->x_posbase, ((uint64_t)nb + 2) * 8);          // and the number of valid positions
+  uint64_t *d_nvalid = c->x_posbase.as<uint64_t>() + nb + 1;
+  HIPCHK(c, hipMemcpyAsync(c->x_loaded.p, loaded.data(), nb, hipMemcpyHostToDevice, c->st));
+  HIPCHK(c, hipMemcpyAsync(c->x_posbase.p, posbase.data(), ((uint64_t)nb + 1) * 8, hipMemcpyHostToDevice, c->st));
+  HIPCHK(c, hipMemsetAsync(d_nvalid, 0, 8, c->st));
   ALLOC(c, c->s_k1, std::max<uint64_t>(N, 1) * 8);
   ALLOC(c, c->x_occ, std::max<uint64_t>(N, 1) * 8);
   if (ensure_sort_temp(c, std::max<uint64_t>(N, 1)) != OIC_OK) return OIC_ENOMEM;
@@ -542,8 +543,8 @@ static int build_table(oic_ctx *c, uint32_t bgn, uint32_t end, std::vector<uint3
   ReadsDev R = dev_reads(c);
   uint64_t *keys = c->s_k1.as<uint64_t>(), *vals = c->x_occ.as<uint64_t>();
   if (N) {
-    hipLaunchKernelGGL(k_kmer_emit, dim3(nb), dim3(256), 0, c->st, R, bgn, nb, d_posbase.as<uint64_t>(), d_loaded.as<uint8_t>(), K,
-                       invalid, keys, vals);
+    hipLaunchKernelGGL(k_kmer_emit, dim3(nb), dim3(256), 0, c->st, R, bgn, nb, c->x_posbase.as<uint64_t>(),
+                       c->x_loaded.as<uint8_t>(), K, invalid, keys, vals);
     const int rc = sort_pairs(c, &keys, &vals, N, 2 * K + 1);   // stable: positions stay in (read, offset) order
     if (rc) return rc;
     // the sorted arrays may have moved into the temp buffers: swap ownership so x_occ holds vals
@@ -557,36 +558,22 @@ static int build_table(oic_ctx *c, uint32_t bgn, uint32_t end, std::vector<uint3
   uint64_t nu = 0;
   if (N) {
     const unsigned g = (unsigned)((N + 255) / 256);
-    hipLaunchKernelGGL(k_unique_flags, dim3(g), dim3(256), 0, c->st, keys, N, invalid, c->s_flag.as<uint32_t>());
+    hipLaunchKernelGGL(k_unique_flags, dim3(g), dim3(256), 0, c->st, keys, N, invalid, c->s_flag.as<uint32_t>(), d_nvalid);
     HIPCHK(c, scan_excl<uint32_t>(c->s_flag.as<uint32_t>(), c->s_idx.as<uint64_t>(), N, c->s_scan.as<uint64_t>(), c->st, &nu));
   }
   ALLOC(c, c->x_ukey, std::max<uint64_t>(nu, 1) * 8);
   ALLOC(c, c->x_ustart, (nu + 1) * 8);
-  // number of valid positions: invalid keys sort last
-  uint64_t nvalid = N;
-  if (N) {
-    std::vector<uint64_t> tail(1);
-    // binary search on host over device keys would need many copies; count invalid windows instead
-    uint64_t ninv = 0;
-    for (uint32_t t = 0; t < nb; t++) (void)t;
-    // invalid windows only exist in reads with N; find the first invalid key by bisection on device data
-    uint64_t lo = 0, hi = N;
-    while (lo < hi) {
-      const uint64_t mid = (lo + hi) / 2;
-      uint64_t kv = 0;
-      HIPCHK(c, hipMemcpyAsync(&kv, keys + mid, 8, hipMemcpyDeviceToHost, c->st));
-      HIPCHK(c, hipStreamSynchronize(c->st));
-      if (kv < invalid) lo = mid + 1; else hi = mid;
-    }
-    nvalid = lo;
-    (void)ninv;
+  const bool count_first = first_t && nu >= limit;
+  if (count_first) {
+    ALLOC(c, c->x_first, (uint64_t)nb * 4);
+    HIPCHK(c, hipMemsetAsync(c->x_first.p, 0, (uint64_t)nb * 4, c->st));
   }
   if (nu) {
     const unsigned g = (unsigned)((N + 255) / 256);
     hipLaunchKernelGGL(k_unique_write, dim3(g), dim3(256), 0, c->st, keys, vals, N, c->s_flag.as<uint32_t>(), c->s_idx.as<uint64_t>(),
-                       c->x_ukey.as<uint64_t>(), c->x_ustart.as<uint64_t>(), d_first.as<uint32_t>());
+                       c->x_ukey.as<uint64_t>(), c->x_ustart.as<uint64_t>(), count_first ? c->x_first.as<uint32_t>() : nullptr);
   }
-  HIPCHK(c, hipMemcpyAsync(c->x_ustart.as<uint64_t>() + nu, &nvalid, 8, hipMemcpyHostToDevice, c->st));
+  HIPCHK(c, hipMemcpyAsync(c->x_ustart.as<uint64_t>() + nu, d_nvalid, 8, hipMemcpyDeviceToDevice, c->st));
   int dbits = std::max(8, std::min(ceil_log2(std::max<uint64_t>(nu, 1)), std::min(2 * K, 28)));
   if (dbits > 2 * K) dbits = 2 * K;
   c->dshift = 2 * K - dbits;
@@ -597,9 +584,10 @@ static int build_table(oic_ctx *c, uint32_t bgn, uint32_t end, std::vector<uint3
     hipLaunchKernelGGL(k_build_dir, dim3(g), dim3(256), 0, c->st, c->x_ukey.as<uint64_t>(), nu, c->dshift, nbk, c->x_dir.as<uint64_t>());
   }
   HIPCHK(c, hipGetLastError());
-  if (first_t) {
+  if (first_t) first_t->clear();
+  if (count_first) {
     first_t->resize(nb);
-    HIPCHK(c, hipMemcpyAsync(first_t->data(), d_first.p, nb * 4, hipMemcpyDeviceToHost, c->st));
+    HIPCHK(c, hipMemcpyAsync(first_t->data(), c->x_first.p, (uint64_t)nb * 4, hipMemcpyDeviceToHost, c->st));
   }
   if (!c->skip.empty()) {
     ALLOC(c, c->x_tscreen, (uint64_t)nb * 4);
@@ -618,7 +606,6 @@ static int build_table(oic_ctx *c, uint32_t bgn, uint32_t end, std::vector<uint3
   }
   HIPCHK(c, hipStreamSynchronize(c->st));
   c->nu = nu;
-  c->nvalid = nvalid;
   c->hbgn = bgn;
   c->hend = end;
   c->nblock = nb;
@@ -645,16 +632,16 @@ extern "C" int oic_index_build(oic_ctx *c, uint32_t bgn, uint32_t end, uint32_t 
     if (c->h_len[r] >= c->P.min_olap) total += (uint64_t)c->h_len[r] + 1;
   }
   std::vector<uint32_t> first;
-  int rc = build_table(c, bgn, cand, &first);
+  int rc = build_table(c, bgn, cand, limit, &first);
   if (rc) return rc;
   uint64_t distinct = 0;
   uint32_t blk = cand;
-  for (uint32_t r = bgn; r <= cand; r++) {
+  for (uint32_t r = bgn; r <= cand && !first.empty(); r++) {
     if (distinct >= limit) { blk = r - 1; break; }
     distinct += first[r - bgn];
   }
   if (blk < cand) {
-    rc = build_table(c, bgn, blk, nullptr);
+    rc = build_table(c, bgn, blk, limit, nullptr);
     if (rc) return rc;
   }
   if (last_loaded) *last_loaded = blk;
