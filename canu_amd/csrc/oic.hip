@@ -729,8 +729,8 @@ static uint32_t ref_end_searched(uint32_t bgn, uint32_t end, uint32_t nthreads) 
   return ((end - bgn) % per == 0) ? end - 1 : end;
 }
 
-// model prediction (log1p cells) for every pair of the batch, on the device
-static int predict_pairs(oic_ctx *c, uint64_t np, std::vector<float> &pred) {
+// model prediction (log1p cells) for every pair of the batch; *bad (on the device) counts those that are not finite
+static int predict_pairs(oic_ctx *c, uint64_t np, uint32_t *bad) {
   ALLOC(c, c->m_feat, np * MLP_IN * 4);
   ALLOC(c, c->m_pred, np * MLP_OUT * 4);
   const unsigned g = (unsigned)((np + 255) / 256);
@@ -738,17 +738,32 @@ static int predict_pairs(oic_ctx *c, uint64_t np, std::vector<float> &pred) {
                      c->m_feat.as<float>());
   hipLaunchKernelGGL(k_mlp_forward, dim3(g), dim3(256), 0, c->st, c->m_feat.as<float>(), np, c->m_param.as<float>(),
                      c->m_mu.as<float>(), c->m_sd.as<float>(), c->m_pred.as<float>());
+  hipLaunchKernelGGL(k_not_finite, dim3(g), dim3(256), 0, c->st, c->m_pred.as<float>(), np, bad);
   HIPCHK(c, hipGetLastError());
-  std::vector<float> y(np * MLP_OUT);
-  HIPCHK(c, hipMemcpyAsync(y.data(), c->m_pred.p, np * MLP_OUT * 4, hipMemcpyDeviceToHost, c->st));
-  HIPCHK(c, hipStreamSynchronize(c->st));
-  pred.resize(np);
-  for (uint64_t p = 0; p < np; p++) pred[p] = y[p * MLP_OUT];
   return OIC_OK;
 }
 
 // the cost model's per-pair predictions (on the device) when they order this batch, else null
 static const float *spec_pred(oic_ctx *c) { return c->batch_pred ? c->m_pred.as<float>() : nullptr; }
+
+// p_order: the batch's pairs in the schedule's processing order.  The hit buffers are free once the match lists exist.
+static int order_pairs(oic_ctx *c, uint64_t np) {
+  const unsigned g = (unsigned)((np + 255) / 256);
+  uint64_t *k = nullptr, *v = nullptr;
+  if (c->P.schedule != OIC_SCHED_PLAIN && np > 1) {
+    ALLOC(c, c->s_k1, np * 8);
+    ALLOC(c, c->s_v1, np * 8);
+    if (ensure_sort_temp(c, np) != OIC_OK) return OIC_ENOMEM;
+    k = c->s_k1.as<uint64_t>();
+    v = c->s_v1.as<uint64_t>();
+    hipLaunchKernelGGL(k_order_keys, dim3(g), dim3(256), 0, c->st, c->p_pairs.as<PairRec>(), np, c->d_len.as<int32_t>(), spec_pred(c), k, v);
+    const int rc = sort_pairs(c, &k, &v, np, ORDER_BITS);
+    if (rc) return rc;
+  }
+  hipLaunchKernelGGL(k_order_write, dim3(g), dim3(256), 0, c->st, v, np, c->p_order.as<uint32_t>());
+  HIPCHK(c, hipGetLastError());
+  return OIC_OK;
+}
 
 // shapes that only the flat-row form runs (4 lanes per DP with a tile of 64 cells or fewer)
 template <int G, int CAP>
@@ -1334,7 +1349,8 @@ static int search_batch(oic_ctx *c, uint32_t s0, uint32_t ns, const std::vector<
     ALLOC(c, c->l_cnt, 64);
     HIPCHK(c, hipMemsetAsync(c->l_cnt.p, 0, 64, c->st));
     // cnt: [0] big pairs, [1] their queue, [2] handed back, [4..5] nodes, [6] queue of few hits, [7] handed back
-    // there, [8] long pairs, [9] parts, [10] pairs and parts with over 128 hits at an offset, [11] their queue
+    // there, [8] long pairs, [9] parts, [10] pairs and parts with over 128 hits at an offset, [11] their queue, [12]
+    // predictions that are not finite
     uint32_t *cnt = c->l_cnt.as<uint32_t>();
     uint32_t *big = c->l_big.as<uint32_t>(), *up = big + np, *lng = up + np + ntile + nlong, *lfirst = lng + nlong, *lcount = lfirst + nlong;
     hipLaunchKernelGGL(k_big_select, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, c->st, c->p_pairs.as<PairRec>(), np,
@@ -1400,6 +1416,11 @@ static int search_batch(oic_ctx *c, uint32_t s0, uint32_t ns, const std::vector<
                        c->p_tmp.as<int4>(), c->p_nodes.as<int4>(), K, LS, c->l_done.as<uint8_t>(), (uint8_t)2, BA.nnodes_total);
   }
   HIPCHK(c, hipGetLastError());
+  const bool predicted = c->P.schedule == OIC_SCHED_LEARNED && c->have_model;
+  if (predicted) {
+    const int rc = predict_pairs(c, np, c->l_cnt.as<uint32_t>() + 12);
+    if (rc) return rc;
+  }
   {
     uint32_t lc[16];
     HIPCHK(c, hipMemcpyAsync(lc, c->l_cnt.p, 64, hipMemcpyDeviceToHost, c->st));
@@ -1409,6 +1430,8 @@ static int search_batch(oic_ctx *c, uint32_t s0, uint32_t ns, const std::vector<
     c->ctr.list_second_level += lc[10];
     memcpy(&batch_nodes, lc + 4, 8);
     c->ctr.nodes += batch_nodes;
+    c->batch_pred = predicted && lc[12] == 0;
+    if (c->batch_pred) c->ctr.learned_pairs += np;
   }
   c->ctr.ms_lists += now_ms() - t1;
 
@@ -1421,22 +1444,10 @@ static int search_batch(oic_ctx *c, uint32_t s0, uint32_t ns, const std::vector<
   ALLOC(c, c->p_stats, STAT_NSTATS * 8);
   HIPCHK(c, hipMemsetAsync(c->p_stats.p, 0, STAT_NSTATS * 8, c->st));
   HIPCHK(c, hipMemsetAsync(c->p_pout.p, 0, np * sizeof(PairOut), c->st));
-  std::vector<uint32_t> order;
-  c->batch_pred = false;
   {
-    std::vector<float> pred;
-    if (c->P.schedule == OIC_SCHED_LEARNED && c->have_model) {
-      int rc = predict_pairs(c, np, pred);
-      if (rc) return rc;
-      bool finite = true;
-      for (float v : pred) finite = finite && std::isfinite(v);
-      if (finite) c->ctr.learned_pairs += np;
-      c->batch_pred = finite;
-    }
-    int rc = make_order(c->P.schedule, c->p_pairs.as<PairRec>(), np, c->h_len.data(), pred.empty() ? nullptr : pred.data(), c->st, order);
-    if (rc) return fail(c, OIC_EHIP, "scheduling failed");
+    const int rc = order_pairs(c, np);
+    if (rc) return rc;
   }
-  HIPCHK(c, hipMemcpyAsync(c->p_order.p, order.data(), np * 4, hipMemcpyHostToDevice, c->st));
 
   // batched schedules: forward DPs of probe and speculative nodes, packed 4 per wavefront
   // Under -partial every extension's delta is needed and none runs ahead; the rounds find no outcomes.
@@ -1470,51 +1481,47 @@ static int search_batch(oic_ctx *c, uint32_t s0, uint32_t ns, const std::vector<
   const uint32_t waves = (uint32_t)c->ncu * 16;
   int rc = in_rounds ? run_rounds(c, A, np, batch_nodes, &ms) : run_pairs<WR_FIRST>(c, A, np, waves, kFirstVals, &ms);
   if (rc) return rc;
-  // pairs whose band outgrew the small tile: rerun with the wide tile
-  std::vector<PairOut> pout(np);
-  HIPCHK(c, hipMemcpyAsync(pout.data(), c->p_pout.p, np * sizeof(PairOut), hipMemcpyDeviceToHost, c->st));
-  HIPCHK(c, hipStreamSynchronize(c->st));
-  std::vector<uint32_t> retry;
-  for (uint64_t p = 0; p < np; p++)
-    if (pout[p].status == 1) retry.push_back((uint32_t)p);
-  if (!retry.empty()) {
-    c->ctr.overflow_retries += retry.size();
-    ALLOC(c, c->p_retry, retry.size() * 4);
-    HIPCHK(c, hipMemcpyAsync(c->p_retry.p, retry.data(), retry.size() * 4, hipMemcpyHostToDevice, c->st));
+  // records to write, and the pairs whose band outgrew the small tile: these run again with the wide tile
+  ALLOC(c, c->p_nout, np * 4);
+  ALLOC(c, c->p_noff, np * 8);
+  ALLOC(c, c->p_retry, np * 4);
+  ALLOC(c, c->s_scan, scan_scratch_words(np) * 8);
+  const unsigned gp = (unsigned)((np + 255) / 256);
+  uint32_t *again = c->p_queue.as<uint32_t>() + 8;
+  uint64_t nrec = 0, stats[STAT_NSTATS];
+  for (int level = 0;; level++) {
+    uint32_t ag[2] = {0, 0};
+    hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, c->st, again, (uint64_t)1, 0u);
+    hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, c->st, again + 1, (uint64_t)1, 0xffffffffu);
+    hipLaunchKernelGGL(k_nout, dim3(gp), dim3(256), 0, c->st, c->p_pout.as<PairOut>(), np, c->p_nout.as<uint32_t>(), c->p_retry.as<uint32_t>(),
+                       again);
+    HIPCHK(c, hipMemcpyAsync(ag, again, sizeof ag, hipMemcpyDeviceToHost, c->st));
+    HIPCHK(c, hipMemcpyAsync(stats, c->p_stats.p, sizeof stats, hipMemcpyDeviceToHost, c->st));
+    HIPCHK(c, scan_excl<uint32_t>(c->p_nout.as<uint32_t>(), c->p_noff.as<uint64_t>(), np, c->s_scan.as<uint64_t>(), c->st, &nrec));
+    if (ag[0] == 0) break;
+    if (level == 1) {
+      PairRec pr;
+      HIPCHK(c, hipMemcpy(&pr, c->p_pairs.as<PairRec>() + ag[1], sizeof pr, hipMemcpyDeviceToHost));
+      return fail(c, OIC_EUNSUPPORTED, "pair S %u (%s) x T %u needs a DP band wider than the widest tile (%d cells)", pr.s_id,
+                  pr.dir ? "reverse" : "forward", pr.t_id, WR_MAX_BAND + 2);
+    }
+    c->ctr.overflow_retries += ag[0];
     A.order = c->p_retry.as<uint32_t>();
     const int32_t rows = c->T.error_bound[std::min<int32_t>(c->maxlen, (int32_t)oic::kMaxReadLen)] + 4;
     const int64_t vcap = std::min<int64_t>((int64_t)rows * WR_MAX_BAND, (int64_t)1 << 25);
-    rc = run_pairs<WR_WIDE>(c, A, retry.size(), std::min<uint32_t>(waves, 256), vcap, &ms);
+    rc = run_pairs<WR_WIDE>(c, A, ag[0], std::min<uint32_t>(waves, 256), vcap, &ms);
     if (rc) return rc;
-    HIPCHK(c, hipMemcpyAsync(pout.data(), c->p_pout.p, np * sizeof(PairOut), hipMemcpyDeviceToHost, c->st));
-    HIPCHK(c, hipStreamSynchronize(c->st));
-    for (uint64_t p = 0; p < np; p++)
-      if (pout[p].status == 1) {
-        PairRec pr;
-        HIPCHK(c, hipMemcpy(&pr, c->p_pairs.as<PairRec>() + p, sizeof pr, hipMemcpyDeviceToHost));
-        return fail(c, OIC_EUNSUPPORTED, "pair S %u (%s) x T %u needs a DP band wider than the widest tile (%d cells)", pr.s_id,
-                    pr.dir ? "reverse" : "forward", pr.t_id, WR_MAX_BAND + 2);
-      }
   }
   c->ctr.ms_dp_kernel += ms;
   c->ctr.ms_pp_kernel += ms;
   c->ctr.ms_extend += now_ms() - t2;
 
   // records
-  ALLOC(c, c->p_nout, np * 4);
-  ALLOC(c, c->p_noff, np * 8);
-  uint64_t nrec = 0;
-  hipLaunchKernelGGL(k_nout, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, c->st, c->p_pout.as<PairOut>(), np, c->p_nout.as<uint32_t>());
-  ALLOC(c, c->s_scan, scan_scratch_words(np) * 8);
-  HIPCHK(c, scan_excl<uint32_t>(c->p_nout.as<uint32_t>(), c->p_noff.as<uint64_t>(), np, c->s_scan.as<uint64_t>(), c->st, &nrec));
   if (nrec) {
     ALLOC(c, c->p_outrec, nrec * sizeof(OutRec));
-    hipLaunchKernelGGL(k_compact_recs, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, c->st, c->p_recs.as<OutRec>(), c->p_pout.as<PairOut>(),
+    hipLaunchKernelGGL(k_compact_recs, dim3(gp), dim3(256), 0, c->st, c->p_recs.as<OutRec>(), c->p_pout.as<PairOut>(),
                        c->p_noff.as<uint64_t>(), np, c->p_outrec.as<OutRec>());
   }
-  uint64_t stats[STAT_NSTATS];
-  HIPCHK(c, hipMemcpyAsync(stats, c->p_stats.p, sizeof stats, hipMemcpyDeviceToHost, c->st));
-  HIPCHK(c, hipStreamSynchronize(c->st));
   for (int i = 0; i < 6; i++) sink->stats[i] += stats[i];
   c->ctr.dp_cells += stats[STAT_CELLS];
   c->ctr.dp_lane_slots += stats[STAT_SLOTS];
@@ -1532,13 +1539,14 @@ static int search_batch(oic_ctx *c, uint32_t s0, uint32_t ns, const std::vector<
   const uint64_t room = (sink->records && sink->capacity > sink->count) ? sink->capacity - sink->count : 0;
   const uint64_t direct = c->pending.empty() ? std::min<uint64_t>(room, nrec) : 0;
   if (direct)
-    HIPCHK(c, hipMemcpy(sink->records + sink->count, c->p_outrec.p, direct * sizeof(OutRec), hipMemcpyDeviceToHost));
+    HIPCHK(c, hipMemcpyAsync(sink->records + sink->count, c->p_outrec.p, direct * sizeof(OutRec), hipMemcpyDeviceToHost, c->st));
   if (nrec > direct) {
     const size_t o = c->pending.size();
     c->pending.resize(o + (nrec - direct));
-    HIPCHK(c, hipMemcpy(c->pending.data() + o, c->p_outrec.as<OutRec>() + direct, (nrec - direct) * sizeof(OutRec),
-                        hipMemcpyDeviceToHost));
+    HIPCHK(c, hipMemcpyAsync(c->pending.data() + o, c->p_outrec.as<OutRec>() + direct, (nrec - direct) * sizeof(OutRec),
+                             hipMemcpyDeviceToHost, c->st));
   }
+  HIPCHK(c, hipStreamSynchronize(c->st));
   sink->count += direct;
   sink->records_needed = sink->count + c->pending.size();
   if (c->tracing) {
@@ -1547,7 +1555,10 @@ static int search_batch(oic_ctx *c, uint32_t s0, uint32_t ns, const std::vector<
                        c->d_len.as<int32_t>(), c->m_feat.as<float>());
     const size_t o = c->tr_feat.size();
     c->tr_feat.resize(o + np * MLP_IN);
-    HIPCHK(c, hipMemcpy(c->tr_feat.data() + o, c->m_feat.p, np * MLP_IN * 4, hipMemcpyDeviceToHost));
+    HIPCHK(c, hipMemcpyAsync(c->tr_feat.data() + o, c->m_feat.p, np * MLP_IN * 4, hipMemcpyDeviceToHost, c->st));
+    std::vector<PairOut> pout(np);
+    HIPCHK(c, hipMemcpyAsync(pout.data(), c->p_pout.p, np * sizeof(PairOut), hipMemcpyDeviceToHost, c->st));
+    HIPCHK(c, hipStreamSynchronize(c->st));
     for (uint64_t p = 0; p < np; p++) {
       c->tr_targ.push_back((float)std::log1p((double)pout[p].cells));
       c->tr_targ.push_back((float)(pout[p].exit_d / 1000.0));

@@ -1849,7 +1849,14 @@ __global__ void k_compact_recs(const OutRec *__restrict__ recs, const PairOut *_
   for (int32_t i = 0; i < n; i++) out[off[p] + i] = recs[p * OIC_MAX_DISTINCT + i];
 }
 
-__global__ void k_nout(const PairOut *__restrict__ pout, uint64_t np, uint32_t *__restrict__ n) {
+// records per pair; the pairs to be run again with the wide band (retry, any order; again[0] of them, again[1] the first)
+__global__ void k_nout(const PairOut *__restrict__ pout, uint64_t np, uint32_t *__restrict__ n, uint32_t *__restrict__ retry,
+                       uint32_t *__restrict__ again) {
   const uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p < np) n[p] = (uint32_t)pout[p].nout;
+  if (p >= np) return;
+  n[p] = (uint32_t)pout[p].nout;
+  if (pout[p].status == 1) {
+    retry[atomicAdd(&again[0], 1u)] = (uint32_t)p;
+    atomicMin(&again[1], (uint32_t)p);
+  }
 }
