@@ -1389,7 +1389,7 @@ static int search_batch(oic_ctx *c, uint32_t s0, uint32_t ns, const std::vector<
     HIPCHK(c, hipStreamSynchronize(c->st));
     uint32_t nit = 0;
     if (nl) {
-      hipLaunchKernelGGL(k_list_items, dim3(nl), dim3(OIC_WAVE), 0, c->st, BA.pairs, lng, c->l_split.as<uint64_t>(), BA.items, cnt + 9, lfirst,
+      hipLaunchKernelGGL(k_list_items, dim3(nl), dim3(LI_THREADS), 0, c->st, BA.pairs, lng, c->l_split.as<uint64_t>(), BA.items, cnt + 9, lfirst,
                          lcount);
       HIPCHK(c, hipMemcpyAsync(&nit, cnt + 9, 4, hipMemcpyDeviceToHost, c->st));
     }

@@ -74,9 +74,11 @@ struct RoundArgs {
 // where an extension's result comes from.
 __global__ void __launch_bounds__(OIC_WAVE) k_resolve_pairs(RoundArgs A) {
   __shared__ PairState st;
+  __shared__ PairStats pst;
   const int lane = lane_id();
   const SearchConst &C = A.C;
   uint64_t cells = 0, exts = 0;
+  clear_pair_stats(pst);
   while (true) {
     uint32_t f = 0;
     if (lane == 0) f = atomicAdd(&A.cnt->queue, 1u);
@@ -111,7 +113,7 @@ __global__ void __launch_bounds__(OIC_WAVE) k_resolve_pairs(RoundArgs A) {
         if (lane == 0) {
           po.status = 2;
           A.pout[p] = po;
-          atomicAdd(&A.stats[STAT_WITHOUT], 1ull);
+          pst.n[STAT_WITHOUT]++;
         }
         continue;
       }
@@ -269,9 +271,11 @@ __global__ void __launch_bounds__(OIC_WAVE) k_resolve_pairs(RoundArgs A) {
     }
     exts += (uint64_t)po.n_ext;
     cells += po.cells;
-    if (lane == 0) finish_pair(C, pr, S_Len, T_Len, st.olap, st.ct, po, A.out + (uint64_t)p * OIC_MAX_DISTINCT, A.pout + p, A.stats);
+    if (lane == 0) finish_pair(C, pr, S_Len, T_Len, st.olap, st.ct, po, A.out + (uint64_t)p * OIC_MAX_DISTINCT, A.pout + p, pst);
   }
-  if (lane == 0) {
+  __syncthreads();
+  add_pair_stats(pst, A.stats);
+  if (lane == 0 && exts) {
     atomicAdd(&A.stats[STAT_CELLS], (unsigned long long)cells);
     atomicAdd(&A.stats[STAT_EXT], (unsigned long long)exts);
   }

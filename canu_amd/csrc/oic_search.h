@@ -644,38 +644,54 @@ __global__ void __launch_bounds__(256) k_list_splits(const PairRec *__restrict__
   if (lane == 0) split[t] = at;
 }
 
-// One wavefront per long pair: its parts, numbered in order from first[j]; count[j] of them.
-__global__ void __launch_bounds__(OIC_WAVE) k_list_items(const PairRec *__restrict__ pairs, const uint32_t *__restrict__ lng,
-                                                         const uint64_t *__restrict__ split, ListItem *__restrict__ items,
-                                                         uint32_t *__restrict__ nitems, uint32_t *__restrict__ first,
-                                                         uint32_t *__restrict__ count) {
-  const int lane = lane_id();
+// One workgroup per long pair: its parts, numbered in order from first[j]; count[j] of them.  Eight wavefronts,
+// because a search's largest pair decides (one wavefront took 3 to 4 ms for 10^7 hits, with the 128-hit level waiting).
+#define LI_THREADS 512
+__global__ void __launch_bounds__(LI_THREADS) k_list_items(const PairRec *__restrict__ pairs, const uint32_t *__restrict__ lng,
+                                                           const uint64_t *__restrict__ split, ListItem *__restrict__ items,
+                                                           uint32_t *__restrict__ nitems, uint32_t *__restrict__ first,
+                                                           uint32_t *__restrict__ count) {
+  __shared__ uint32_t sum[LI_THREADS / OIC_WAVE], sId;
+  const int lane = lane_id(), tid = threadIdx.x, w = tid / OIC_WAVE;
   const uint32_t j = blockIdx.x, p = lng[j];
   const uint64_t hb = pairs[p].hb, he = pairs[p].he;
   const uint64_t t0 = (hb + LW_SPLIT - 1) / LW_SPLIT, t1 = (he - 1) / LW_SPLIT + 1;
-  uint32_t n = 1;
-  for (uint64_t t = t0; t < t1; t += OIC_WAVE)
-    n += (uint32_t)__builtin_popcountll(__ballot(t + lane < t1 && split[t + lane] != ~0ull));
-  uint32_t id = 0;
-  if (lane == 0) {
-    id = atomicAdd(nitems, n);
+  uint32_t mine = 0;
+  for (uint64_t t = t0 + tid; t < t1; t += LI_THREADS) mine += split[t] != ~0ull ? 1u : 0u;
+  for (int o = 32; o > 0; o >>= 1) mine += __shfl_xor(mine, o);
+  if (lane == 0) sum[w] = mine;
+  __syncthreads();
+  if (tid == 0) {
+    uint32_t n = 1;
+    for (int x = 0; x < LI_THREADS / OIC_WAVE; x++) n += sum[x];
+    const uint32_t id = atomicAdd(nitems, n);
+    sId = id;
     first[j] = id;
     count[j] = n;
     items[id].b = hb;
     items[id].pair = p;
     items[id + n - 1].e = he;
   }
-  id = (uint32_t)uni((int32_t)id);
-  for (uint64_t t = t0; t < t1; t += OIC_WAVE) {
-    const uint64_t at = t + lane < t1 ? split[t + lane] : ~0ull;
+  __syncthreads();
+  uint32_t id = sId;
+  for (uint64_t t = t0; t < t1; t += LI_THREADS) {
+    const uint64_t at = t + tid < t1 ? split[t + tid] : ~0ull;
     const uint64_t b = __ballot(at != ~0ull);
+    __syncthreads();                          // sum's readers are done
+    if (lane == 0) sum[w] = (uint32_t)__builtin_popcountll(b);
+    __syncthreads();
+    uint32_t before = 0, all = 0;
+    for (int x = 0; x < LI_THREADS / OIC_WAVE; x++) {
+      before += x < w ? sum[x] : 0u;
+      all += sum[x];
+    }
     if (at != ~0ull) {
-      const uint32_t k = id + (uint32_t)__builtin_popcountll(b & ((1ull << lane) - 1));
+      const uint32_t k = id + before + (uint32_t)__builtin_popcountll(b & ((1ull << lane) - 1));
       items[k].e = at;
       items[k + 1].b = at;
       items[k + 1].pair = p;
     }
-    id += (uint32_t)__builtin_popcountll(b);
+    id += all;
   }
 }
 
@@ -771,6 +787,7 @@ __global__ void __launch_bounds__(64) k_build_lists_wave(BigListArgs A) {
   const uint32_t nlist = A.big ? *A.nbig : (uint32_t)((A.np + LW_TAKE - 1) / LW_TAKE);
   const uint32_t nbig = nlist + (A.nitems ? *A.nitems : 0u);
   uint32_t work = 0, more = 0;      // pairs of a queue entry still to do (the small level)
+  uint64_t made = 0;                // nodes of this wavefront's pairs, added to the batch's at the end
   for (;;) {
     uint32_t p;
     if (more) {
@@ -1196,7 +1213,7 @@ __global__ void __launch_bounds__(64) k_build_lists_wave(BigListArgs A) {
       }
       continue;
     }
-    __threadfence();
+    __threadfence_block();          // dq is read back by this wavefront only (a fence for the device flushes the L2)
     __syncthreads();
     int4 *out = (part ? A.tmp : A.nodes) + hb;
     const int4 *R = sR[cur];
@@ -1239,7 +1256,7 @@ __global__ void __launch_bounds__(64) k_build_lists_wave(BigListArgs A) {
       A.items[entry & ~LW_ITEM] = item;
     } else if (lane == 0) {
       pr.nnodes = nA + ndq;
-      atomicAdd(A.nnodes_total, (unsigned long long)(nA + ndq));
+      made += (uint64_t)(nA + ndq);
       pr.consistent = consistent ? 1 : 0;
       pr.diag_bgn = (int32_t)(A.hval[hb] & 0x1fffff);
       pr.diag_end = (int32_t)(A.hval[he - 1] & 0x1fffff);
@@ -1251,6 +1268,7 @@ __global__ void __launch_bounds__(64) k_build_lists_wave(BigListArgs A) {
       A.pairs[p] = pr;
     }
   }
+  if (lane == 0 && made) atomicAdd(A.nnodes_total, (unsigned long long)made);
 }
 
 // ------------------------------------------------------------------ per-pair Process_Matches
@@ -1643,9 +1661,23 @@ __device__ __forceinline__ bool hopeless_pair(const SearchConst &C, const PairRe
   return hopeless;
 }
 
+// A wavefront's counts of its pairs' outcomes (STAT_WITHOUT .. STAT_DOVE), in LDS, added to the batch's once.  With
+// an atomic per pair and counter, all on one cache line, they bounded the launch: k_resolve_pairs over 82 thousand
+// pairs without an overlap 4.0 -> 1.1 ms, over 90 thousand with repeats 4.8 -> 1.8 ms.
+struct PairStats {
+  uint32_t n[STAT_DOVE + 1];
+};
+__device__ __forceinline__ void clear_pair_stats(PairStats &st) {
+  if (lane_id() <= STAT_DOVE) st.n[lane_id()] = 0;
+}
+__device__ __forceinline__ void add_pair_stats(const PairStats &st, unsigned long long *stats) {
+  const int lane = lane_id();
+  if (lane <= STAT_DOVE && st.n[lane]) atomicAdd(&stats[lane], (unsigned long long)st.n[lane]);
+}
+
 // a pair's end, on one lane: the selection among its distinct overlaps, its records and counts
 __device__ __forceinline__ void finish_pair(const SearchConst &C, const PairRec &pr, int32_t S_Len, int32_t T_Len, OlapDev *olap, int32_t ct,
-                                            PairOut po, OutRec *recs, PairOut *pout, unsigned long long *stats) {
+                                            PairOut po, OutRec *recs, PairOut *pout, PairStats &st) {
   int32_t deleted[OIC_MAX_DISTINCT] = {0, 0, 0};
   select_distinct(C, olap, ct, deleted);
   int32_t nout = 0;
@@ -1664,16 +1696,11 @@ __device__ __forceinline__ void finish_pair(const SearchConst &C, const PairRec 
   po.contained = cont;
   po.dovetail = dove;
   *pout = po;
-  if (nout == 0) atomicAdd(&stats[STAT_WITHOUT], 1ull);
-  else {
-    atomicAdd(&stats[STAT_WITH], 1ull);
-    if (nout > 1) atomicAdd(&stats[STAT_MULTI], 1ull);
-  }
-  atomicAdd(&stats[STAT_TOTAL], (unsigned long long)nout);
-  if (!C.partial) {
-    atomicAdd(&stats[STAT_CONT], (unsigned long long)cont);
-    atomicAdd(&stats[STAT_DOVE], (unsigned long long)dove);
-  }
+  st.n[nout == 0 ? STAT_WITHOUT : STAT_WITH]++;
+  if (nout > 1) st.n[STAT_MULTI]++;
+  st.n[STAT_TOTAL] += (uint32_t)nout;
+  st.n[STAT_CONT] += cont;
+  st.n[STAT_DOVE] += dove;
 }
 
 // Process_Matches (overlapInCore-Process_String_Overlaps.C:353-547) for one candidate pair per
@@ -1684,8 +1711,10 @@ __global__ void __launch_bounds__(OIC_WAVE) __attribute__((amdgpu_waves_per_eu(4
   __shared__ OlapDev olap[OIC_MAX_DISTINCT];
   __shared__ int32_t olap_ct;
   __shared__ uint32_t next_item;
+  __shared__ PairStats pst;
   const int lane = lane_id();
   const uint32_t w = blockIdx.x;
+  clear_pair_stats(pst);
   const DPScratch sc = wave_scratch(A, w);
   const SearchConst &C = A.C;
 
@@ -1724,7 +1753,7 @@ __global__ void __launch_bounds__(OIC_WAVE) __attribute__((amdgpu_waves_per_eu(4
       if (lane == 0) {
         po.status = 2;
         A.pout[p] = po;
-        atomicAdd(&A.stats[STAT_WITHOUT], 1ull);
+        pst.n[STAT_WITHOUT]++;
       }
       continue;
     }
@@ -1826,9 +1855,10 @@ __global__ void __launch_bounds__(OIC_WAVE) __attribute__((amdgpu_waves_per_eu(4
     }
 
     po.cells = cells - cells0;
-    if (lane == 0) finish_pair(C, pr, S_Len, T_Len, olap, olap_ct, po, A.recs + (uint64_t)p * OIC_MAX_DISTINCT, A.pout + p, A.stats);
+    if (lane == 0) finish_pair(C, pr, S_Len, T_Len, olap, olap_ct, po, A.recs + (uint64_t)p * OIC_MAX_DISTINCT, A.pout + p, pst);
     __syncthreads();
   }
+  add_pair_stats(pst, A.stats);
   for (int o = 32; o > 0; o >>= 1) lane_bases += __shfl_xor(lane_bases, o);
   if (lane == 0) {
     atomicAdd(&A.stats[STAT_BASES], (unsigned long long)lane_bases);
