@@ -79,6 +79,11 @@ constexpr uint64_t kPassBytesPerHit = 140;   // device bytes a search pass holds
 // at 2, 4, 8, 16, 32 per wavefront: 755 low-error reads 42, 37, 31, 29, 29 ms, 37 reads 6.8, 6.3, 5.6, 6.1, 5.9 ms,
 // 146 reads under -partial 12.5, 10.4, 9.8, 10.6, 12.9 ms; fewer rounds end fewer launches on their longest
 // extension, and past 8 the extensions that turn out to be removed cost more than that.
+// forward DPs of one pass up to which each takes a wavefront of its own, per CU: as measured (256 CUs), 17 ns a task
+// there, against 6 ns and 2 to 3 ms in the packed kernel whatever their number.  Whole calls at 64, 256 and 512 per CU:
+// 1490 pairs (126 thousand tasks) 26.1, 26.3, 23.3 ms, 82 thousand pairs 55.0, 54.9, 52.4, 90 thousand 37.0, 37.0,
+// 35.6, 113 thousand 27.2, 27.1, 26.6 ms; 37 low-error reads 11.0 -> 8.8 and 755 reads 45 -> 40 ms at each.
+constexpr uint64_t kFewTasks = 512;
 constexpr uint64_t kRoundTasks = (uint64_t)1 << 24;
 constexpr uint64_t kRoundWords = (uint64_t)1 << 27, kRoundWordsMin = (uint64_t)1 << 16;
 constexpr uint32_t kAheadMin = 2, kAheadMax = 64, kAheadFill = 8;
@@ -920,6 +925,7 @@ static int run_forward_passes(oic_ctx *c, uint64_t np, uint64_t H) {
   FA.stats = c->b_stats.as<unsigned long long>();
   FA.ntasks_dev = nullptr;
   FA.tstamp = nullptr;
+  FA.few = 0;
   double ms = 0;
   ALLOC(c, c->b_ovf, 2 * np * sizeof(FwdTask));
   ALLOC(c, c->b_novf, 16);
@@ -1033,11 +1039,13 @@ static int run_forward_passes_graph(oic_ctx *c, uint64_t np, uint64_t H, uint64_
     FA.nodes = c->p_nodes.as<int4>();
     FA.outc = c->b_outc.as<uint64_t>();
     FwdTask *ovf = c->b_ovf.as<FwdTask>();
+    const uint64_t few = c->tune.fwd_counters ? 0 : kFewTasks * (uint64_t)c->ncu;    // the counters are the packed kernel's
     // one pass: launch slot k (0 probe, 1 spec) uses queues/stats 3k..3k+2 and overflow counts 8+2k, 9+2k
     auto pass = [&](int k, const FwdTask *tasks, uint64_t n, const uint32_t *n_dev, uint64_t cap, FwdTask *ov1, FwdTask *ov2) -> int {
       FA.tasks = tasks; FA.ntasks = n; FA.ntasks_dev = n_dev;
       FA.queue = cnt + 3 * k; FA.stats = stats + 8 * (3 * k); FA.ovf = ov1; FA.novf = cnt + 8 + 2 * k;
       FA.tstamp = tst + 2 * k;
+      FA.few = few; FA.all = tasks; FA.nall = n; FA.nall_dev = n_dev;
       int rc = enqueue_fwd_narrow(c, FA, cap, ev ? ev[6 * k] : nullptr, ev ? ev[6 * k + 1] : nullptr);
       if (rc) return rc;
       FA.tstamp = nullptr;
@@ -1045,6 +1053,7 @@ static int run_forward_passes_graph(oic_ctx *c, uint64_t np, uint64_t H, uint64_
       FA.queue = cnt + 3 * k + 1; FA.stats = stats + 8 * (3 * k + 1); FA.ovf = ov2; FA.novf = cnt + 9 + 2 * k;
       if (c->tune.fwd_counters) enqueue_fwd<64, WR_FIRST, true>(c, FA, cap, ev ? ev[6 * k + 2] : nullptr, ev ? ev[6 * k + 3] : nullptr);
       else enqueue_fwd<64, WR_FIRST, false>(c, FA, cap, ev ? ev[6 * k + 2] : nullptr, ev ? ev[6 * k + 3] : nullptr);
+      FA.few = 0;
       FA.tasks = ov2; FA.ntasks = 0; FA.ntasks_dev = cnt + 9 + 2 * k;
       FA.queue = cnt + 3 * k + 2; FA.stats = stats + 8 * (3 * k + 2); FA.ovf = nullptr; FA.novf = nullptr;
       if (c->tune.fwd_counters) enqueue_fwd<64, WR_WIDE, true>(c, FA, cap, ev ? ev[6 * k + 4] : nullptr, ev ? ev[6 * k + 5] : nullptr);

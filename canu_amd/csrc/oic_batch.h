@@ -24,6 +24,14 @@
 
 #define OIC_SEQ_WIN 64      // words (16 bases each) of each tail staged in LDS
 #define FWD_CHUNK 8         // consecutive tasks a group takes from the queue at once
+// Items that a persistent wavefront takes from a queue at once, fewer as the rest runs out.  One counter answers about
+// 120 million times a second, whoever asks (8 ns each): 8 tasks for each group of the flat kernel were 3.5 of the 5.5 ms
+// of 3.5 million short DPs, and left groups idle at the end of long ones.  Per wavefront, shared by its groups: 5.5 ->
+// 4.1 ms there, 38.8 -> 36.1 ms for 6.7 million DPs of 4 % error reads.
+__device__ __forceinline__ uint32_t queue_share(uint64_t rest, uint32_t least, uint32_t most) {
+  const uint64_t s = rest / (2 * (uint64_t)gridDim.x);
+  return s < least ? least : (s > most ? most : (uint32_t)s);
+}
 
 struct FwdTask {
   uint32_t pair;
@@ -43,6 +51,10 @@ struct FwdArgs {
   FwdTask *ovf;             // tasks whose band outgrew the tile are appended here (if not null)
   uint32_t *novf;
   const uint32_t *ntasks_dev;  // if not null, the task count is read here when the kernel starts
+  uint64_t few;                // with at most so many tasks the packed kernel leaves them to k_fwd_wave,
+  const FwdTask *all;          // whose tasks are then these, the packed kernel's own: nall, or *nall_dev of them
+  uint64_t nall;
+  const uint32_t *nall_dev;
   unsigned long long *tstamp;  // if not null: [0] earliest wavefront start, [1] latest end (wall clock)
 };
 
@@ -329,6 +341,7 @@ __global__ void __launch_bounds__(OIC_WAVE) k_fwd_tasks(FwdArgs A) {
   uint32_t rows_acc = 0, slots_acc = 0, wrows_acc = 0, bases_acc = 0, siters_acc = 0, wsiters_acc = 0;
   uint64_t ti = 0, tend = 0;
   const uint64_t ntasks = A.ntasks_dev ? (uint64_t)*A.ntasks_dev : A.ntasks;
+  if (ntasks <= A.few) return;
   if (A.tstamp && lane == 0) atomicMin(&A.tstamp[0], (unsigned long long)wall_clock64());
 
   while (true) {
@@ -441,12 +454,17 @@ __global__ void __launch_bounds__(OIC_WAVE) k_fwd_tasks(FwdArgs A) {
 }
 
 // The same tasks one to a wavefront (oic_wdp.h): the packed kernels' tasks whose band outgrew their tile, then
-// those whose band outgrew the first level.
+// those whose band outgrew the first level; and all of them when they are few.  A DP's row takes the packed kernel
+// about 1.5 us with 16 DPs in step and 0.2 us here, so few tasks (at most `few`) end earlier here, and true
+// overlaps, whose bands outgrow the packed tile after some hundred rows, aren't begun twice.
 template <int RING, bool STATS>
 __global__ void __launch_bounds__(OIC_WAVE) __attribute__((amdgpu_waves_per_eu(4, 8))) k_fwd_wave(FwdArgs A) {
   __shared__ WaveBand<RING> band;
   const int lane = lane_id();
-  const uint32_t ntasks = (uint32_t)uni((int32_t)(A.ntasks_dev ? *A.ntasks_dev : (uint32_t)A.ntasks));
+  const uint32_t nall = A.few ? (uint32_t)uni((int32_t)(A.nall_dev ? *A.nall_dev : (uint32_t)A.nall)) : 0u;
+  const bool direct = A.few && nall <= A.few;
+  const uint32_t ntasks = direct ? nall : (uint32_t)uni((int32_t)(A.ntasks_dev ? *A.ntasks_dev : (uint32_t)A.ntasks));
+  const FwdTask *tasks = direct ? A.all : A.tasks;
   const DPScratch sc = {};
   uint64_t cells_acc = 0, slots_acc = 0, bases_acc = 0;
   uint32_t rows_acc = 0;
@@ -455,7 +473,7 @@ __global__ void __launch_bounds__(OIC_WAVE) __attribute__((amdgpu_waves_per_eu(4
     if (lane == 0) f = atomicAdd(A.queue, 1u);
     const uint32_t ti = (uint32_t)uni((int32_t)f);
     if (ti >= ntasks) break;
-    const FwdTask tk = A.tasks[ti];
+    const FwdTask tk = tasks[ti];
     const PairRec pr = A.pairs[tk.pair];
     const uint64_t gnode = pr.hb + tk.node;
     const int4 nd = A.nodes[gnode];
@@ -832,6 +850,7 @@ k_fwd_sm(FwdArgs A) {
   uint32_t rows_acc = 0, slots_acc = 0, wrows_acc = 0, bases_acc = 0, siters_acc = 0, wsiters_acc = 0, wchunks_acc = 0;
   uint64_t ti = 0, tend = 0;
   const uint64_t ntasks = A.ntasks_dev ? (uint64_t)*A.ntasks_dev : A.ntasks;
+  if (ntasks <= A.few) return;
   if (A.tstamp && lane == 0) atomicMin(&A.tstamp[0], (unsigned long long)wall_clock64());
 
   SMDP s;

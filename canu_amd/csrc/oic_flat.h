@@ -287,8 +287,10 @@ k_fwd_flat(FwdArgs A) {
   uint64_t cells_acc = 0;
   uint32_t rows_acc = 0;
   uint64_t lstat[6] = {0, 0, 0, 0, 0, 0};   // lane slots, bases, slide windows, wave slide windows, wave chunks, wave rows
-  uint64_t ti = 0, tend = 0;
+  uint64_t ti = 0;
+  uint32_t pool = 0, pool_end = 0;   // the wavefront's tasks still to be given to its groups
   const uint64_t ntasks = A.ntasks_dev ? (uint64_t)*A.ntasks_dev : A.ntasks;
+  if (ntasks <= A.few) return;
   if (A.tstamp && lane == 0) atomicMin(&A.tstamp[0], (unsigned long long)wall_clock64());
 
   SMDP s;
@@ -338,7 +340,6 @@ k_fwd_flat(FwdArgs A) {
       if (!overflow) cells_acc += res.cells;
       rows_acc += res.rows;
     }
-    ti++;
     state = 0;
   };
   // the forward DP is over: take its outcome, then run the reverse DP or finish the task
@@ -351,14 +352,26 @@ k_fwd_flat(FwdArgs A) {
   };
 
   while (true) {
-    while (state == 0) {
-      if (ti == tend) {                      // group-uniform: take the next FWD_CHUNK tasks
+    // groups without a DP take the wavefront's next tasks, and the wavefront new ones when those run out
+    for (uint64_t asking; (asking = __ballot(state == 0)) != 0;) {
+      uint64_t first = 0;                    // their first lanes
+#pragma unroll
+      for (int i = 0; i < OIC_WAVE / G; i++) first |= 1ull << (i * G);
+      const uint32_t want = (uint32_t)__builtin_popcountll(asking & first), left = pool_end - pool;
+      uint32_t more = 0;
+      if (want > left) {
+        const uint32_t share = queue_share(pool < ntasks ? ntasks - pool : 0, OIC_WAVE / G, 8 * (OIC_WAVE / G));
         uint32_t f = 0;
-        if (gl == 0) f = atomicAdd(A.queue, (uint32_t)FWD_CHUNK);
-        ti = (uint32_t)__shfl((int)f, g * G);  // from the group's first lane
-        tend = ti + FWD_CHUNK < ntasks ? ti + FWD_CHUNK : ntasks;
+        if (lane == 0) f = atomicAdd(A.queue, share);
+        more = (uint32_t)uni((int32_t)f);
+        pool_end = more + share;
       }
-      if (ti >= ntasks) { state = 3; break; }
+      const uint32_t rank = (uint32_t)__builtin_popcountll(asking & first & ((1ull << (g * G)) - 1));
+      const uint32_t mine = rank < left ? pool + rank : more + (rank - left);
+      pool = want > left ? more + (want - left) : pool + want;
+      if (state != 0) continue;
+      ti = mine;
+      if (ti >= ntasks) { state = 3; continue; }
       res.cells = 0; res.rows = 0; res.slots = 0; res.wrows = 0; res.bases = 0; res.siters = 0; res.wsiters = 0; res.wchunks = 0;
       res.mte = true; res.overflow = false; res.e = 0; res.d = 0;
       lmte = true;
@@ -390,7 +403,7 @@ k_fwd_flat(FwdArgs A) {
       if (!sm_start<G, SW>(s, res, A.R.words, A.R.nmask, L.tile[g], L.seq[g][0], L.seq[g][1], g, gl)) {
         flat_desc_start<G, CAP>(L, s, g, gl);
         state = 1;
-        break;
+        continue;
       }
       forward_done();
     }

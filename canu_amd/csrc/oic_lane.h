@@ -100,6 +100,7 @@ k_fwd_lane(FwdArgs A) {
   int32_t *const my = ring + lane;              // slot s of this lane: my[s * 64]
   uint32_t *const sa = stage + lane, *const sb = stage + LN_SW * OIC_WAVE + lane;   // word k: s?[k * 64]
   const uint64_t ntasks = A.ntasks_dev ? (uint64_t)*A.ntasks_dev : A.ntasks;
+  if (ntasks <= A.few) return;
   if (A.tstamp && lane == 0) atomicMin(&A.tstamp[0], (unsigned long long)wall_clock64());
   const uint32_t *__restrict__ words = A.R.words;
   const DPTables &tb = A.tb;

@@ -79,10 +79,15 @@ __global__ void __launch_bounds__(OIC_WAVE) k_resolve_pairs(RoundArgs A) {
   const SearchConst &C = A.C;
   uint64_t cells = 0, exts = 0;
   clear_pair_stats(pst);
-  while (true) {
-    uint32_t f = 0;
-    if (lane == 0) f = atomicAdd(&A.cnt->queue, 1u);
-    const uint32_t qi = (uint32_t)uni((int32_t)f);
+  // a pair each, the most expensive ones, then four at a time from the queue
+  uint32_t qi = blockIdx.x, qend = qi + 1;
+  for (;; qi++) {
+    if (qi == qend) {
+      uint32_t f = 0;
+      if (lane == 0) f = atomicAdd(&A.cnt->queue, 4u);
+      qi = gridDim.x + (uint32_t)uni((int32_t)f);
+      qend = qi + 4;
+    }
     if (qi >= A.n) break;
     const uint32_t p = A.list[qi];
     const PairRec pr = A.pairs[p];
