@@ -86,7 +86,9 @@ constexpr uint64_t kPassBytesPerHit = 140;   // device bytes a search pass holds
 constexpr uint64_t kFewTasks = 512;
 constexpr uint64_t kRoundTasks = (uint64_t)1 << 24;
 constexpr uint64_t kRoundWords = (uint64_t)1 << 27, kRoundWordsMin = (uint64_t)1 << 16;
-constexpr uint32_t kAheadMin = 2, kAheadMax = 64, kAheadFill = 8;
+// With more pairs than wavefronts a round's last extensions cost more than that still: 755 reads (11.4 thousand pairs)
+// 39.2 -> 35.7 ms at 16, the same at 24 and 32, and 113 thousand pairs of compressed reads 24.0 -> 23.7 ms.
+constexpr uint32_t kAheadMin = 2, kAheadMax = 64, kAheadFill = 8, kAheadFillMany = 16;
 
 }  // namespace
 
@@ -1180,7 +1182,7 @@ static int run_rounds(oic_ctx *c, const PairKernelArgs &PA, uint64_t np, uint64_
   A.recs = c->r_recs.as<ExtRec>();
   A.masks = c->r_masks.as<uint64_t>();
   A.cnt = c->r_cnt.as<RoundCount>();
-  const uint32_t ewaves = (uint32_t)c->ncu * 16;
+  const uint32_t ewaves = (uint32_t)c->ncu * 16, fill = np > ewaves ? kAheadFillMany : kAheadFill;
   HIPCHK(c, hipEventRecord(c->ev0, c->st));
   hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, c->st, (uint32_t *)A.cnt, (uint64_t)(sizeof(RoundCount) / 4), 0u);
   A.list = PA.order;
@@ -1190,7 +1192,7 @@ static int run_rounds(oic_ctx *c, const PairKernelArgs &PA, uint64_t np, uint64_
   uint32_t left = 0;
   for (int round = 0;; round++) {
     A.open = open[round & 1];
-    A.ahead = (int32_t)std::max<uint32_t>(kAheadMin, std::min<uint32_t>(kAheadMax, kAheadFill * ewaves / std::max<uint32_t>(A.n, 1)));
+    A.ahead = (int32_t)std::max<uint32_t>(kAheadMin, std::min<uint32_t>(kAheadMax, fill * ewaves / std::max<uint32_t>(A.n, 1)));
     A.resume = round > 0 ? 1 : 0;
     hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, c->st, (uint32_t *)A.cnt, (uint64_t)4, 0u);
     hipLaunchKernelGGL(k_resolve_pairs, dim3(std::min<uint32_t>(A.n, (uint32_t)c->ncu * 32)), dim3(OIC_WAVE), 0, c->st, A);

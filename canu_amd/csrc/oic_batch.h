@@ -99,7 +99,7 @@ __device__ __forceinline__ uint32_t win16_staged(const uint32_t *__restrict__ wo
   const int32_t q = t.r0 + p;
   const int32_t wi = q >> 4;
   const uint32_t sh = (uint32_t)q * 2u;   // alignbit shifts by this modulo 32: 2 (q mod 16)
-  if (wi + 1 < SW) return __builtin_amdgcn_alignbit(t.lds[wi + 1], t.lds[wi], sh);
+  if (SW > 0 && wi + 1 < SW) return __builtin_amdgcn_alignbit(t.lds[wi + 1], t.lds[wi], sh);
   return __builtin_amdgcn_alignbit(words[t.w0 + wi + 1], words[t.w0 + wi], sh);
 }
 
@@ -587,10 +587,17 @@ __device__ __forceinline__ void words5_staged(const uint32_t *__restrict__ words
 }
 
 // the three words from word wi of a staged tail: read from its LDS copy (at a clamped index, so
-// always in bounds), and reloaded from HBM by the lanes whose words lie past the copy
+// always in bounds), and reloaded from HBM by the lanes whose words lie past the copy; with no copy
+// (SW = 0), in one load
 template <int SW = OIC_SEQ_WIN>
 __device__ __forceinline__ void words3_staged(const uint32_t *__restrict__ words, const Staged &t, int32_t wi, uint32_t &w0,
                                               uint32_t &w1, uint32_t &w2) {
+  if constexpr (SW == 0) {
+    struct __attribute__((packed, aligned(4))) Words3 { uint32_t x, y, z; };
+    const Words3 v = *(const Words3 *)(words + t.w0 + wi);
+    w0 = v.x; w1 = v.y; w2 = v.z;
+    return;
+  }
   const int32_t wl = wi < SW - 3 ? wi : SW - 3;
   w0 = t.lds[wl]; w1 = t.lds[wl + 1]; w2 = t.lds[wl + 2];
   if (wi > SW - 3) {

@@ -15,10 +15,11 @@
 // LDS decides how many wavefronts a CU holds, so each DP keeps one band buffer, updated in place:
 // in a chunk every lane reads its three cells of the previous row before any lane writes, and the
 // one cell a run's first lane needs from the chunk before (its left neighbour, already
-// overwritten) comes from the lane that read it there, by a shuffle.  With 4 lanes per DP the
-// first 128 bases of each tail are staged (SW = 8 words), else 1024: longer windows measured slower
-// on both the repeat-rich and the low-error reads, their copy at every DP start costing more than
-// the cached reads past them.
+// overwritten) comes from the lane that read it there, by a shuffle.  With 4 lanes per DP the tails
+// are read where they are (SW = 0): a DP soon passes any copy that LDS has room for, and a chunk in
+// which one lane has done so runs both reads.  (128 bases staged, 114 VGPRs, 16 wavefronts per CU:
+// 36.1 ms for 6.7 million DPs of 4 % error reads; none, 106 VGPRs: 32.8 ms; held to 96 VGPRs, which
+// takes no spill, and 20 wavefronts: 29.4 ms.)  With 8 lanes per DP the first 1024 bases are staged.
 
 #pragma once
 
@@ -31,7 +32,7 @@ struct FlatDesc {
 };
 
 template <int G>
-constexpr int flat_sw() { return G == 4 ? 8 : OIC_SEQ_WIN; }
+constexpr int flat_sw() { return G == 4 ? 0 : OIC_SEQ_WIN; }
 
 // Each DP's band buffer holds its CAP ring cells, then copies of cells 0 and 1 (so the three cells
 // d - 1, d, d + 1 are three consecutive words from (d - 1) mod CAP), then one spare word: strides of
@@ -41,7 +42,7 @@ struct FlatLDS {
   static constexpr int NG = OIC_WAVE / G;
   static constexpr int SW = flat_sw<G>();
   // a DP's two staged tails side by side (A, then T; SW + 1 words each): one base register
-  // addresses both within the 8-bit dword offsets of paired LDS reads
+  // addresses both within the 8-bit dword offsets of paired LDS reads (SW = 0: not used)
   uint32_t seq[NG][2][SW + 1];
   int32_t tile[NG][CAP + 3];
   FlatDesc desc[NG];
@@ -50,13 +51,14 @@ struct FlatLDS {
   int32_t start[OIC_WAVE];
 };
 
-// Wavefronts per SIMD the flat kernel's LDS allows, at most 4: registers are held to that
-// occupancy (128 VGPRs), which the cell loop's per-lane DP copy needs without spilling.
-// (4 x 64: 10 KB of LDS per wavefront, 16 per CU.)
+// Wavefronts per SIMD the flat kernel's LDS allows, at most 5 without staged tails and 4 with them:
+// registers are held to that occupancy (96 and 128 VGPRs), which takes no spill.
+// (4 x 64: 6 KB of LDS per wavefront, 20 per CU.)
 template <int G, int CAP>
 constexpr int flat_waves_per_eu() {
   constexpr int w = (163840 / (int)sizeof(FlatLDS<G, CAP>) + 3) / 4;
-  return w < 1 ? 1 : (w > 4 ? 4 : w);
+  constexpr int most = flat_sw<G>() ? 4 : 5;
+  return w < 1 ? 1 : (w > most ? most : w);
 }
 
 // the descriptor fields that stay fixed for a DP's rows, written when the DP starts
