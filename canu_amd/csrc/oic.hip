@@ -757,7 +757,7 @@ static const float *spec_pred(oic_ctx *c) { return c->batch_pred ? c->m_pred.as<
 static int order_pairs(oic_ctx *c, uint64_t np) {
   const unsigned g = (unsigned)((np + 255) / 256);
   uint64_t *k = nullptr, *v = nullptr;
-  if (c->P.schedule != OIC_SCHED_PLAIN && np > 1) {
+  if (np > 1) {
     ALLOC(c, c->s_k1, np * 8);
     ALLOC(c, c->s_v1, np * 8);
     if (ensure_sort_temp(c, np) != OIC_OK) return OIC_ENOMEM;

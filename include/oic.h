@@ -68,7 +68,7 @@ typedef struct oic_params {
   int32_t  schedule;         /* OIC_SCHED_* */
 } oic_params;
 
-#define OIC_SCHED_PLAIN    0  /* one candidate pair per wavefront, pairs in discovery order */
+#define OIC_SCHED_PLAIN    0  /* one candidate pair per wavefront, by a static cost estimate */
 #define OIC_SCHED_BATCHED  1  /* binned, load-balanced persistent launches (static length bins) */
 #define OIC_SCHED_LEARNED  2  /* as BATCHED, pairs binned and ordered by the learned cost model */
 
