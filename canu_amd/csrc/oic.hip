@@ -1041,7 +1041,8 @@ static int run_forward_passes_graph(oic_ctx *c, uint64_t np, uint64_t H, uint64_
     FA.nodes = c->p_nodes.as<int4>();
     FA.outc = c->b_outc.as<uint64_t>();
     FwdTask *ovf = c->b_ovf.as<FwdTask>();
-    const uint64_t few = c->tune.fwd_counters ? 0 : kFewTasks * (uint64_t)c->ncu;    // the counters are the packed kernel's
+    // the counters are the packed kernel's, and a form other than the flat rows is one that was asked for
+    const uint64_t few = c->tune.fwd_counters || c->tune.fwd_loop != 2 ? 0 : kFewTasks * (uint64_t)c->ncu;
     // one pass: launch slot k (0 probe, 1 spec) uses queues/stats 3k..3k+2 and overflow counts 8+2k, 9+2k
     auto pass = [&](int k, const FwdTask *tasks, uint64_t n, const uint32_t *n_dev, uint64_t cap, FwdTask *ov1, FwdTask *ov2) -> int {
       FA.tasks = tasks; FA.ntasks = n; FA.ntasks_dev = n_dev;
