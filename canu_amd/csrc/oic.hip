@@ -73,19 +73,24 @@ int ceil_log2(uint64_t x) {
 }
 
 constexpr int64_t kFirstVals = (int64_t)1 << 19;        // band cells a wavefront keeps for its traceback at the first level
-constexpr uint64_t kPassBytesPerHit = 140;   // device bytes a search pass holds per seed hit (hits, sort, lists, nodes, outcomes)
-// rounds of Process_Matches (oic_rounds.h): extensions and node-mask words a batch may hold; how many extensions a
-// pair may ask for in one round: as many as give each resident wavefront kAheadFill, within the limits.  Measured
-// at 2, 4, 8, 16, 32 per wavefront: 755 low-error reads 42, 37, 31, 29, 29 ms, 37 reads 6.8, 6.3, 5.6, 6.1, 5.9 ms,
-// 146 reads under -partial 12.5, 10.4, 9.8, 10.6, 12.9 ms; fewer rounds end fewer launches on their longest
-// extension, and past 8 the extensions that turn out to be removed cost more than that.
+// device bytes a search pass holds per seed hit (hits, sort, lists, nodes, outcomes).  Its candidate pairs, with some 300
+// bytes each, and Process_Matches' scratch (kRound*, and a row store per wavefront) come out of the rest.
+constexpr uint64_t kPassBytesPerHit = 140;
 // forward DPs of one pass up to which each takes a wavefront of its own, per CU: as measured (256 CUs), 17 ns a task
 // there, against 6 ns and 2 to 3 ms in the packed kernel whatever their number.  Whole calls at 64, 256 and 512 per CU:
 // 1490 pairs (126 thousand tasks) 26.1, 26.3, 23.3 ms, 82 thousand pairs 55.0, 54.9, 52.4, 90 thousand 37.0, 37.0,
 // 35.6, 113 thousand 27.2, 27.1, 26.6 ms; 37 low-error reads 11.0 -> 8.8 and 755 reads 45 -> 40 ms at each.
 constexpr uint64_t kFewTasks = 512;
+// Rounds of Process_Matches (oic_rounds.h).  They hold a state of 208 bytes per pair, so more pairs than kRoundPairs
+// take their rounds one part after another (in processing order: 78 thousand pairs are a whole pass of the repeat-rich
+// 30x workload), and extensions and node-mask words within these limits (0.9 GB and 1 GB).
+constexpr uint64_t kRoundPairs = (uint64_t)1 << 20;
 constexpr uint64_t kRoundTasks = (uint64_t)1 << 24;
 constexpr uint64_t kRoundWords = (uint64_t)1 << 27, kRoundWordsMin = (uint64_t)1 << 16;
+// How many extensions a pair may ask for in one round: as many as give each resident wavefront kAheadFill, within the
+// limits.  Measured at 2, 4, 8, 16, 32 per wavefront: 755 low-error reads 42, 37, 31, 29, 29 ms, 37 reads 6.8, 6.3, 5.6,
+// 6.1, 5.9 ms, 146 reads under -partial 12.5, 10.4, 9.8, 10.6, 12.9 ms; fewer rounds end fewer launches on their longest
+// extension, and past 8 the extensions that turn out to be removed cost more than that.
 // With more pairs than wavefronts a round's last extensions cost more than that still: 755 reads (11.4 thousand pairs)
 // 39.2 -> 35.7 ms at 16, the same at 24 and 32, and 113 thousand pairs of compressed reads 24.0 -> 23.7 ms.
 constexpr uint32_t kAheadMin = 2, kAheadMax = 64, kAheadFill = 8, kAheadFillMany = 16;
@@ -1156,8 +1161,8 @@ static int run_forward_passes_graph(oic_ctx *c, uint64_t np, uint64_t H, uint64_
   return OIC_OK;
 }
 
-// Process_Matches of the batch's pairs in rounds (oic_rounds.h).  list (np pairs, processing order) may be
-// overwritten.  Pairs that the rounds' arrays could not hold run one to a wavefront at the end.
+// Process_Matches of the np pairs of PA.order in rounds (oic_rounds.h).  Pairs that the rounds' arrays could not hold
+// run one to a wavefront at the end.
 static int run_rounds(oic_ctx *c, const PairKernelArgs &PA, uint64_t np, uint64_t nnodes, double *ms) {
   RoundArgs A{};
   A.R = PA.R;
@@ -1186,7 +1191,8 @@ static int run_rounds(oic_ctx *c, const PairKernelArgs &PA, uint64_t np, uint64_
   const uint32_t ewaves = (uint32_t)c->ncu * 16, fill = np > ewaves ? kAheadFillMany : kAheadFill;
   HIPCHK(c, hipEventRecord(c->ev0, c->st));
   hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, c->st, (uint32_t *)A.cnt, (uint64_t)(sizeof(RoundCount) / 4), 0u);
-  A.list = PA.order;
+  A.order = PA.order;
+  A.list = nullptr;
   A.n = (uint32_t)np;
   uint32_t *open[2] = {c->r_open.as<uint32_t>(), c->r_open.as<uint32_t>() + np};
   RoundCount rc{};
@@ -1225,7 +1231,7 @@ static int run_rounds(oic_ctx *c, const PairKernelArgs &PA, uint64_t np, uint64_
   hipEventElapsedTime(&f, c->ev0, c->ev1);
   *ms += f;
   if (left) {
-    hipLaunchKernelGGL(k_reopen_pairs, dim3(left), dim3(OIC_WAVE), 0, c->st, A.pairs, A.open, A.nodes);
+    hipLaunchKernelGGL(k_reopen_pairs, dim3(left), dim3(OIC_WAVE), 0, c->st, A.pairs, A.order, A.open, A.nodes);
     PairKernelArgs B = PA;
     B.order = A.open;
     return run_pairs<WR_FIRST>(c, B, left, (uint32_t)c->ncu * 16, kFirstVals, ms);
@@ -1491,7 +1497,12 @@ static int search_batch(oic_ctx *c, uint32_t s0, uint32_t ns, const std::vector<
   A.stats = c->p_stats.as<unsigned long long>();
   double ms = 0;
   const uint32_t waves = (uint32_t)c->ncu * 16;
-  int rc = in_rounds ? run_rounds(c, A, np, batch_nodes, &ms) : run_pairs<WR_FIRST>(c, A, np, waves, kFirstVals, &ms);
+  int rc = in_rounds ? OIC_OK : run_pairs<WR_FIRST>(c, A, np, waves, kFirstVals, &ms);
+  for (uint64_t p0 = 0; in_rounds && p0 < np && rc == OIC_OK; p0 += kRoundPairs) {
+    PairKernelArgs B = A;
+    B.order += p0;
+    rc = run_rounds(c, B, std::min(np - p0, kRoundPairs), batch_nodes, &ms);
+  }
   if (rc) return rc;
   // records to write, and the pairs whose band outgrew the small tile: these run again with the wide tile
   ALLOC(c, c->p_nout, np * 4);

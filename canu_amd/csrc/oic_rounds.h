@@ -49,12 +49,13 @@ struct RoundArgs {
   int4 *nodes;
   uint64_t *outc;            // per node: pack_outcome, kind 3 (OUTC_EXT): the extension's index in the low word
   const float *pred;         // the cost model's log(1 + DP cells) per pair (two floats a pair), or nullptr
-  const uint32_t *list;      // open pairs, n of them; those still open afterwards go to open[]
-  uint32_t n;
+  const uint32_t *order;     // the pairs of these rounds
+  const uint32_t *list;      // their open ones, n places in order[], or nullptr: all n of them; those still open
+  uint32_t n;                // afterwards go to open[]
   uint32_t *open;
   int resume;                // 0: the first round
   int32_t ahead;             // extensions a pair may ask for at once
-  PairState *state;          // per pair
+  PairState *state;          // per place in order[]
   ExtNode *tasks;
   ExtRec *recs;
   uint64_t *masks;
@@ -89,7 +90,7 @@ __global__ void __launch_bounds__(OIC_WAVE) k_resolve_pairs(RoundArgs A) {
       qend = qi + 4;
     }
     if (qi >= A.n) break;
-    const uint32_t p = A.list[qi];
+    const uint32_t at = A.list ? A.list[qi] : qi, p = A.order[at];
     const PairRec pr = A.pairs[p];
     int4 *nodes = A.nodes + pr.hb;
     uint64_t *outc = A.outc + pr.hb;
@@ -100,7 +101,7 @@ __global__ void __launch_bounds__(OIC_WAVE) k_resolve_pairs(RoundArgs A) {
     bool first = true;
     __syncthreads();
     if (A.resume) {
-      const uint32_t *src = (const uint32_t *)(A.state + p);
+      const uint32_t *src = (const uint32_t *)(A.state + at);
       for (int i = lane; i < (int)(sizeof(PairState) / 4); i += OIC_WAVE) ((uint32_t *)&st)[i] = src[i];
       __syncthreads();
       po = st.po;
@@ -261,10 +262,10 @@ __global__ void __launch_bounds__(OIC_WAVE) k_resolve_pairs(RoundArgs A) {
       if (lane == 0) {
         st.po = po;
         st.first = first ? 1 : 0;
-        A.open[atomicAdd(&A.cnt->nopen, 1u)] = p;
+        A.open[atomicAdd(&A.cnt->nopen, 1u)] = at;
       }
       __syncthreads();
-      uint32_t *dst = (uint32_t *)(A.state + p);
+      uint32_t *dst = (uint32_t *)(A.state + at);
       for (int i = lane; i < (int)(sizeof(PairState) / 4); i += OIC_WAVE) dst[i] = ((const uint32_t *)&st)[i];
       continue;
     }
@@ -348,9 +349,12 @@ __global__ void __launch_bounds__(OIC_WAVE) __attribute__((amdgpu_waves_per_eu(4
   }
 }
 
-// pairs given back to k_process_pairs (one wavefront each) start over
-__global__ void __launch_bounds__(OIC_WAVE) k_reopen_pairs(const PairRec *__restrict__ pairs, const uint32_t *__restrict__ list,
-                                                           int4 *__restrict__ nodes) {
-  const PairRec pr = pairs[list[blockIdx.x]];
+// pairs given back to k_process_pairs (one wavefront each) start over; their places become their numbers
+__global__ void __launch_bounds__(OIC_WAVE) k_reopen_pairs(const PairRec *__restrict__ pairs, const uint32_t *__restrict__ order,
+                                                           uint32_t *__restrict__ open, int4 *__restrict__ nodes) {
+  const uint32_t p = order[open[blockIdx.x]];
+  const PairRec pr = pairs[p];
+  __syncthreads();
+  if (lane_id() == 0) open[blockIdx.x] = p;
   for (int32_t i = lane_id(); i < pr.nnodes; i += OIC_WAVE) nodes[pr.hb + i].w = 0;
 }
