@@ -1161,8 +1161,7 @@ static int run_forward_passes_graph(oic_ctx *c, uint64_t np, uint64_t H, uint64_
   return OIC_OK;
 }
 
-// Process_Matches of the np pairs of PA.order in rounds (oic_rounds.h).  Pairs that the rounds' arrays could not hold
-// run one to a wavefront at the end.
+// Process_Matches of the np pairs of PA.order in rounds (oic_rounds.h).
 static int run_rounds(oic_ctx *c, const PairKernelArgs &PA, uint64_t np, uint64_t nnodes, double *ms) {
   RoundArgs A{};
   A.R = PA.R;
@@ -1174,8 +1173,8 @@ static int run_rounds(oic_ctx *c, const PairKernelArgs &PA, uint64_t np, uint64_
   A.out = PA.recs;
   A.pout = PA.pout;
   A.stats = PA.stats;
-  // every node is extended at most once; a mask is a bit per node of the task's pair
-  A.task_cap = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(nnodes, 1), kRoundTasks);
+  // a node is extended once as long as the stores hold; a mask is a bit per node of the task's pair
+  A.task_cap = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(nnodes, kAheadMax), kRoundTasks);
   A.word_cap = std::max<uint64_t>(kRoundWordsMin, std::min<uint64_t>(4 * nnodes, kRoundWords));
   ALLOC(c, c->r_state, np * sizeof(PairState));
   ALLOC(c, c->r_open, 2 * np * 4);
@@ -1196,10 +1195,10 @@ static int run_rounds(oic_ctx *c, const PairKernelArgs &PA, uint64_t np, uint64_
   A.n = (uint32_t)np;
   uint32_t *open[2] = {c->r_open.as<uint32_t>(), c->r_open.as<uint32_t>() + np};
   RoundCount rc{};
-  uint32_t left = 0;
+  bool asking = true;
   for (int round = 0;; round++) {
     A.open = open[round & 1];
-    A.ahead = (int32_t)std::max<uint32_t>(kAheadMin, std::min<uint32_t>(kAheadMax, fill * ewaves / std::max<uint32_t>(A.n, 1)));
+    A.ahead = asking ? (int32_t)std::max<uint32_t>(kAheadMin, std::min<uint32_t>(kAheadMax, fill * ewaves / std::max<uint32_t>(A.n, 1))) : 0;
     A.resume = round > 0 ? 1 : 0;
     hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, c->st, (uint32_t *)A.cnt, (uint64_t)4, 0u);
     hipLaunchKernelGGL(k_resolve_pairs, dim3(std::min<uint32_t>(A.n, (uint32_t)c->ncu * 32)), dim3(OIC_WAVE), 0, c->st, A);
@@ -1207,35 +1206,37 @@ static int run_rounds(oic_ctx *c, const PairKernelArgs &PA, uint64_t np, uint64_
     c->ctr.pp_launches++;
     HIPCHK(c, hipMemcpyAsync(&rc, A.cnt, sizeof rc, hipMemcpyDeviceToHost, c->st));
     HIPCHK(c, hipStreamSynchronize(c->st));
-    const uint32_t nt = std::min(rc.ntasks, A.task_cap);
     if (rc.nopen == 0) break;
-    if (nt == A.task0) { left = rc.nopen; break; }   // nothing more fits
-    A.task1 = nt;
-    const uint32_t waves = std::min<uint32_t>(ewaves, nt - A.task0);
-    int e = ensure_wave_scratch(c, waves, kFirstVals);
-    if (e) return e;
-    A.sc0 = scratch0(c);
-    A.row_stride = c->sc_rows;
-    A.val_stride = c->sc_stride;
-    A.delta_stride = c->sc_rows + 4;
-    hipLaunchKernelGGL(k_extend_nodes, dim3(waves), dim3(OIC_WAVE), 0, c->st, A);
-    HIPCHK(c, hipGetLastError());
-    c->ctr.spec_tasks += nt - A.task0;
-    A.task0 = nt;
     A.list = A.open;
     A.n = rc.nopen;
+    if (!asking) {   // every open pair has forgotten its results
+      hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, c->st, (uint32_t *)A.cnt, (uint64_t)(sizeof(RoundCount) / 4), 0u);
+      A.task0 = 0;
+      asking = true;
+      continue;
+    }
+    const uint32_t nt = (uint32_t)std::min<uint64_t>(rc.asked >> ROUND_WORD_BITS, A.task_cap);
+    A.task1 = nt;
+    const uint32_t waves = std::min<uint32_t>(ewaves, nt - A.task0);
+    if (waves) {
+      int e = ensure_wave_scratch(c, waves, kFirstVals);
+      if (e) return e;
+      A.sc0 = scratch0(c);
+      A.row_stride = c->sc_rows;
+      A.val_stride = c->sc_stride;
+      A.delta_stride = c->sc_rows + 4;
+      hipLaunchKernelGGL(k_extend_nodes, dim3(waves), dim3(OIC_WAVE), 0, c->st, A);
+      HIPCHK(c, hipGetLastError());
+    }
+    c->ctr.spec_tasks += nt - A.task0;
+    A.task0 = nt;
+    asking = rc.full == 0;
   }
   HIPCHK(c, hipEventRecord(c->ev1, c->st));
   HIPCHK(c, hipEventSynchronize(c->ev1));
   float f = 0;
   hipEventElapsedTime(&f, c->ev0, c->ev1);
   *ms += f;
-  if (left) {
-    hipLaunchKernelGGL(k_reopen_pairs, dim3(left), dim3(OIC_WAVE), 0, c->st, A.pairs, A.order, A.open, A.nodes);
-    PairKernelArgs B = PA;
-    B.order = A.open;
-    return run_pairs<WR_FIRST>(c, B, left, (uint32_t)c->ncu * 16, kFirstVals, ms);
-  }
   return OIC_OK;
 }
 

@@ -12,6 +12,13 @@
 //                    delta, and which of the pair's nodes lie on the alignment, as a bit mask.
 // The rounds end when no pair is open.  `ahead` is chosen per round so that the asked extensions fill the
 // machine a few times: many when few pairs are open (they would idle it), few when many are.
+//
+// Results and node masks wait in stores of a limited size (a mask has a bit per node of its pair, so the thousands
+// of extensions of one satellite pair need more than any store).  When an ask does not fit, the round's other
+// extensions run, one launch of k_resolve_pairs without asking uses what results there are, and the stores start
+// again empty; a pair forgets the results that it has not used by then, `ahead` of them at most.  (Rounds that went on
+// until the task slots were used up, and then one wavefront for the pair from its start: 1794 extensions of one tandem
+// pair 598 ms, 121 launches; so 130 ms, 37.)
 #pragma once
 
 #include "oic_batch.h"
@@ -36,11 +43,16 @@ struct PairState {
   PairOut po;
 };
 
-struct RoundCount {         // cleared before each round but for ntasks and nwords, which run on
-  uint32_t queue, nopen, equeue, pad;
-  uint32_t ntasks, full;    // extensions asked since the batch began; 1 when the arrays did not hold one
-  unsigned long long nwords;
+struct RoundCount {         // cleared before each round but for `asked`, which runs on until the stores are emptied
+  uint32_t queue, nopen, equeue;
+  uint32_t full;            // 1: an ask did not fit
+  unsigned long long asked; // extensions << ROUND_WORD_BITS | their mask words
 };
+// One atomic reserves both, so that the first ask of empty stores gets the first places of both and fits.  Asks that do
+// not fit count too: those of one launch are at most 64 extensions for each of 2^20 pairs and 64 words for each pair and
+// one for each match node (at most one a seed hit, which take over 100 bytes of the device's memory each), so neither
+// field overflows.
+#define ROUND_WORD_BITS 36
 
 struct RoundArgs {
   ReadsDev R;
@@ -54,13 +66,13 @@ struct RoundArgs {
   uint32_t n;                // afterwards go to open[]
   uint32_t *open;
   int resume;                // 0: the first round
-  int32_t ahead;             // extensions a pair may ask for at once
+  int32_t ahead;             // extensions a pair may ask for at once; 0: none, and results not used now are forgotten
   PairState *state;          // per place in order[]
   ExtNode *tasks;
   ExtRec *recs;
   uint64_t *masks;
   uint32_t task_cap, task0, task1;   // [task0, task1): k_extend_nodes' tasks of this round
-  uint64_t word_cap;
+  uint64_t word_cap;         // both at least 64; word_cap at least a mask of the pair with the most nodes
   RoundCount *cnt;
   OutRec *out;
   PairOut *pout;
@@ -168,6 +180,12 @@ __global__ void __launch_bounds__(OIC_WAVE) k_resolve_pairs(RoundArgs A) {
         if (pr.consistent) break;
         continue;
       }
+      if (kind != OUTC_EXT && A.ahead == 0) {
+        for (int32_t i = lane; i < nn; i += OIC_WAVE)
+          if (outcome_kind(outc[i]) == OUTC_EXT) outc[i] = 0;
+        suspended = true;
+        break;
+      }
       if (kind != OUTC_EXT) {
         // ask for this node's extension and for the next ones in picking order
         int32_t want = pr.consistent ? 1 : A.ahead;
@@ -185,16 +203,15 @@ __global__ void __launch_bounds__(OIC_WAVE) k_resolve_pairs(RoundArgs A) {
           const bool c = i < nn && !nodes[i].w && (outcome_kind(outc[i]) & 1) == 0;
           have += (int32_t)__builtin_popcountll(lanes(c));
         }
-        const int32_t cnt = have < want ? have : want;
         const uint32_t nw = (uint32_t)(nn + 63) / 64;
-        uint32_t slot = 0;
-        uint64_t word = 0;
-        if (lane == 0) {
-          slot = atomicAdd(&A.cnt->ntasks, (uint32_t)cnt);
-          word = atomicAdd(&A.cnt->nwords, (unsigned long long)cnt * nw);
-        }
-        slot = (uint32_t)uni((int32_t)slot);
-        word = (uint64_t)uni64((int64_t)word);
+        const uint64_t room = A.word_cap / nw;
+        if (room < (uint64_t)want) want = (int32_t)room;
+        const int32_t cnt = have < want ? have : want;
+        unsigned long long before = 0;
+        if (lane == 0) before = atomicAdd(&A.cnt->asked, ((unsigned long long)cnt << ROUND_WORD_BITS) + (unsigned long long)cnt * nw);
+        before = (unsigned long long)uni64((int64_t)before);
+        const uint32_t slot = (uint32_t)(before >> ROUND_WORD_BITS);
+        const uint64_t word = before & ((1ull << ROUND_WORD_BITS) - 1);
         const bool fits = (uint64_t)slot + cnt <= A.task_cap && word + (uint64_t)cnt * nw <= A.word_cap;
         if (!fits) {
           if (lane == 0) A.cnt->full = 1;
@@ -347,14 +364,4 @@ __global__ void __launch_bounds__(OIC_WAVE) __attribute__((amdgpu_waves_per_eu(4
     atomicAdd(&A.stats[STAT_SLOTS], (unsigned long long)slots);
     atomicAdd(&A.stats[STAT_DPCALLS], (unsigned long long)calls);
   }
-}
-
-// pairs given back to k_process_pairs (one wavefront each) start over; their places become their numbers
-__global__ void __launch_bounds__(OIC_WAVE) k_reopen_pairs(const PairRec *__restrict__ pairs, const uint32_t *__restrict__ order,
-                                                           uint32_t *__restrict__ open, int4 *__restrict__ nodes) {
-  const uint32_t p = order[open[blockIdx.x]];
-  const PairRec pr = pairs[p];
-  __syncthreads();
-  if (lane_id() == 0) open[blockIdx.x] = p;
-  for (int32_t i = lane_id(); i < pr.nnodes; i += OIC_WAVE) nodes[pr.hb + i].w = 0;
 }

@@ -1,5 +1,5 @@
-"""Process_Matches in rounds over more candidate pairs than take their rounds together (2^20): reads of one short
-tandem array, every pair a candidate with several match nodes, against the oracle."""
+"""Process_Matches in rounds (oic_rounds.h) beyond what its arrays hold at once, against the oracle: more candidate pairs
+than take their rounds together (2^20), and pairs whose extensions need several fillings of the mask store."""
 import numpy as np
 import pytest
 
@@ -7,6 +7,19 @@ from canu_amd import oic, readsim
 from oracle import oracle
 
 pytestmark = pytest.mark.gpu
+
+
+def tandem_pair(seed, unit, copies, div, err):
+    """Two reads of one tandem array whose copies differ by div, with err sequencing differences."""
+    rng = np.random.default_rng(seed)
+    base = rng.integers(0, 4, unit)
+    array = np.concatenate([np.where(rng.random(unit) < div, rng.integers(0, 4, unit), base) for _ in range(copies)])
+    seqs = []
+    for _ in range(2):
+        u = rng.random(len(array))
+        s = np.where(u < err / 2, (array + 1) % 4, array)[u < 1 - err / 2]
+        seqs.append("".join("ACGT"[x] for x in s[int(rng.integers(0, unit)):]))
+    return readsim.from_strings(seqs)
 
 
 def array_reads(n, seed):
@@ -23,15 +36,31 @@ def array_reads(n, seed):
     return readsim.from_strings(seqs)
 
 
-@pytest.mark.parametrize("partial", [False, True])
-def test_more_pairs_than_one_part(partial):
-    R = array_reads(1500, 81)
-    eng = oic.Engine(kmer=22, maxerate=0.045, minlength=40, threads=1, schedule=oic.SCHED_BATCHED, partial=partial)
+def run_both(R, minlength, partial):
+    eng = oic.Engine(kmer=22, maxerate=0.045, minlength=minlength, threads=1, schedule=oic.SCHED_BATCHED, partial=partial)
     eng.load_reads(R)
     res = eng.run()
-    ref = oracle.run(R, kmer=22, maxErate=0.045, minOlap=40, nThreads=1, ompThreads=16, partial=int(partial))
-    assert res.counters["pairs"] == ref["pairs"] > 1 << 20
+    ref = oracle.run(R, kmer=22, maxErate=0.045, minOlap=minlength, nThreads=1, ompThreads=16, partial=int(partial))
+    assert res.counters["pairs"] == ref["pairs"]
     a, b = oic.sort_records(res.records), oracle.sort_records(ref["records"])
-    assert len(a) == len(b) > 1 << 20 and all(np.array_equal(a[f], b[f]) for f in ("a_iid", "b_iid", "w0", "w1"))
+    assert len(a) == len(b) and all(np.array_equal(a[f], b[f]) for f in ("a_iid", "b_iid", "w0", "w1"))
     assert list(res.stats) == list(ref["stats"])
     assert res.counters["extensions"] == ref["extensions"] and res.counters["dp_cells"] == ref["cells_used"]
+    return res
+
+
+@pytest.mark.parametrize("partial", [False, True])
+def test_more_pairs_than_one_part(partial):
+    res = run_both(array_reads(1500, 81), 40, partial)
+    assert res.counters["pairs"] > 1 << 20 and len(res.records) > 1 << 20
+
+
+@pytest.mark.parametrize("copies", [60, 100])
+def test_store_is_emptied_when_full(copies):
+    """A pair asks for at most 64 extensions a round, each with a mask of nodes / 64 words, and the store holds 4 words
+    a node (65536 at least): a few hundred extensions.  Rounds that went on with a full store, until tasks without
+    work had used up a place for every node, were more than (nodes - that many) / 64."""
+    c = run_both(tandem_pair(75, 130, copies, 0.02, 0.012), 500, True).counters
+    words, store = (c["nodes"] + 63) // 64, max(1 << 16, 4 * c["nodes"])
+    assert c["pairs"] == 1 and c["extensions"] * words > 2 * store
+    assert c["pp_launches"] < c["nodes"] / 128 < (c["nodes"] - store / words) / 64
