@@ -102,7 +102,7 @@ struct oic_ctx {
   oic::Tables T;
   std::string err;
   hipStream_t st = nullptr;
-  hipStream_t st2 = nullptr;      // second stream: the 512-hit list level beside the 128-hit one
+  hipStream_t st2 = nullptr;      // second stream: the list levels of pairs with few hits beside the others
   hipEvent_t evl[2] = {};
   int ncu = 0;
 
@@ -1362,16 +1362,17 @@ static int search_batch(oic_ctx *c, uint32_t s0, uint32_t ns, const std::vector<
     const uint64_t ntile = (H + LW_SPLIT - 1) / LW_SPLIT;
     const uint64_t nlong = H / LW_LONG + 1;              // long pairs at most
     ALLOC(c, c->l_done, np);
-    ALLOC(c, c->l_big, (2 * np + ntile + 4 * nlong) * 4);       // big, up (pairs and parts), long pairs and their parts
+    ALLOC(c, c->l_big, (3 * np + ntile + 4 * nlong) * 4);       // big, up (pairs and parts), long pairs and their parts, crowded
     ALLOC(c, c->l_split, ntile * 8);
     ALLOC(c, c->l_items, (ntile + nlong) * sizeof(ListItem));   // at most one part begins in a tile, and one at a pair's start
     ALLOC(c, c->l_cnt, 64);
     HIPCHK(c, hipMemsetAsync(c->l_cnt.p, 0, 64, c->st));
     // cnt: [0] big pairs, [1] their queue, [2] handed back, [4..5] nodes, [6] queue of few hits, [7] handed back
     // there, [8] long pairs, [9] parts, [10] pairs and parts with over 128 hits at an offset, [11] their queue, [12]
-    // predictions that are not finite
+    // predictions that are not finite, [13] pairs of few hits with over 64 at an offset, [14] their queue
     uint32_t *cnt = c->l_cnt.as<uint32_t>();
     uint32_t *big = c->l_big.as<uint32_t>(), *up = big + np, *lng = up + np + ntile + nlong, *lfirst = lng + nlong, *lcount = lfirst + nlong;
+    uint32_t *crowded = lcount + nlong;
     hipLaunchKernelGGL(k_big_select, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, c->st, c->p_pairs.as<PairRec>(), np,
                        (uint64_t)c->tune.list_wave_min_hits, c->l_done.as<uint8_t>(), big, cnt, lng, cnt + 8);
     hipLaunchKernelGGL(k_list_splits, dim3((unsigned)((ntile + 3) / 4)), dim3(256), 0, c->st, c->p_pairs.as<PairRec>(), c->s_flag.as<uint32_t>(),
@@ -1392,16 +1393,25 @@ static int search_batch(oic_ctx *c, uint32_t s0, uint32_t ns, const std::vector<
     BA.nodes = c->p_nodes.as<int4>();
     BA.K = K;
     const uint64_t ncu = (uint64_t)std::max(c->ncu, 1);
-    // Second stream, beside the others: the pairs with fewer hits, at 64 hits per offset.
+    // Second stream, beside the others: the pairs with fewer hits, at 64 hits per offset, and what is more crowded at 512.
     BigListArgs BS = BA;
     BS.big = nullptr;
     BS.nitems = nullptr;
     BS.next = cnt + 6;
-    BS.handed_back = cnt + 7;
+    BS.up = crowded;
+    BS.nup = cnt + 13;
+    BigListArgs BC = BS;
+    BC.big = crowded;
+    BC.nbig = cnt + 13;
+    BC.next = cnt + 14;
+    BC.handed_back = cnt + 7;
+    BC.up = nullptr;
+    BC.nup = nullptr;
     HIPCHK(c, hipEventRecord(c->evl[0], c->st));
     HIPCHK(c, hipStreamWaitEvent(c->st2, c->evl[0], 0));
     hipLaunchKernelGGL(k_build_lists_wave<LW_CAP_SMALL>, dim3((unsigned)std::min<uint64_t>((np + LW_TAKE - 1) / LW_TAKE, 32 * ncu)), dim3(64),
                        0, c->st2, BS);
+    hipLaunchKernelGGL(k_build_lists_wave<LW_CAP>, dim3((unsigned)std::min<uint64_t>(np, 4 * ncu)), dim3(64), 0, c->st2, BC);
     HIPCHK(c, hipEventRecord(c->evl[1], c->st2));
     uint32_t nl = 0;
     HIPCHK(c, hipMemcpyAsync(&nl, cnt + 8, 4, hipMemcpyDeviceToHost, c->st));
@@ -1430,7 +1440,7 @@ static int search_batch(oic_ctx *c, uint32_t s0, uint32_t ns, const std::vector<
       hipLaunchKernelGGL(k_list_copy, dim3((nit + 3) / 4), dim3(256), 0, c->st, BA, nit);
     }
     HIPCHK(c, hipStreamWaitEvent(c->st, c->evl[1], 0));
-    // pairs a wavefront handed back (an offset of more than 512 hits, or 64 at the level of few hits)
+    // pairs a wavefront handed back (an offset of more than 512 hits)
     hipLaunchKernelGGL(k_build_lists, dim3((unsigned)((np + 127) / 128)), dim3(128), 0, c->st, c->p_pairs.as<PairRec>(), np, hv,
                        c->p_tmp.as<int4>(), c->p_nodes.as<int4>(), K, LS, c->l_done.as<uint8_t>(), (uint8_t)2, BA.nnodes_total);
   }
@@ -1445,8 +1455,8 @@ static int search_batch(oic_ctx *c, uint32_t s0, uint32_t ns, const std::vector<
     HIPCHK(c, hipMemcpyAsync(lc, c->l_cnt.p, 64, hipMemcpyDeviceToHost, c->st));
     HIPCHK(c, hipStreamSynchronize(c->st));
     c->ctr.list_wave_pairs += lc[0] + lc[8];
-    c->ctr.list_handed_back += lc[2];
-    c->ctr.list_second_level += lc[10];
+    c->ctr.list_handed_back += lc[2] + lc[7];
+    c->ctr.list_second_level += lc[10] + lc[13];
     memcpy(&batch_nodes, lc + 4, 8);
     c->ctr.nodes += batch_nodes;
     c->batch_pred = predicted && lc[12] == 0;

@@ -131,9 +131,10 @@ typedef struct oic_counters {
   uint64_t fwd_bases;
   uint64_t graphs_launched;    /* forward-pass hipGraphs launched */
   uint64_t list_wave_pairs;    /* pairs whose match list the 128-hit wavefront level built */
-  uint64_t list_handed_back;   /* of those, pairs with an offset of more hits than the wavefront holds */
-  uint64_t list_second_level;  /* of those, pairs taken on by the 512-hit wavefront level (an offset
-                                  with more than 128 hits) */
+  uint64_t list_handed_back;   /* pairs (parts of long ones) with an offset of more than 512 hits, whose pair's
+                                  list one thread built */
+  uint64_t list_second_level;  /* pairs (parts of long ones) taken on by the 512-hit wavefront level: an offset
+                                  with more than 128 hits, or 64 at the level of pairs with few hits */
   double   ms_index, ms_gather, ms_lists, ms_extend, ms_total;
   double   ms_dp_kernel;       /* device time of all DP kernels (HIP events) */
   double   ms_fwd_kernel;      /* of which the packed forward-DP kernels */
