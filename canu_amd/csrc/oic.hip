@@ -2054,14 +2054,16 @@ constexpr size_t kQueueOff = 0;
 constexpr size_t kTaskOff = 256;
 constexpr size_t kResOff = kTaskOff + up256((size_t)kMaxTasks * sizeof(oic_dp_task));
 constexpr size_t kDeltaOff = kResOff + up256((size_t)kMaxTasks * sizeof(oic_dp_result));
-constexpr size_t kRetryOff = kDeltaOff + up256((size_t)kMaxDeltaInts * 4);
-constexpr size_t kRowmOff = kRetryOff + up256((size_t)kMaxTasks * 4);
+constexpr size_t kRowmOff = kDeltaOff + up256((size_t)kMaxDeltaInts * 4);
 constexpr size_t kRowValOff = kRowmOff + up256((size_t)kWaves * kRows * 4);
 constexpr int64_t kValStride = kVals + WR_VAL_SLACK(kRows);
 constexpr size_t kDbufOff = kRowValOff + up256((size_t)kWaves * kValStride * 4);
 constexpr size_t kLdOff = kDbufOff + up256((size_t)kWaves * (kRows + 4) * 4);
 constexpr size_t kRdOff = kLdOff + up256((size_t)kWaves * (kRows + 4) * 4);
 constexpr size_t kBytes = kRdOff + up256((size_t)kWaves * (kRows + 4) * 4);   // about 42 MB
+// One level (oic_wdp.h) runs every DP that the row store holds: a row keeps at most two cells more than the row before,
+// so a band wider than the first level's has kept (wr_band / 2)^2 cells by then.
+static_assert((int64_t)(wr_band<WR_FIRST>() / 2) * (wr_band<WR_FIRST>() / 2) > kVals, "a band of the second level may fit the store");
 }  // namespace na
 
 __device__ __align__(256) uint8_t scratch[na::kBytes];
@@ -2112,7 +2114,7 @@ extern "C" int oic_prefix_dp_batch_noalloc(oic_ctx *c, const oic_dp_task *tasks,
   int32_t *dd = (int32_t *)(base + na::kDeltaOff);
   uint32_t *queue = (uint32_t *)(base + na::kQueueOff);
   HIPCHK(c, hipMemcpyAsync(dt, tasks, (size_t)n * sizeof(oic_dp_task), hipMemcpyHostToDevice, c->st));
-  hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, c->st, queue, (uint64_t)kBatchCounters, 0u);
+  hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, c->st, queue, (uint64_t)1, 0u);
   if (delta) {
     const uint64_t nd = (uint64_t)n * stride;
     hipLaunchKernelGGL(k_fill_u32, dim3((unsigned)((nd + 255) / 256)), dim3(256), 0, c->st, (uint32_t *)dd, nd, 0u);
@@ -2137,21 +2139,7 @@ extern "C" int oic_prefix_dp_batch_noalloc(oic_ctx *c, const oic_dp_task *tasks,
   A.val_stride = na::kValStride;
   A.delta_stride_sc = na::kRows + 4;
   const uint32_t waves = std::min<uint32_t>(n, na::kWaves);
-  int32_t max_limit = 0;
-  for (uint32_t i = 0; i < n; i++) max_limit = std::max(max_limit, tasks[i].error_limit);
-  const bool two = 2 * max_limit + 1 > wr_band<WR_FIRST>();   // some band may outgrow the first level
-  if (two) {
-    A.retry = (uint32_t *)(base + na::kRetryOff);
-    A.nretry = queue + 1;
-  }
   hipLaunchKernelGGL(k_dp_batch<WR_FIRST>, dim3(waves), dim3(OIC_WAVE), 0, c->st, A);
-  if (two) {
-    A.todo = A.retry;
-    A.ntodo = queue + 1;
-    A.retry = nullptr;
-    A.queue = queue + 2;
-    hipLaunchKernelGGL(k_dp_batch<WR_WIDE>, dim3(waves), dim3(OIC_WAVE), 0, c->st, A);
-  }
   HIPCHK(c, hipGetLastError());
   HIPCHK(c, hipMemcpyAsync(res, dr, (size_t)n * sizeof(oic_dp_result), hipMemcpyDeviceToHost, c->st));
   if (delta) HIPCHK(c, hipMemcpyAsync(delta, dd, (size_t)n * stride * 4, hipMemcpyDeviceToHost, c->st));
