@@ -906,6 +906,7 @@ static int run_fwd_binned(oic_ctx *c, FwdArgs FA, uint64_t n, double *ms) {
   if (rc) return rc;
   HIPCHK(c, hipMemcpy(&nov, FA.novf, 4, hipMemcpyDeviceToHost));
   if (nov == 0) return OIC_OK;
+  c->ctr.overflow_retries += nov;
   FA.tasks = FA.ovf;
   FA.ovf = nullptr;
   return c->tune.fwd_counters ? run_fwd<64, WR_WIDE, true>(c, FA, nov, ms) : run_fwd<64, WR_WIDE, false>(c, FA, nov, ms);
@@ -1025,6 +1026,8 @@ static int run_forward_passes_graph(oic_ctx *c, uint64_t np, uint64_t H, uint64_
   unsigned long long *stats = c->b_stats.as<unsigned long long>();
   const unsigned g = (unsigned)((np + 255) / 256);
   const bool graph = c->tune.fwd_graph != 0;
+  // the counters are the packed kernel's, and a form other than the flat rows is one that was asked for
+  const uint64_t few = c->tune.fwd_counters || c->tune.fwd_loop != 2 ? 0 : kFewTasks * (uint64_t)c->ncu;
   hipEvent_t *ev = graph ? nullptr : c->evf;
   if (graph) HIPCHK(c, hipStreamBeginCapture(c->st, hipStreamCaptureModeThreadLocal));
   // everything up to the end of the capture; an error inside it still ends the capture below, so
@@ -1046,8 +1049,6 @@ static int run_forward_passes_graph(oic_ctx *c, uint64_t np, uint64_t H, uint64_
     FA.nodes = c->p_nodes.as<int4>();
     FA.outc = c->b_outc.as<uint64_t>();
     FwdTask *ovf = c->b_ovf.as<FwdTask>();
-    // the counters are the packed kernel's, and a form other than the flat rows is one that was asked for
-    const uint64_t few = c->tune.fwd_counters || c->tune.fwd_loop != 2 ? 0 : kFewTasks * (uint64_t)c->ncu;
     // one pass: launch slot k (0 probe, 1 spec) uses queues/stats 3k..3k+2 and overflow counts 8+2k, 9+2k
     auto pass = [&](int k, const FwdTask *tasks, uint64_t n, const uint32_t *n_dev, uint64_t cap, FwdTask *ov1, FwdTask *ov2) -> int {
       FA.tasks = tasks; FA.ntasks = n; FA.ntasks_dev = n_dev;
@@ -1145,14 +1146,14 @@ static int run_forward_passes_graph(oic_ctx *c, uint64_t np, uint64_t H, uint64_
     c->ctr.spec_wave_slide_iters += x[6];
     c->ctr.spec_wave_chunks += x[7];
   }
-  for (int i : {0, 3}) {   // the packed narrow-band launches
-    if (i == 3 && nt == 0) continue;
+  for (int i : {0, 3}) {   // the packed narrow-band launches, but for those that left their few tasks to k_fwd_wave
+    if ((i == 0 ? np : nt) <= few) continue;
     c->ctr.fwd_launches++;
     c->ctr.fwd_cells += st[8 * i];
     c->ctr.fwd_bases += st[8 * i + 4];
     c->ctr.ms_fwd_narrow += f[i];
   }
-  c->ctr.overflow_retries += cn[8] + cn[10];
+  c->ctr.overflow_retries += cn[8] + cn[9] + cn[10] + cn[11];
   c->ctr.spec_tasks += np + nt;
   double ms = 0;
   for (float x : f) ms += x;
@@ -1228,7 +1229,6 @@ static int run_rounds(oic_ctx *c, const PairKernelArgs &PA, uint64_t np, uint64_
       hipLaunchKernelGGL(k_extend_nodes, dim3(waves), dim3(OIC_WAVE), 0, c->st, A);
       HIPCHK(c, hipGetLastError());
     }
-    c->ctr.spec_tasks += nt - A.task0;
     A.task0 = nt;
     asking = rc.full == 0;
   }
@@ -1565,6 +1565,7 @@ static int search_batch(oic_ctx *c, uint32_t s0, uint32_t ns, const std::vector<
   c->ctr.pp_cells += stats[STAT_PPCELLS];
   c->ctr.pp_bases += stats[STAT_BASES];
   if (in_rounds) {
+    c->ctr.spec_tasks += stats[STAT_AHEAD];
     c->ctr.spec_cells += stats[STAT_PPCELLS];
     c->ctr.spec_bases += stats[STAT_BASES];
   }

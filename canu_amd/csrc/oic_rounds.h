@@ -315,7 +315,7 @@ __global__ void __launch_bounds__(OIC_WAVE) __attribute__((amdgpu_waves_per_eu(4
   sc.ldelta += (int64_t)blockIdx.x * A.delta_stride;
   sc.rdelta += (int64_t)blockIdx.x * A.delta_stride;
   uint64_t cells_acc = 0, slots = 0, bases = 0;
-  uint32_t calls = 0;
+  uint32_t calls = 0, ran = 0;
   while (true) {
     uint32_t f = 0;
     if (lane == 0) f = atomicAdd(&A.cnt->equeue, 1u);
@@ -339,6 +339,7 @@ __global__ void __launch_bounds__(OIC_WAVE) __attribute__((amdgpu_waves_per_eu(4
       A.recs[ti] = r;
     }
     cells_acc += cells;
+    ran++;
     if (x.overflow || pr.consistent || !(x.kind == 3 || C.partial)) continue;
     // the pair's nodes on this alignment (:476-490)
     const int32_t nn = uni(pr.nnodes);
@@ -363,5 +364,6 @@ __global__ void __launch_bounds__(OIC_WAVE) __attribute__((amdgpu_waves_per_eu(4
     atomicAdd(&A.stats[STAT_PPCELLS], (unsigned long long)cells_acc);
     atomicAdd(&A.stats[STAT_SLOTS], (unsigned long long)slots);
     atomicAdd(&A.stats[STAT_DPCALLS], (unsigned long long)calls);
+    atomicAdd(&A.stats[STAT_AHEAD], (unsigned long long)ran);
   }
 }

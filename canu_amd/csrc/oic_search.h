@@ -1657,6 +1657,7 @@ struct PairOut {
 #define STAT_DPCALLS 11
 #define STAT_BASES   12
 #define STAT_PPCELLS 13   // cells of the DPs this kernel runs itself (full extensions)
+#define STAT_AHEAD   14   // extensions that k_extend_nodes ran
 #define STAT_NSTATS  16
 
 // A node's cached outcome in one 64-bit word, so a finished task makes one store: the kind in bits

@@ -111,22 +111,24 @@ typedef struct oic_counters {
   uint64_t pairs;              /* candidate (S, orientation, T) pairs */
   uint64_t nodes;              /* match nodes */
   uint64_t extensions;         /* Extend_Alignment calls */
-  uint64_t dp_calls;           /* forward / reverse DP runs executed */
-  uint64_t dp_cells;           /* (e, d) cell updates executed, row-0 slide counted as one */
-  uint64_t dp_lane_slots;      /* lane-cells issued (cells plus idle lanes of partial chunks) */
-  uint64_t dp_bases;           /* bases compared in slides, plus one terminating compare per cell */
-  uint64_t overflow_retries;   /* DP tasks re-run with a wider band tile */
+  uint64_t dp_calls;           /* forward / reverse DP runs Process_Matches executed itself, under the batched and
+                                  learned schedules also those of extensions run ahead whose result it did not use */
+  uint64_t dp_cells;           /* (e, d) cell updates of the extensions it used, row-0 slide counted as one */
+  uint64_t dp_lane_slots;      /* lane-cells issued for dp_calls (cells plus idle lanes of partial chunks) */
+  uint64_t dp_bases;           /* bases compared in their slides, plus one terminating compare per cell */
+  uint64_t overflow_retries;   /* DP tasks and pairs re-run with a wider band tile */
   uint64_t spec_tasks;         /* forward DPs and whole extensions run ahead of their pair's Process_Matches
                                   (batched and learned schedules) */
-  uint64_t spec_cells;         /* cells of those runs, used or not */
+  uint64_t spec_cells;         /* cells of those runs, used or not: the forward passes' and pp_cells */
   uint64_t spec_rows;          /* DP rows (e >= 1) of those runs (with tuning.fwd_counters) */
   uint64_t spec_lane_slots;    /* lane-cells issued by those runs (with tuning.fwd_counters) */
   uint64_t spec_wave_rows;     /* row iterations wavefronts executed for them (a wavefront waits for
                                   its slowest packed DP) (with tuning.fwd_counters) */
-  uint64_t spec_bases;         /* bases compared by those runs */
+  uint64_t spec_bases;         /* bases compared by those runs: the forward passes' and pp_bases */
   uint64_t spec_slide_iters;   /* 16-base window compares of their slides, per lane (with tuning.fwd_counters) */
   uint64_t spec_wave_slide_iters; /* slide iterations wavefronts executed (with tuning.fwd_counters) */
-  uint64_t fwd_launches;       /* launches of the packed narrow-band forward kernel */
+  uint64_t fwd_launches;       /* launches of the packed narrow-band forward kernel, without those that left their
+                                  few tasks to the one-per-wavefront kernel */
   uint64_t fwd_cells;          /* cells and bases of those launches */
   uint64_t fwd_bases;
   uint64_t graphs_launched;    /* forward-pass hipGraphs launched */
@@ -144,7 +146,7 @@ typedef struct oic_counters {
   double   ms_fwd_graph;       /* forward-pass graphs, HIP events around their launches */
   double   ms_pp_kernel;       /* Process_Matches (k_process_pairs, or the rounds of k_resolve_pairs and
                                   k_extend_nodes), HIP events around its launches */
-  uint64_t pp_cells;           /* DP cells it computes itself (full extensions with row storage) */
+  uint64_t pp_cells;           /* DP cells it computes itself (full extensions with row storage), used or not */
   uint64_t pp_bases;           /* bases it compares in their slides, plus one per cell */
   uint64_t learned_pairs;      /* pairs the learned cost model ordered (OIC_SCHED_LEARNED with a model) */
   uint64_t pp_launches;        /* launches of k_process_pairs or k_resolve_pairs */
