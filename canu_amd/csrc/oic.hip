@@ -1362,17 +1362,15 @@ static int search_batch(oic_ctx *c, uint32_t s0, uint32_t ns, const std::vector<
     const uint64_t ntile = (H + LW_SPLIT - 1) / LW_SPLIT;
     const uint64_t nlong = H / LW_LONG + 1;              // long pairs at most
     ALLOC(c, c->l_done, np);
-    ALLOC(c, c->l_big, (3 * np + ntile + 4 * nlong) * 4);       // big, up (pairs and parts), long pairs and their parts, crowded
+    ALLOC(c, c->l_big, (2 * np + ntile + 4 * nlong) * 4);       // big, up (pairs and parts), long pairs and their parts
     ALLOC(c, c->l_split, ntile * 8);
     ALLOC(c, c->l_items, (ntile + nlong) * sizeof(ListItem));   // at most one part begins in a tile, and one at a pair's start
     ALLOC(c, c->l_cnt, 64);
     HIPCHK(c, hipMemsetAsync(c->l_cnt.p, 0, 64, c->st));
-    // cnt: [0] big pairs, [1] their queue, [2] handed back, [4..5] nodes, [6] queue of few hits, [7] handed back
-    // there, [8] long pairs, [9] parts, [10] pairs and parts with over 128 hits at an offset, [11] their queue, [12]
-    // predictions that are not finite, [13] pairs of few hits with over 64 at an offset, [14] their queue
+    // cnt: [0] big pairs, [1] their queue, [2] handed back, [4..5] nodes, [6] queue of few hits, [8] long pairs, [9]
+    // parts, [10] pairs and parts too crowded for their first level, [11] their queue, [12] predictions that are not finite
     uint32_t *cnt = c->l_cnt.as<uint32_t>();
     uint32_t *big = c->l_big.as<uint32_t>(), *up = big + np, *lng = up + np + ntile + nlong, *lfirst = lng + nlong, *lcount = lfirst + nlong;
-    uint32_t *crowded = lcount + nlong;
     hipLaunchKernelGGL(k_big_select, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, c->st, c->p_pairs.as<PairRec>(), np,
                        (uint64_t)c->tune.list_wave_min_hits, c->l_done.as<uint8_t>(), big, cnt, lng, cnt + 8);
     hipLaunchKernelGGL(k_list_splits, dim3((unsigned)((ntile + 3) / 4)), dim3(256), 0, c->st, c->p_pairs.as<PairRec>(), c->s_flag.as<uint32_t>(),
@@ -1393,25 +1391,19 @@ static int search_batch(oic_ctx *c, uint32_t s0, uint32_t ns, const std::vector<
     BA.nodes = c->p_nodes.as<int4>();
     BA.K = K;
     const uint64_t ncu = (uint64_t)std::max(c->ncu, 1);
-    // Second stream, beside the others: the pairs with fewer hits, at 64 hits per offset, and what is more crowded at 512.
+    // what the two first levels (up to 128 hits per offset, 64 for pairs with few hits) find more crowded runs at 512
+    // hits after them
+    BA.up = up;
+    BA.nup = cnt + 10;
+    // Second stream, beside the others: the pairs with fewer hits.
     BigListArgs BS = BA;
     BS.big = nullptr;
     BS.nitems = nullptr;
     BS.next = cnt + 6;
-    BS.up = crowded;
-    BS.nup = cnt + 13;
-    BigListArgs BC = BS;
-    BC.big = crowded;
-    BC.nbig = cnt + 13;
-    BC.next = cnt + 14;
-    BC.handed_back = cnt + 7;
-    BC.up = nullptr;
-    BC.nup = nullptr;
     HIPCHK(c, hipEventRecord(c->evl[0], c->st));
     HIPCHK(c, hipStreamWaitEvent(c->st2, c->evl[0], 0));
     hipLaunchKernelGGL(k_build_lists_wave<LW_CAP_SMALL>, dim3((unsigned)std::min<uint64_t>((np + LW_TAKE - 1) / LW_TAKE, 32 * ncu)), dim3(64),
                        0, c->st2, BS);
-    hipLaunchKernelGGL(k_build_lists_wave<LW_CAP>, dim3((unsigned)std::min<uint64_t>(np, 4 * ncu)), dim3(64), 0, c->st2, BC);
     HIPCHK(c, hipEventRecord(c->evl[1], c->st2));
     uint32_t nl = 0;
     HIPCHK(c, hipMemcpyAsync(&nl, cnt + 8, 4, hipMemcpyDeviceToHost, c->st));
@@ -1422,9 +1414,6 @@ static int search_batch(oic_ctx *c, uint32_t s0, uint32_t ns, const std::vector<
                          lcount);
       HIPCHK(c, hipMemcpyAsync(&nit, cnt + 9, 4, hipMemcpyDeviceToHost, c->st));
     }
-    // first level: up to 128 hits per offset; what it finds more crowded runs at 512 hits after it
-    BA.up = up;
-    BA.nup = cnt + 10;
     hipLaunchKernelGGL(k_build_lists_wave<LW_CAP_FIRST>, dim3((unsigned)std::min<uint64_t>(np + ntile, 16 * ncu)), dim3(64), 0, c->st, BA);
     BigListArgs B3 = BA;
     B3.big = up;
@@ -1433,13 +1422,13 @@ static int search_batch(oic_ctx *c, uint32_t s0, uint32_t ns, const std::vector<
     B3.next = cnt + 11;
     B3.up = nullptr;
     B3.nup = nullptr;
+    HIPCHK(c, hipStreamWaitEvent(c->st, c->evl[1], 0));
     hipLaunchKernelGGL(k_build_lists_wave<LW_CAP>, dim3((unsigned)std::min<uint64_t>(np + ntile, 4 * ncu)), dim3(64), 0, c->st, B3);
     if (nl) {
       HIPCHK(c, hipStreamSynchronize(c->st));   // nit
       hipLaunchKernelGGL(k_list_join, dim3(nl), dim3(OIC_WAVE), 0, c->st, BA, lng, lfirst, lcount);
       hipLaunchKernelGGL(k_list_copy, dim3((nit + 3) / 4), dim3(256), 0, c->st, BA, nit);
     }
-    HIPCHK(c, hipStreamWaitEvent(c->st, c->evl[1], 0));
     // pairs a wavefront handed back (an offset of more than 512 hits)
     hipLaunchKernelGGL(k_build_lists, dim3((unsigned)((np + 127) / 128)), dim3(128), 0, c->st, c->p_pairs.as<PairRec>(), np, hv,
                        c->p_tmp.as<int4>(), c->p_nodes.as<int4>(), K, LS, c->l_done.as<uint8_t>(), (uint8_t)2, BA.nnodes_total);
@@ -1455,8 +1444,8 @@ static int search_batch(oic_ctx *c, uint32_t s0, uint32_t ns, const std::vector<
     HIPCHK(c, hipMemcpyAsync(lc, c->l_cnt.p, 64, hipMemcpyDeviceToHost, c->st));
     HIPCHK(c, hipStreamSynchronize(c->st));
     c->ctr.list_wave_pairs += lc[0] + lc[8];
-    c->ctr.list_handed_back += lc[2] + lc[7];
-    c->ctr.list_second_level += lc[10] + lc[13];
+    c->ctr.list_handed_back += lc[2];
+    c->ctr.list_second_level += lc[10];
     memcpy(&batch_nodes, lc + 4, 8);
     c->ctr.nodes += batch_nodes;
     c->batch_pred = predicted && lc[12] == 0;

@@ -595,7 +595,7 @@ __global__ void k_build_lists(PairRec *__restrict__ pairs, uint64_t np, const ui
 // (the 512-hit kernel), or, from the last level, back to the one-thread builder (done[p] = 2).
 #define LW_CAP 512        // hits per offset of the last wavefront level
 #define LW_CAP_FIRST 128  // of the first: a quarter of the LDS, four times the wavefronts per CU
-// Of the level for pairs with few hits in all; more crowded ones go on to the last level beside it (from here straight
+// Of the level for pairs with few hits in all; more crowded ones go on to the last level (from here straight
 // to one thread each, 2 us a hit after all other lists: 56 850 pairs, 12 000 of them with 100 or 500 hits at an offset,
 // 6.8 and 9.0 ms; so 1.6 ms).
 #define LW_CAP_SMALL 64
