@@ -76,10 +76,14 @@ constexpr int64_t kFirstVals = (int64_t)1 << 19;        // band cells a wavefron
 // device bytes a search pass holds per seed hit (hits, sort, lists, nodes, outcomes).  Its candidate pairs, with some 300
 // bytes each, and Process_Matches' scratch (kRound*, and a row store per wavefront) come out of the rest.
 constexpr uint64_t kPassBytesPerHit = 140;
-// forward DPs of one pass up to which each takes a wavefront of its own, per CU: as measured (256 CUs), 17 ns a task
-// there, against 6 ns and 2 to 3 ms in the packed kernel whatever their number.  Whole calls at 64, 256 and 512 per CU:
-// 1490 pairs (126 thousand tasks) 26.1, 26.3, 23.3 ms, 82 thousand pairs 55.0, 54.9, 52.4, 90 thousand 37.0, 37.0,
-// 35.6, 113 thousand 27.2, 27.1, 26.6 ms; 37 low-error reads 11.0 -> 8.8 and 755 reads 45 -> 40 ms at each.
+// Forward DPs of one pass up to which each takes a wavefront of its own, per CU (131072 on 256 CUs): there a task costs
+// 8 to 16 ns and a pass nearly nothing, in the packed kernel 1 to 6 ns and 1.2 to 1.6 ms whatever their number.
+// The two passes of a search of 42, 90, 131, 199 and 301 thousand tasks (4 % error, 1120 cells a task) take 1.0, 1.8,
+// 2.4, 3.5 and 5.1 ms one to a wavefront and 1.6, 1.8, 2.1, 2.7 and 3.2 ms packed: equal at 93 thousand; with repeats
+// (700 cells) they are equal at 125 thousand, on compressed reads (80 cells) at 85, and on low-error reads (12 thousand
+// cells: true overlaps, which outgrow the packed tile and start again) 40, 96 and 160 thousand tasks take 0.9, 1.1 and 1.3
+// against 2.0, 2.0 and 2.4 ms.  Between 85 and 131 thousand the limit costs the first three up to 0.3 ms a pass of few and
+// spares the last 1.0; a count of tasks cannot tell them apart.
 constexpr uint64_t kFewTasks = 512;
 // Rounds of Process_Matches (oic_rounds.h).  They hold a state of 208 bytes per pair, so more pairs than kRoundPairs
 // take their rounds one part after another (in processing order: 78 thousand pairs are a whole pass of the repeat-rich

@@ -94,8 +94,9 @@ __device__ __forceinline__ float row_sum_f(float v) {
 // Bound by latency at the batches in use: 128 workgroups at 4096 samples, each one chunk: 4 barriers and about
 // 110 matrix instructions of 32 cycles a wavefront.  The form before it (one wavefront per 64 samples, lane =
 // sample, then lane = unit, on the vector unit with one operand of each product from LDS, 256 VGPRs, an atomic per
-// wavefront and parameter) took 257 us a batch; training on 60 000 samples for 2 epochs took 8.9 ms as a whole, now
-// 1.2 ms, most of it the host's shuffles and copies.
+// wavefront and parameter) took 257 us a batch, this one 10; training on 60 000 samples for 2 epochs took 8.9 ms as a
+// whole, now 1.2 ms: about half are the 30 dependent steps (this kernel, 10 us, k_mlp_adam, 6, and 2 us gaps), the rest
+// the host's sums and shuffles, buffers and copies.
 #define MLP_TILES 2                       // of 16 samples
 #define MLP_CHUNK (16 * MLP_TILES)
 #define MLP_LD    (MLP_H + 4)

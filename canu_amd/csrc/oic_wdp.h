@@ -31,9 +31,9 @@
 // One wavefront per workgroup: its LDS operations complete in order, so fences only keep the compiler's order.
 // wave_rows is not inlined: the kernels' other live values would otherwise be spilled around its loops.
 // Bound by the issue of a wavefront's instructions, one wavefront's chain when calls are few.  Measured as whole
-// calls, first form -> wide rows only -> both: 12 DPs of 600 bases 150 -> 95 -> 75 us, 400 of 12 kbp 1.43 -> 0.97
-// -> 0.90 ms, 600 extensions of 8 kbp 4.7 -> 2.7 -> 1.9 ms, a search with one candidate pair per wavefront (951
-// thousand extensions of 4 %-error reads) 101 -> 51 -> 37 ms.
+// calls, first form -> wide rows only -> both: 12 DPs of 600 bases 150 -> 95 -> 89 us, 400 of 12 kbp 1.32 -> 0.97
+// -> 0.90 ms, 600 extensions of 8 kbp 4.7 -> 2.7 -> 2.5 ms, a search with one candidate pair per wavefront (951
+// thousand extensions of 4 %-error reads) 101 -> 51 ms and, after other steps, 44 -> 37 ms.
 #pragma once
 
 #include "oic_dp.h"
