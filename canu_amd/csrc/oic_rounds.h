@@ -190,11 +190,15 @@ __global__ void __launch_bounds__(OIC_WAVE) k_resolve_pairs(RoundArgs A) {
         // ask for this node's extension and for the next ones in picking order
         int32_t want = pr.consistent ? 1 : A.ahead;
         if (A.pred && want > 1) {
-          // no more than the cost model expects: its cells still to come over those of an extension so far
+          // No more than the cost model expects, its cells still to come over those of an extension so far, but half of
+          // what the pair may ask for at the least, and no limit once it has used up what the model expected.  (Down to
+          // one, and one for each round from there on: 900 low-error reads 43.7 ms in 42 rounds, 2500 compressed reads
+          // 1605 ms in 827; so 23.1 ms in 8 and 1323 in 178, as without a model, with 4 % fewer extensions of the first.)
           const float left = expm1f(A.pred[2 * (uint64_t)p]) - (float)po.cells;
           const float each = po.n_ext > 0 ? (float)po.cells / (float)po.n_ext : (float)outcome_cells(bo);
           const float k = each > 0.f ? left / each : 1.f;
-          want = k < (float)want ? (k > 1.f ? (int32_t)k : 1) : want;
+          const int32_t least = want / 2;
+          if (left > 0.f && k < (float)want) want = k > (float)least ? (int32_t)k : least;
         }
         want = uni(want);
         int32_t have = 0;

@@ -1,5 +1,6 @@
 """Process_Matches in rounds (oic_rounds.h) beyond what its arrays hold at once, against the oracle: more candidate pairs
-than take their rounds together (2^20), and pairs whose extensions need several fillings of the mask store."""
+than take their rounds together (2^20), and pairs whose extensions need several fillings of the mask store; and pairs
+with more extensions than the cost model expects."""
 import numpy as np
 import pytest
 
@@ -36,8 +37,14 @@ def array_reads(n, seed):
     return readsim.from_strings(seqs)
 
 
-def run_both(R, minlength, partial):
-    eng = oic.Engine(kmer=22, maxerate=0.045, minlength=minlength, threads=1, schedule=oic.SCHED_BATCHED, partial=partial)
+def run_both(R, minlength, partial, expected=None):
+    """expected: a model that expects so many DP cells of every pair, in place of the static estimate."""
+    schedule = oic.SCHED_BATCHED if expected is None else oic.SCHED_LEARNED
+    eng = oic.Engine(kmer=22, maxerate=0.045, minlength=minlength, threads=1, schedule=schedule, partial=partial)
+    if expected is not None:
+        w = np.zeros(oic.NPARAM, np.float32)
+        w[-2] = np.log1p(expected)
+        eng.set_model(w, np.zeros(oic.NFEAT, np.float32), np.ones(oic.NFEAT, np.float32))
     eng.load_reads(R)
     res = eng.run()
     ref = oracle.run(R, kmer=22, maxErate=0.045, minOlap=minlength, nThreads=1, ompThreads=16, partial=int(partial))
@@ -64,3 +71,14 @@ def test_store_is_emptied_when_full(copies):
     words, store = (c["nodes"] + 63) // 64, max(1 << 16, 4 * c["nodes"])
     assert c["pairs"] == 1 and c["extensions"] * words > 2 * store
     assert c["pp_launches"] < c["nodes"] / 128 < (c["nodes"] - store / words) / 64
+
+
+@pytest.mark.parametrize("expected", [0, 1000, 100_000])
+def test_used_up_prediction_does_not_add_rounds(expected):
+    """Low-error pairs, of some ten extensions of several thousand cells each.  A model that expects too little holds
+    back what a pair asks for until its expectation is used up, for a round or two; a round an extension from then on
+    would be tens."""
+    R = readsim.simulate(readsim.PRESETS["c1"].scaled(60_000, seed=82))
+    few, many = run_both(R, 500, False, expected).counters, run_both(R, 500, False).counters
+    assert few["learned_pairs"] == few["pairs"] and few["extensions"] > 8 * few["pairs"]
+    assert few["pp_launches"] <= many["pp_launches"] + 3
