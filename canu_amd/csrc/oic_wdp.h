@@ -366,15 +366,16 @@ __device__ __forceinline__ bool lane_in(uint64_t mask) { return __builtin_amdgcn
 // diagonals.
 // Not inlined: its loops then have the registers to themselves (inlined, a kernel's own values and the N form's
 // took 150 and more, or spilled into the rows).  Aligned, so that its loops keep their place in the lines of the
-// instruction cache whatever stands before it: the same instructions 44 and 56 bytes into a line and at its start took
-// 23.5, 24.1 and 23.8 ms for 951 thousand extensions in k_process_pairs and 25.0, 24.7 and 24.6 ms for 150 thousand in
-// k_extend_nodes.
+// instruction cache whatever stands before it: moved by words, the same instructions take 23.6 to 24.2 ms for 951 thousand
+// extensions in k_process_pairs and 24.5 to 25.0 ms for 150 thousand in k_extend_nodes.  The two words at its start put
+// them where neither is slow (23.6 and 24.7; without them 23.9 and 24.8, two words further 23.8 and 24.7).
 template <int RING, bool ROWS, bool HASN>
 __device__ __attribute__((noinline, aligned(64))) WRows wave_rows(const uint32_t *words_, const uint32_t *nmask_, int64_t a0_, int64_t t0_, uint32_t flags_,
                                                      int32_t m_, int32_t n_, int32_t limit_, int32_t row0_, const int32_t *match_limit_,
                                                      double bmv, double slope_min, uint32_t end_dist_, int32_t *rowm_, int32_t *rowVal_,
                                                      int32_t val_cap_, int32_t max_rows_, int32_t *band_) {
   constexpr int32_t MASK = RING - 1;
+  asm volatile("s_nop 0\n\ts_nop 0");
   const int lane = lane_id();
   const uint32_t flags = (uint32_t)uni((int32_t)flags_), end_dist = (uint32_t)uni((int32_t)end_dist_);
   const bool is_forward = flags & WR_FORWARD, store = ROWS && (flags & WR_STORE), partial = flags & WR_PARTIAL;
